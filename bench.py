@@ -439,8 +439,8 @@ def main():
     dw = G.normal(3 * n, 3005).reshape(n, 3)
     ctx.set_noise(dw)
     sp_pairs = nqp * ctx.elem_point_pairs()  # (Gauss point, particle) pairs per spread
-    names = ["bin", "scan", "place_sort", "gather_forces", "count_lists", "scan64", "fill_ell", "elist_count",
-             "elist_fill", "box_count", "box_fill", "axpby"]
+    names = ["bin", "scan", "place_sort", "gather_forces", "count_lists", "build_sizes", "scan64", "fill_ell", "elist_count",
+             "elist_fill", "box_fill", "axpby"]
     res = measure(G, ctx, args, IF, nqp_1d, order, lo, hi, dw,
                   [G.FP32C] if args.no_fp64 else [G.FP32C, G.FP64], names)
 

@@ -127,9 +127,8 @@ int tune_pick(ggem_ctx* ctx, const std::string& key, int ncand, const std::funct
   return best;
 }
 
-// Staged neighbour records of the FP32C lists (per brick of cells): counts,
-// their scans, one synchronisation for the sizes, then records, target
-// layout and record numbers.
+// Staged neighbour records of the lists (per brick of cells): records and
+// record numbers, with the sizes of the build's census.
 int prepare_box(ggem_ctx* ctx) {
   ctx->box_valid = false;
   ctx->box_unstaged = false;
@@ -138,69 +137,36 @@ int prepare_box(ggem_ctx* ctx) {
   // tensors stay in list order); FP32C the kept pairs' in the brick layout
   ctx->box_fp64 = ctx->p.precision == GGEM_FP64;
   if (!box_supported(ctx)) return GGEM_OK;
-  const size_t nb = size_t(ctx->grid.n_cells >> (3 * kBrickBits));
-  if (ctx->box_brick_cap < nb + 1) {
-    if (ctx->box_cnt) (void)hipFree(ctx->box_cnt);
-    ctx->box_cnt = ctx->box_off = ctx->box_ecnt = ctx->box_eoff = nullptr;
-    ctx->box_brick_cap = 0;
-    GGEM_HIP(ctx, hipMalloc(&ctx->box_cnt, sizeof(int64_t) * 4 * (nb + 1)));
-    ctx->box_brick_cap = nb + 1;
-  }
-  ctx->box_off = ctx->box_cnt + ctx->box_brick_cap;
-  ctx->box_ecnt = ctx->box_cnt + 2 * ctx->box_brick_cap;
-  ctx->box_eoff = ctx->box_cnt + 3 * ctx->box_brick_cap;
-  if (!ctx->box_max_d) GGEM_HIP(ctx, hipMalloc(&ctx->box_max_d, 3 * sizeof(int32_t)));
-  int rc;
-  if ((rc = ensure(ctx, &ctx->box_tgt, &ctx->box_tgt_cap, size_t(ctx->n)))) return rc;
-  if ((rc = ensure(ctx, &ctx->box_base, &ctx->box_base_cap, size_t(ctx->n)))) return rc;
-  if ((rc = grow_scan64(ctx, int64_t(nb) + 1))) return rc;
-  hipError_t e = launch_box_count(ctx);
-  if (e != hipSuccess) return hip_fail(ctx, e, "box_count");
-  if ((e = launch_scan64(ctx, ctx->box_cnt, int64_t(nb), ctx->box_off)) != hipSuccess ||
-      (e = launch_scan64(ctx, ctx->box_ecnt, int64_t(nb), ctx->box_eoff)) != hipSuccess)
-    return hip_fail(ctx, e, "box scan");
-  int64_t total[2] = {0, 0};
-  int64_t mx[3] = {0, 0, 0};
-  {
-    int64_t v[5];
-    if ((rc = peek(ctx, {{ctx->box_off + nb, 8}, {ctx->box_eoff + nb, 8}, {ctx->box_max_d, 4}, {ctx->box_max_d + 1, 4},
-                         {ctx->box_max_d + 2, 4}}, v)))
-      return rc;
-    total[0] = v[0];
-    total[1] = v[1];
-    mx[0] = v[2];
-    mx[1] = v[3];
-    mx[2] = v[4];
-  }
   // no brick staged, or a brick too crowded for the entry layout: the
   // list-order kernels serve
-  if (total[0] <= 0 || mx[0] <= 0 || mx[1] > kBoxMaxTargets) return GGEM_OK;
-  if ((rc = ensure(ctx, &ctx->box_slot, &ctx->box_rec_cap, size_t(total[0])))) return rc;
-  if ((rc = ensure(ctx, &ctx->box_pos, &ctx->box_pos_cap, size_t(total[0])))) return rc;
-  const size_t ne = size_t(std::max<int64_t>(ctx->box_fp64 ? ctx->ell_len : total[1], 1));
+  if (ctx->box_recs <= 0 || ctx->max_recs <= 0 || ctx->max_targets > kBoxMaxTargets) return GGEM_OK;
+  int rc;
+  if ((rc = ensure(ctx, &ctx->box_base, &ctx->box_base_cap, size_t(ctx->n)))) return rc;
+  if ((rc = ensure(ctx, &ctx->box_slot, &ctx->box_rec_cap, size_t(ctx->box_recs)))) return rc;
+  if ((rc = ensure(ctx, &ctx->box_pos, &ctx->box_pos_cap, size_t(ctx->box_recs)))) return rc;
+  const size_t ne = size_t(std::max<int64_t>(ctx->box_fp64 ? ctx->ell_len : ctx->box_entries, 1));
   if ((rc = ensure(ctx, &ctx->box_idx, &ctx->box_idx_cap, ne))) return rc;
   // bricks that are not staged fill their tensors from the lists
-  ctx->box_unstaged = mx[2] > 0;
+  ctx->box_unstaged = ctx->unstaged > 0;
   if (ctx->box_unstaged && (rc = ensure_ell(ctx))) return rc;
-  if ((e = launch_box_fill(ctx, int32_t(mx[0]), int32_t(mx[1]))) != hipSuccess) return hip_fail(ctx, e, "box_fill");
-  ctx->box_max = int32_t(mx[0]);
+  const hipError_t e = launch_box_fill(ctx);
+  if (e != hipSuccess) return hip_fail(ctx, e, "box_fill");
+  ctx->box_max = ctx->max_recs;
   ctx->box_valid = true;
   return GGEM_OK;
 }
 
 int ensure_ell(ggem_ctx* ctx) {
   if (ctx->ell_valid) return GGEM_OK;
-  // slice offsets (the scan of the slice lengths of the count pass), one
-  // synchronisation for the size, then the lists
-  const int64_t nsl = (ctx->n + kSlice - 1) / kSlice;
-  hipError_t e = launch_scan64(ctx, ctx->slice_len, nsl, ctx->slice_off);
-  if (e != hipSuccess) return hip_fail(ctx, e, "scan64");
-  int64_t len = 0;
-  int rc = peek(ctx, {{ctx->slice_off + nsl, 8}}, &len);
-  if (rc) return rc;
-  ctx->ell_len = len;
+  hipError_t e = hipSuccess;
+  int rc = GGEM_OK;
+  if (ctx->ell_len < 0) {  // the lengths changed since the build (kept lists): scan them again
+    const int64_t nsl = (ctx->n + kSlice - 1) / kSlice;
+    if ((e = launch_scan64(ctx, ctx->slice_len, nsl, ctx->slice_off)) != hipSuccess) return hip_fail(ctx, e, "scan64");
+    if ((rc = peek(ctx, {{ctx->slice_off + nsl, 8}}, &ctx->ell_len))) return rc;
+  }
   size_t cap = size_t(ctx->ell_cap);
-  if ((rc = ensure(ctx, &ctx->ell, &cap, size_t(std::max<int64_t>(len, 1))))) return rc;
+  if ((rc = ensure(ctx, &ctx->ell, &cap, size_t(std::max<int64_t>(ctx->ell_len, 1))))) return rc;
   ctx->ell_cap = int64_t(cap);
   if ((e = launch_fill_ell(ctx)) != hipSuccess) return hip_fail(ctx, e, "fill_ell");
   ctx->ell_valid = true;
@@ -381,16 +347,16 @@ void free_all(ggem_ctx* ctx) {
   f(ctx->perm);
   f(ctx->slot_of);
   f(ctx->slot_cell);
-  f(ctx->xs);
   f(ctx->x4);
   f(ctx->fs);
-  f(ctx->fs32);
   f(ctx->fg32);
   f(ctx->fg64);
   f(ctx->u_loc);
   f(ctx->u_out);
   f(ctx->cell_count);
   f(ctx->pcell);
+  f(ctx->prank);
+  f(ctx->arrived);
   f(ctx->cell_start);
   f(ctx->scan_tmp);
   f(ctx->flag);
@@ -409,9 +375,7 @@ void free_all(ggem_ctx* ctx) {
   f(ctx->box_slot);
   f(ctx->box_pos);
   f(ctx->box_idx);
-  f(ctx->box_max_d);
   f(ctx->spread_unstaged);
-  f(ctx->brick_recs);
   f(ctx->pc32);
   f(ctx->coef64);
   f(ctx->noise);
@@ -451,8 +415,6 @@ void free_all(ggem_ctx* ctx) {
   f(ctx->rhs_el);
   if (ctx->par_h) (void)hipHostFree(ctx->par_h);
   ctx->par_h = nullptr;
-  f(ctx->peek_d);
-  ctx->peek_d = nullptr;
   if (ctx->peek_h) (void)hipHostFree(ctx->peek_h);
   ctx->peek_h = nullptr;
   if (ctx->par_ev) (void)hipEventDestroy(ctx->par_ev);
@@ -501,11 +463,10 @@ int grow_scan64(ggem_ctx* ctx, int64_t len) {
 
 int ggem::peek(ggem_ctx* ctx, std::initializer_list<std::pair<const void*, int32_t>> items, int64_t* out) {
   if (items.size() > size_t(kPeekMax)) return fail(ctx, GGEM_ERR_INVALID_ARG, "too many values to read back");
-  if (!ctx->peek_d) GGEM_HIP(ctx, hipMalloc(&ctx->peek_d, sizeof(int64_t) * kPeekMax));
   if (!ctx->peek_h) GGEM_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->peek_h), sizeof(int64_t) * kPeekMax));
   PeekArgs p{};
   p.n = int32_t(items.size());
-  p.dst = ctx->peek_d;
+  p.dst = ctx->peek_h;
   int i = 0;
   for (const auto& it : items) {
     p.src[i] = it.first;
@@ -514,7 +475,6 @@ int ggem::peek(ggem_ctx* ctx, std::initializer_list<std::pair<const void*, int32
   }
   hipError_t e = launch_peek(ctx, p);
   if (e != hipSuccess) return hip_fail(ctx, e, "readback");
-  GGEM_HIP(ctx, hipMemcpyAsync(ctx->peek_h, ctx->peek_d, sizeof(int64_t) * p.n, hipMemcpyDeviceToHost, ctx->stream));
   const int rc = sync(ctx);
   if (rc) return rc;
   for (int k = 0; k < p.n; ++k) out[k] = ctx->peek_h[k];
@@ -797,10 +757,8 @@ int set_particles_impl(ggem_ctx* ctx, int64_t n, const double* xyz, const double
     f_(ctx->perm);
     f_(ctx->slot_of);
     f_(ctx->slot_cell);
-    f_(ctx->xs);
     f_(ctx->x4);
     f_(ctx->fs);
-    f_(ctx->fs32);
     f_(ctx->fg32);
     f_(ctx->fg64);
     f_(ctx->u_loc);
@@ -810,12 +768,13 @@ int set_particles_impl(ggem_ctx* ctx, int64_t n, const double* xyz, const double
     f_(ctx->slice_off);
     f_(ctx->pc32);
     f_(ctx->pcell);
+    f_(ctx->prank);
+    f_(ctx->arrived);
     ctx->pc32 = nullptr;
-    ctx->pcell = nullptr;
-    ctx->x_in = ctx->f_in = ctx->xs = ctx->fs = ctx->u_loc = ctx->u_out = nullptr;
+    ctx->pcell = ctx->prank = ctx->arrived = nullptr;
+    ctx->x_in = ctx->f_in = ctx->fs = ctx->u_loc = ctx->u_out = nullptr;
     ctx->elem = ctx->perm = ctx->slot_of = ctx->slot_cell = ctx->nbr_cnt = nullptr;
     ctx->x4 = nullptr;
-    ctx->fs32 = nullptr;
     ctx->fg32 = nullptr;
     ctx->fg64 = nullptr;
     ctx->slice_len = ctx->slice_off = nullptr;
@@ -828,12 +787,12 @@ int set_particles_impl(ggem_ctx* ctx, int64_t n, const double* xyz, const double
     GGEM_HIP(ctx, hipMalloc(&ctx->perm, sizeof(int32_t) * n));
     GGEM_HIP(ctx, hipMalloc(&ctx->slot_of, sizeof(int32_t) * n));
     GGEM_HIP(ctx, hipMalloc(&ctx->slot_cell, sizeof(int32_t) * n));
-    GGEM_HIP(ctx, hipMalloc(&ctx->xs, sizeof(double) * n3));
     GGEM_HIP(ctx, hipMalloc(&ctx->x4, sizeof(double4) * n));
     GGEM_HIP(ctx, hipMalloc(&ctx->pc32, sizeof(float4) * n));
     GGEM_HIP(ctx, hipMalloc(&ctx->pcell, sizeof(int32_t) * n));
+    GGEM_HIP(ctx, hipMalloc(&ctx->prank, sizeof(int32_t) * n));
+    GGEM_HIP(ctx, hipMalloc(&ctx->arrived, sizeof(int32_t) * n));
     GGEM_HIP(ctx, hipMalloc(&ctx->fs, sizeof(double) * n3));
-    GGEM_HIP(ctx, hipMalloc(&ctx->fs32, sizeof(float) * n3));
     GGEM_HIP(ctx, hipMalloc(&ctx->fg32, sizeof(float4) * n));
     GGEM_HIP(ctx, hipMalloc(&ctx->fg64, sizeof(double4) * n));
     GGEM_HIP(ctx, hipMalloc(&ctx->u_loc, sizeof(double) * n3));
@@ -872,6 +831,25 @@ int set_particles_impl(ggem_ctx* ctx, int64_t n, const double* xyz, const double
 
 namespace {
 
+// The arrays a build writes its census and sizes to.
+int ensure_build(ggem_ctx* ctx) {
+  const size_t nb = size_t(ctx->grid.n_cells >> (3 * kBrickBits));
+  if (!ctx->peek_h) GGEM_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->peek_h), sizeof(int64_t) * kPeekMax));
+  if (ctx->box_brick_cap < nb + 1) {
+    if (ctx->box_cnt) (void)hipFree(ctx->box_cnt);
+    ctx->box_cnt = nullptr;
+    ctx->box_brick_cap = 0;
+    GGEM_HIP(ctx, hipMalloc(&ctx->box_cnt, sizeof(int64_t) * 4 * (nb + 1)));
+    ctx->box_brick_cap = nb + 1;
+  }
+  ctx->box_off = ctx->box_cnt + ctx->box_brick_cap;
+  ctx->box_ecnt = ctx->box_cnt + 2 * ctx->box_brick_cap;
+  ctx->box_eoff = ctx->box_cnt + 3 * ctx->box_brick_cap;
+  int rc = grow_scan64(ctx, int64_t(nb) + 1);
+  if (!rc) rc = ensure(ctx, &ctx->box_tgt, &ctx->box_tgt_cap, size_t(std::max<int64_t>(ctx->n, 1)));
+  return rc;
+}
+
 // GGEM_COMPAT_STALE_LISTS after a build: a particle whose new list is
 // empty keeps its previous one (point_particle.h:189-194); then every
 // particle's effective list is stored by particle id in the reference's
@@ -886,6 +864,7 @@ int keep_lists(ggem_ctx* ctx) {
   int64_t v[2] = {0, 0};
   if ((rc = peek(ctx, {{ctx->flag, 4}, {ctx->pairs_d, 8}}, v))) return rc;
   ctx->stale_lists = v[0] != 0;
+  if (ctx->stale_lists) ctx->ell_len = -1;
   ctx->pairs = v[1];
   if ((rc = ensure(ctx, &ctx->keep_cnt, &ctx->keep_cnt_cap, size_t(std::max<int64_t>(n, 1))))) return rc;
   if ((rc = ensure(ctx, &ctx->keep_off2, &ctx->keep_off2_cap, size_t(n + 1)))) return rc;
@@ -928,31 +907,43 @@ int ggem_build_neighbors(ggem_ctx* ctx) {
   ctx->elist_valid = false;
   ctx->coef64_valid = false;
   ctx->box_built = false;
-  hipError_t e = launch_bin(ctx, hyst);
-  if (e != hipSuccess) return hip_fail(ctx, e, "bin");
+  int rc = ensure_build(ctx);
+  if (rc) return rc;
+  hipError_t e = hipSuccess;
+  if (!ctx->counters_clear && (e = launch_clear_counters(ctx)) != hipSuccess) return hip_fail(ctx, e, "counters");
+  ctx->counters_clear = false;
+  if ((e = launch_bin(ctx, hyst)) != hipSuccess) return hip_fail(ctx, e, "bin");
   if ((e = launch_scan(ctx)) != hipSuccess) return hip_fail(ctx, e, "scan");
   if ((e = launch_place(ctx)) != hipSuccess) return hip_fail(ctx, e, "place");
-  if ((e = launch_gather_forces(ctx)) != hipSuccess) return hip_fail(ctx, e, "gather_forces");
-  {
-    int rc0 = ensure(ctx, &ctx->brick_recs, &ctx->brick_recs_cap,
-                     size_t(std::max<int64_t>(ctx->grid.n_cells >> (3 * kBrickBits), 1)));
-    if (rc0) return rc0;
-  }
   if ((e = launch_count_lists(ctx)) != hipSuccess) return hip_fail(ctx, e, "count");
-  // one synchronisation: the out-of-domain flag and the pair count (the
-  // sliced layout is laid out and filled by ensure_ell when a kernel that
-  // reads it is about to run)
-  int64_t v[2] = {0, 0};
-  int rc = peek(ctx, {{ctx->flag, 4}, {ctx->pairs_d, 8}}, v);
-  if (rc) return rc;
+  // one synchronisation: the out-of-domain flag and every size of the lists
+  // and of the staged records (both are laid out here and filled when a
+  // kernel that reads them is about to run)
+  int64_t* const v = ctx->peek_h;
+  if ((e = launch_build_sizes(ctx, v)) != hipSuccess) return hip_fail(ctx, e, "build sizes");
+  if ((rc = sync(ctx))) return rc;
+  ctx->counters_clear = true;
   const int64_t flag = v[0], pairs = v[1];
   if (flag) {
     ctx->elem_valid = false;
     // point_mesh.C:602-612: a particle no element contains is fatal
     return fail(ctx, GGEM_ERR_OUT_OF_DOMAIN, "a particle lies outside the mesh");
   }
+  ctx->box_recs = v[2];
+  ctx->box_entries = v[3];
+  ctx->ell_len = v[4];
+  ctx->max_recs = int32_t(v[5]);
+  ctx->max_targets = int32_t(v[6]);
+  ctx->unstaged = int32_t(v[7]);
+  if (ctx->box_recs < 0 || ctx->box_entries < 0 || ctx->ell_len < 0) {  // arrays longer than one block scans
+    const int64_t nb = ctx->grid.n_cells >> (3 * kBrickBits), nsl = (ctx->n + kSlice - 1) / kSlice;
+    int64_t w[3];
+    if ((rc = peek(ctx, {{ctx->box_off + nb, 8}, {ctx->box_eoff + nb, 8}, {ctx->slice_off + nsl, 8}}, w))) return rc;
+    ctx->box_recs = w[0];
+    ctx->box_entries = w[1];
+    ctx->ell_len = w[2];
+  }
   ctx->pairs = pairs;
-  ctx->ell_len = -1;
   ctx->ell_valid = false;
   ctx->elem_valid = true;
   ctx->built = true;

@@ -163,29 +163,21 @@ struct BoxGeom {
     z = div_small(yz, inv_ey);
     y = yz - z * ey;
   }
+  // box cell of grid cell (i, j, k) of the brick
+  __device__ __forceinline__ int box_cell(int i, int j, int k) const {
+    return ((k - oz) * ey + (j - oy)) * ex + (i - ox);
+  }
+  // periodic shift code (2 bits per axis) of box cell (x, y, z) seen from
+  // the brick: 2 past the low face, 1 past the high one
+  __device__ __forceinline__ uint32_t shift_code(int x, int y, int z) const {
+    const int X = ox + x, Y = oy + y, Z = oz + z;
+    const uint32_t cx = X < 0 ? 2u : (X >= n[0] ? 1u : 0u), cy = Y < 0 ? 2u : (Y >= n[1] ? 1u : 0u),
+                   cz = Z < 0 ? 2u : (Z >= n[2] ? 1u : 0u);
+    return cx | (cy << 2) | (cz << 4);
+  }
   // brick-order index of grid cell (i, j, k) of the system
   __device__ __forceinline__ int64_t index(int i, int j, int k) const {
     return coff + cell_index_nb(nb0, nb1, i, j, k);
-  }
-  // global cell of box cell q; false outside a non-periodic domain
-  __device__ __forceinline__ bool cell(int q, int64_t& c) const {
-    int x, y, z;
-    xyz(q, x, y, z);
-    int X = ox + x, Y = oy + y, Z = oz + z;
-    if (X < 0 || X >= n[0]) {
-      if (!per[0]) return false;
-      X = wrap_axis(X, n[0]);
-    }
-    if (Y < 0 || Y >= n[1]) {
-      if (!per[1]) return false;
-      Y = wrap_axis(Y, n[1]);
-    }
-    if (Z < 0 || Z >= n[2]) {
-      if (!per[2]) return false;
-      Z = wrap_axis(Z, n[2]);
-    }
-    c = index(X, Y, Z);
-    return true;
   }
 };
 
@@ -194,36 +186,60 @@ struct BoxGeom {
 // particles of the box cells before q (cst[nbc] = all of them).  Cells
 // outside a non-periodic domain are empty.  s_w holds NT/64 ints.  Ends
 // with a barrier.
+// A thread takes whole box rows: the cells of a row lie in memory in runs
+// of up to eight (brick by brick), so an address, a wrap and one clamped
+// group of nine loads serve a run (a thread that took single cells spent
+// its time on their coordinates and on 64 scattered lines per load).
 template <int NT>
 __device__ __forceinline__ void stage_box_cells(const BoxGeom& B, const int32_t* __restrict__ cs,
                                                 int32_t* first, int32_t* cst, int32_t* s_w) {
-  const int per = (B.nbc + NT - 1) / NT;
-  const int q0 = min(B.nbc, int(threadIdx.x) * per), q1 = min(B.nbc, q0 + per);
+  constexpr int M = (1 << kBrickBits) - 1;
+  const int nr = B.ey * B.ez;
+  const int per = (nr + NT - 1) / NT;
+  const int r0 = min(nr, int(threadIdx.x) * per), r1 = min(nr, r0 + per);
   int mine = 0;
-  // eight cells at a time, their cell-start loads all in flight (cells
-  // outside the domain or past the chunk read cell 0 and count nothing)
-  constexpr int G = 8;
-  for (int q = q0; q < q1; q += G) {
-    int64_t c[G];
-    bool in[G];
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-      in[u] = q + u < q1 && B.cell(q + u, c[u]);
-      if (!in[u]) c[u] = 0;
+  for (int r = r0; r < r1; ++r) {
+    const int z = div_small(r, B.inv_ey);
+    int Y = B.oy + (r - z * B.ey), Z = B.oz + z;
+    bool in = true;
+    if (Y < 0 || Y >= B.n[1]) {
+      in = B.per[1] != 0;
+      if (in) Y = wrap_axis(Y, B.n[1]);
     }
-    int f[G], e[G];
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-      f[u] = cs[c[u]];
-      e[u] = cs[c[u] + 1];
+    if (Z < 0 || Z >= B.n[2]) {
+      in = in && B.per[2] != 0;
+      if (in) Z = wrap_axis(Z, B.n[2]);
     }
+    const int64_t row = in ? B.index(0, Y, Z) : 0;  // brick-order index of the row's cell 0
+    const int q = r * B.ex;
+    for (int x = 0; x < B.ex;) {
+      int X = B.ox + x, len = B.ex - x;
+      bool inx = in;
+      if (X < 0 || X >= B.n[0]) {
+        inx = in && B.per[0] != 0;
+        if (inx) X = wrap_axis(X, B.n[0]);
+        else if (X < 0) len = min(len, -X);
+      }
+      if (inx) len = min(len, min(M + 1 - (X & M), B.n[0] - X));
+      if (!inx) {
+        for (int u = 0; u < len; ++u) {
+          cst[q + x + u] = mine;
+          if (first) first[q + x + u] = 0;
+        }
+      } else {
+        const int32_t* __restrict__ p = cs + row + (int64_t(X >> kBrickBits) << (3 * kBrickBits)) + (X & M);
+        int32_t v[M + 2];
 #pragma unroll
-    for (int u = 0; u < G; ++u) {
-      if (q + u >= q1) break;
-      const int k = in[u] ? e[u] - f[u] : 0;
-      cst[q + u] = k;
-      if (first) first[q + u] = in[u] ? f[u] : 0;
-      mine += k;
+        for (int u = 0; u <= M + 1; ++u) v[u] = p[min(u, len)];
+#pragma unroll
+        for (int u = 0; u <= M; ++u) {
+          if (u >= len) break;
+          cst[q + x + u] = mine + (v[u] - v[0]);
+          if (first) first[q + x + u] = v[u];
+        }
+        mine += v[M + 1] - v[0];  // (v[len], clamped)
+      }
+      x += len;
     }
   }
   int incl = mine;
@@ -235,12 +251,8 @@ __device__ __forceinline__ void stage_box_cells(const BoxGeom& B, const int32_t*
   __syncthreads();
   int run = incl - mine;
   for (int w = 0; w < int(threadIdx.x >> 6); ++w) run += s_w[w];
-  for (int q = q0; q < q1; ++q) {
-    const int k = cst[q];
-    cst[q] = run;
-    run += k;
-  }
-  if (threadIdx.x == NT - 1) cst[B.nbc] = run;  // the last thread ends at the total
+  for (int q = r0 * B.ex; q < r1 * B.ex; ++q) cst[q] += run;
+  if (threadIdx.x == NT - 1) cst[B.nbc] = run + mine;  // the last thread ends at the total
   __syncthreads();
 }
 
@@ -302,6 +314,144 @@ template <class Run>
 __device__ __forceinline__ void box_walk(const BoxGeom& B, const StencilRow* __restrict__ rows, int nrows,
                                          int ci, int cj, int ck, Run&& run) {
   box_walk_rows(B, rows, 0, nrows, ci, cj, ck, run);
+}
+
+// The stencil rows as offsets of box cells: row r of the cell at box cell
+// q covers box cells q + lo .. q + hi - 1 (hi one past the end).  Box cells
+// outside a non-periodic domain are empty and periodic images lie in the
+// box unwrapped, so no row is clamped or skipped.
+struct BoxRow {
+  int32_t lo, hi;
+};
+__device__ __forceinline__ void stage_box_rows(const BoxGeom& B, const StencilRow* __restrict__ rows, int nrows,
+                                               BoxRow* rt) {
+  for (int r = int(threadIdx.x); r < nrows; r += int(blockDim.x)) {
+    const StencilRow R = rows[r];
+    const int q = (R.dk * B.ey + R.dj) * B.ex;
+    rt[r] = BoxRow{q + R.di_lo, q + R.di_hi + 1};
+  }
+}
+
+// Stencil rows r0 .. r1 - 1 of the cell at box cell q as ranges of box
+// records, run(a, b) for records a .. b - 1, rows in stencil order, x
+// ascending.  Four rows' ranges are read before the first is walked: a walk
+// is a chain of LDS reads otherwise.
+template <class Run>
+__device__ __forceinline__ void box_walk_flat(const BoxRow* rt, const int32_t* cst, int r0, int r1, int q, Run&& run) {
+  constexpr int U = 4;
+  for (int r = r0; r < r1; r += U) {
+    int a[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const BoxRow w = rt[min(r + u, r1 - 1)];
+      a[u] = cst[q + w.lo];
+      b[u] = r + u < r1 ? cst[q + w.hi] : a[u];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) run(a[u], b[u]);
+  }
+}
+
+// The records of the stencil of the cell at box cell q one by one, rec(r),
+// in record order (the rows are uniform over the wave: scalar reads).
+template <class Rec>
+__device__ __forceinline__ void box_walk_rec(const BoxGeom& B, const StencilRow* __restrict__ rows, int nrows,
+                                             const int32_t* cst, int q, Rec&& rec) {
+  for (int r = 0; r < nrows; ++r) {
+    const StencilRow R = rows[r];
+    const int qr = q + (R.dk * B.ey + R.dj) * B.ex;
+    for (int i = cst[qr + R.di_lo], e = cst[qr + R.di_hi + 1]; i < e; ++i) rec(i);
+  }
+}
+
+// Membership of the stencil by cell difference: per (dj, dk) the packed
+// x range of its row, lo + 128 | (hi + 128) << 8 (empty: lo > hi).
+constexpr int kStencilTab = 1024;
+struct BoxStencil {
+  uint16_t* t;  // [kStencilTab] in LDS
+  int ry, rz, wy;
+  bool ok;      // the table holds this stencil
+  // whole block; ends without a barrier (the table is read after the next)
+  __device__ __forceinline__ void init(const BoxGeom& B, const StencilRow* __restrict__ rows, int nrows) {
+    ry = (B.ey - (1 << kBrickBits)) / 2;
+    rz = (B.ez - (1 << kBrickBits)) / 2;
+    wy = 2 * ry + 1;
+    const int size = wy * (2 * rz + 1);
+    ok = size <= kStencilTab;
+    if (!ok) return;
+    for (int i = int(threadIdx.x); i < size; i += int(blockDim.x)) t[i] = 0x00FFu;
+    __syncthreads();
+    for (int r = int(threadIdx.x); r < nrows; r += int(blockDim.x)) {
+      const StencilRow R = rows[r];
+      t[(R.dk + rz) * wy + R.dj + ry] = uint16_t((R.di_lo + 128) | ((R.di_hi + 128) << 8));
+    }
+  }
+  // d: cell difference + 128 per axis, one byte each (record - target)
+  __device__ __forceinline__ bool has(uint32_t d) const {
+    const uint32_t j = ((d >> 8) & 0xffu) - uint32_t(128 - ry), k = ((d >> 16) & 0xffu) - uint32_t(128 - rz);
+    if (j >= uint32_t(wy) || k > uint32_t(2 * rz)) return false;
+    const uint32_t w = t[k * uint32_t(wy) + j], x = d & 0xffu;
+    return x >= (w & 0xffu) && x <= (w >> 8);
+  }
+};
+
+// One wave over the records of the z layers within reach of box layer bz:
+// emit(r, k) for the k-th record (in record order) with test(r), 64 records
+// at a time; returns their number (uniform over the wave).
+template <class Test, class Emit>
+__device__ __forceinline__ int wave_records(const BoxGeom& B, const BoxStencil& st, const int32_t* cst, int bz,
+                                            Test&& test, Emit&& emit) {
+  const int exy = B.ex * B.ey, lane = int(threadIdx.x) & 63;
+  const int r0 = cst[(bz - st.rz) * exy], r1 = cst[(bz + st.rz + 1) * exy];
+  int n = 0;
+  for (int b = r0; b < r1; b += 64) {
+    const int r = b + lane;
+    const bool in = r < r1 && test(r);
+    const uint64_t m = __ballot(in);
+    if (in) emit(r, n + __popcll(m & ((uint64_t(1) << lane) - 1)));
+    n += __popcll(m);
+  }
+  return n;
+}
+
+// A brick with few targets for its stencil's rows takes its lists from
+// wave_records: a lane per target costs the wave every row and, row by row,
+// its longest run (and leaves lanes idle below 64 targets); a wave per target
+// costs the records of the z layers in reach, of which a wide stencil keeps
+// more.  Record fill with a lane per target and with a wave per target: 44 ->
+// 16 us at 100 beads, 156 -> 80 us for chains in a slit (25,600 beads, 69
+// rows, 31 targets in the median brick and 167 in the largest), 821 -> 413 us
+// for 64 suspensions (272,000 beads, 69 rows, 34 targets); at 125,000 beads
+// (21 rows, 244 targets) 49 -> 110 us, so that stays with a lane per target.
+__device__ __forceinline__ bool wave_walk(int nt, int nrows) { return nt <= kWaveWalkPerRow * nrows; }
+
+// Share [i0, i1) of a brick's nt targets for this block: with wave_walk, one
+// of up to gridDim.y blocks for every kShareTargets targets.
+__device__ __forceinline__ void brick_share(int nt, bool waves, int& i0, int& i1) {
+  const int shares = waves ? max(1, min(int(gridDim.y), (nt + kShareTargets - 1) / kShareTargets)) : 1;
+  const int y = min(int(blockIdx.y), shares);
+  i0 = int(int64_t(nt) * y / shares);
+  i1 = int(int64_t(nt) * min(y + 1, shares) / shares);
+}
+
+// Lanes that share one target's stencil walk in a brick kernel of NT
+// threads: the largest power of two, 16 at most, that still gives every
+// target of the brick its lanes in one pass.  A brick with few targets
+// leaves its threads idle while each target's one lane walks its 69 rows
+// (two-unit elements).  With one lane each, and the records counted in a
+// pass of its own, the counts took 36 + 5 us at 100 beads and 38 + 9 us for
+// 25,600 chain beads in a slit; now 11 and 26 us together.
+template <int NT>
+__device__ __forceinline__ int walk_lanes(int nt) {
+  int g = 1;
+  while (g < 16 && 2 * g * nt <= NT) g *= 2;
+  return g;
+}
+
+// sum of v over the g consecutive lanes (g a power of two) of the lane's group
+__device__ __forceinline__ int group_sum(int v, int g) {
+  for (int o = 1; o < g; o <<= 1) v += __shfl_xor(v, o, 64);
+  return v;
 }
 
 // Walk the particle slots of every element of the stencil of element

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <functional>
 #include <initializer_list>
@@ -82,6 +83,8 @@ constexpr int kSlice = 64;  // targets per neighbour-list slice (one wave)
 constexpr int kCellBitsX = 11, kCellBitsY = 11, kCellBitsZ = 10;
 // most particles of one brick of cells for the staged FP32C entry layout
 constexpr int kBoxMaxTargets = 65536;
+constexpr int kBoxMaxRows = 512;  // stencil rows a brick kernel keeps in LDS
+constexpr int kBoxMaxRecs = 2048;  // records of a staged brick (64 KiB of LDS)
 
 struct Profiler {
   struct Rec {
@@ -140,21 +143,22 @@ struct ggem_ctx {
   int32_t* perm = nullptr;    // [n] slot -> particle
   int32_t* slot_of = nullptr; // [n] particle -> slot
   int32_t* slot_cell = nullptr;
-  double* xs = nullptr;       // [3][n] sorted SoA positions
   double4* x4 = nullptr;      // [n] sorted positions, one 32-byte record per slot
   double* fs = nullptr;       // [3][n] sorted SoA forces (FP64)
-  float* fs32 = nullptr;      // [3][n] sorted SoA forces (FP32)
   float4* fg32 = nullptr;     // [n] forces by slot, gather copy (FP32)
   double4* fg64 = nullptr;    // [n] forces by slot, gather copy (FP64)
   double* u_loc = nullptr;    // [3n] interleaved, particle order
   double* u_out = nullptr;    // [3n] interleaved, particle order
   int32_t* pcell = nullptr;       // [n] brick-order cell of each particle
-  int32_t* cell_count = nullptr;  // [n_cells]
+  int32_t* prank = nullptr;       // [n] place of each particle in its cell, in arrival order
+  int32_t* arrived = nullptr;     // [n] particles by cell, in arrival order
+  int32_t* cell_count = nullptr;  // [n_cells], zero between builds
   int32_t* cell_start = nullptr;  // [n_cells + 1], by brick-order cell index
   int32_t* scan_tmp = nullptr;
   int64_t scan_tmp_len = 0;
   int32_t* flag = nullptr;        // device error flag
   int64_t* pairs_d = nullptr;     // pair count reduction
+  bool counters_clear = false;    // cell_count, flag and pairs_d are zero (a complete build leaves them so)
   int64_t pairs = -1;
   bool built = false;
   // the slot-ordered positions (xs, x4, pc32) hold the particles' current
@@ -222,9 +226,11 @@ struct ggem_ctx {
   size_t box_pos_cap = 0;
   uint16_t* box_idx = nullptr;    // [entries] the neighbour's record number (staged bricks)
   size_t box_idx_cap = 0;
-  int32_t* brick_recs = nullptr;  // [n_bricks] particles in each brick's box (list count pass)
-  size_t brick_recs_cap = 0;
-  int32_t* box_max_d = nullptr;   // [3] largest record count of a staged brick, most targets of a brick, unstaged bricks with targets
+  // the census of the current build (k_brick_count, k_build_sizes)
+  int64_t box_recs = 0, box_entries = 0;  // records and entries of all staged bricks
+  int32_t max_recs = 0;           // largest record count of a staged brick
+  int32_t max_targets = 0;        // most targets of a brick
+  int32_t unstaged = 0;           // bricks with targets that are not staged
   uint8_t* spread_unstaged = nullptr;  // [bricks] the brick spreading's boxes over its record table
   size_t spread_unstaged_cap = 0;
   int32_t box_max = 0;            // same on the host; 0 when no brick is staged
@@ -285,8 +291,7 @@ struct ggem_ctx {
   int32_t* sys_slot = nullptr;       // [n] system of each slot
   int64_t sys_cap = 0;
   double* par_h = nullptr;           // pinned staging of per-system recurrence parameters
-  int64_t* peek_d = nullptr;         // [kPeekMax] device values gathered for one readback
-  int64_t* peek_h = nullptr;         // [kPeekMax] their pinned host copy
+  int64_t* peek_h = nullptr;         // [kPeekMax] pinned: device values gathered for one readback
   int32_t cheb_terms = 1 << 30;      // terms of the last reference-mode Chebyshev call (its statistics read)
   size_t par_cap = 0;
   hipEvent_t par_ev = nullptr;
@@ -348,6 +353,30 @@ namespace ggem {
 // since the build, or some lists are kept ones.
 inline bool explicit_minimg(const ggem_ctx* c) { return c->exact_minimg || c->stale_pos || c->stale_lists; }
 
+// stencil rows the brick kernels' LDS tables hold (the largest system's)
+inline int32_t box_rows_cap(const ggem_ctx* c) {
+  int32_t cap = c->n_rows;
+  if (c->nsys > 1) {
+    cap = 0;
+    for (const SysGrid& s : c->sys_h) cap = s.nrows > cap ? s.nrows : cap;
+  }
+  return cap < kBoxMaxRows ? cap : kBoxMaxRows;
+}
+// Blocks that share a brick's targets in the list and record fills where a
+// wave takes a target at a time (wave_walk, brick_share: gridDim.y blocks
+// are launched, a brick uses one per kShareTargets targets).  Where all
+// blocks are resident at once, the most crowded brick sets the time
+// otherwise; 4096 bricks fill the chip by themselves and staging a brick
+// twice only costs.
+constexpr int kShareTargets = 32;
+constexpr int kWaveWalkPerRow = 4;  // wave_walk: targets per stencil row
+inline unsigned brick_split(const ggem_ctx* c) {
+  const int64_t nb = c->grid.n_cells >> (3 * kBrickBits);
+  const int64_t most = std::min<int64_t>(c->max_targets, int64_t(kWaveWalkPerRow) * box_rows_cap(c));
+  const int64_t s = (most + kShareTargets - 1) / kShareTargets;
+  return nb > 2048 || s < 1 ? 1u : unsigned(std::min<int64_t>(s, 8));
+}
+
 // error helpers
 int fail(ggem_ctx* ctx, int code, const std::string& msg);
 int hip_fail(ggem_ctx* ctx, hipError_t e, const char* what);
@@ -385,8 +414,16 @@ hipError_t launch_bin(ggem_ctx* ctx, bool hysteresis);
 hipError_t launch_scan(ggem_ctx* ctx);
 hipError_t launch_place(ggem_ctx* ctx);
 hipError_t launch_gather_forces(ggem_ctx* ctx);
-// per-slot counts, per-slice lengths and the total pair count
+// zero the build's counters (cell_count, flag, pairs_d)
+hipError_t launch_clear_counters(ggem_ctx* ctx);
+// per-slot counts, per-slice lengths, the total pair count and the census
+// of the staged records
 hipError_t launch_count_lists(ggem_ctx* ctx);
+// record, entry and slice offsets and the sizes a build reads back: host[8]
+// (pinned) = flag, pairs, records, entries, list slots (-1: the total at the
+// end of the scanned array), largest record count, most targets of a
+// brick, unstaged bricks
+hipError_t launch_build_sizes(ggem_ctx* ctx, int64_t* host);
 // exclusive scan of int64 values; out[len] receives the total
 hipError_t launch_scan64(ggem_ctx* ctx, const int64_t* in, int64_t len, int64_t* out);
 hipError_t launch_fill_ell(ggem_ctx* ctx);
@@ -461,11 +498,8 @@ struct ChebEpi {
 };
 // pair tensors of every list entry for the given precision
 hipError_t launch_pair_tensors(ggem_ctx* ctx, int precision);
-// FP32C staged records: box_cnt per brick (and box_max_d by a reduction)
-hipError_t launch_box_count(ggem_ctx* ctx);
-// records, target layout and record numbers of every brick, with box_off
-// and box_eoff scanned from the counts
-hipError_t launch_box_fill(ggem_ctx* ctx, int32_t max_records, int32_t max_targets);
+// records and record numbers of every staged brick
+hipError_t launch_box_fill(ggem_ctx* ctx);
 // whether the context's FP32C lists can be staged per brick
 bool box_supported(const ggem_ctx* ctx);
 hipError_t launch_pair_beads(ggem_ctx* ctx, int precision, int epi, const double* u_glob,
@@ -479,9 +513,8 @@ hipError_t launch_apply(ggem_ctx* ctx, int precision, int nrhs, const SlotVec& x
 
 // ---- launchers (kernels_spread.hip) ----
 // Fe[e][j][l] (node_major: Fe[e][l][j])
-// Small device values (int32 or int64 each) read back in one kernel, one
-// copy into pinned host memory and one synchronisation; out gets them as
-// int64.
+// Small device values (int32 or int64 each) written to pinned host memory
+// by one kernel, then one synchronisation; out gets them as int64.
 constexpr int kPeekMax = 8;
 struct PeekArgs {
   const void* src[kPeekMax];

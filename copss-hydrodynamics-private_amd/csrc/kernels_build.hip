@@ -86,7 +86,8 @@ __device__ __forceinline__ SysView sys_view(const Grid& g, const StencilRow* row
 template <bool BATCH>
 __global__ void k_bin(Grid g, const SysGrid* __restrict__ sys, const int32_t* __restrict__ sys_part,
                       int64_t n, const double* __restrict__ x, int32_t* __restrict__ elem, int use_prev,
-                      int32_t* __restrict__ pcell, int32_t* __restrict__ count, int32_t* __restrict__ flag) {
+                      int32_t* __restrict__ pcell, int32_t* __restrict__ prank, int32_t* __restrict__ count,
+                      int32_t* __restrict__ flag) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const SysView v = sys_view<BATCH>(g, nullptr, 0, nullptr, sys, sys_part, i);
@@ -104,35 +105,7 @@ __global__ void k_bin(Grid g, const SysGrid* __restrict__ sys, const int32_t* __
   const int64_t c = v.coff + elem_cell(v.g, e);
   elem[i] = int32_t(v.eoff + e);
   pcell[i] = int32_t(c);
-  atomicAdd(&count[c], 1);
-}
-
-// system of each slot (batched contexts)
-__global__ void k_slot_sys(int64_t n, const int32_t* __restrict__ perm, const int32_t* __restrict__ sys_part,
-                           int32_t* __restrict__ sys_slot) {
-  const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (s < n) sys_slot[s] = sys_part[perm[s]];
-}
-
-// FP32C position records: each particle's FP64 offset from its cell centre
-// rounded to FP32, the cell's (i, j, k) packed into the fourth word.  A
-// pair displacement is then (cell difference) h + (offset difference), all
-// terms small, in FP32.
-template <bool BATCH>
-__global__ void k_cell_rel(Grid g, const SysGrid* __restrict__ sys, const int32_t* __restrict__ sys_slot,
-                           int64_t n, const int32_t* __restrict__ slot_cell, const double4* __restrict__ x4,
-                           float4* __restrict__ pc) {
-  const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  const SysView v = sys_view<BATCH>(g, nullptr, 0, nullptr, sys, sys_slot, s);
-  int ci, cj, ck;
-  cell_ijk(v.g, slot_cell[s] - v.coff, ci, cj, ck);
-  const double4 p = x4[s];
-  const double cx = v.g.bmin[0] + (double(ci) + 0.5) * v.g.h[0];
-  const double cy = v.g.bmin[1] + (double(cj) + 0.5) * v.g.h[1];
-  const double cz = v.g.bmin[2] + (double(ck) + 0.5) * v.g.h[2];
-  const uint32_t packed = uint32_t(ci) | (uint32_t(cj) << kCellBitsX) | (uint32_t(ck) << (kCellBitsX + kCellBitsY));
-  pc[s] = make_float4(float(p.x - cx), float(p.y - cy), float(p.z - cz), __uint_as_float(packed));
+  prank[i] = atomicAdd(&count[c], 1);  // a place in the cell, in arrival order
 }
 
 // system of each particle from the particle ranges (binary search)
@@ -171,7 +144,8 @@ __device__ __forceinline__ int32_t block_exclusive_scan(int32_t v, int32_t* sh, 
   return incl - v;
 }
 
-__global__ void k_scan_tiles(const int32_t* __restrict__ in, int64_t len, int32_t* __restrict__ out,
+// (the counts are left zero for the next build)
+__global__ void k_scan_tiles(int32_t* __restrict__ in, int64_t len, int32_t* __restrict__ out,
                              int32_t* __restrict__ tile_sums) {
   __shared__ int32_t sh[kScanThreads];
   const int64_t base = int64_t(blockIdx.x) * kScanTile + int64_t(threadIdx.x) * kScanItems;
@@ -180,6 +154,7 @@ __global__ void k_scan_tiles(const int32_t* __restrict__ in, int64_t len, int32_
 #pragma unroll
   for (int q = 0; q < kScanItems; ++q) {
     v[q] = (base + q < len) ? in[base + q] : 0;
+    if (base + q < len) in[base + q] = 0;
     s += v[q];
   }
   int32_t total;
@@ -206,72 +181,98 @@ __global__ void k_scan_sums(int32_t* __restrict__ sums, int64_t ntiles) {
   }
 }
 
-__global__ void k_scan_add(int32_t* __restrict__ out, int64_t len, const int32_t* __restrict__ sums,
+// Carry into one tile per block: the sum of the tiles before it, added up
+// by the block itself (a launch less than scanning the sums first; at most
+// kScanSelfMax tiles, 8 loads a thread at 2M cells), or the scanned sums'.
+constexpr int64_t kScanSelfMax = 4096;
+__global__ void k_scan_add(int32_t* __restrict__ out, int64_t len, const int32_t* __restrict__ sums, int scanned,
                            int32_t total_n) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < len) out[i] += sums[i / kScanTile];
-  if (i == 0) out[len] = total_n;
-}
-
-// Place every particle into its cell's slot range (arbitrary order within
-// the cell), then sort each cell by particle id and fill the slot arrays.
-__global__ void k_place(int64_t n, const int32_t* __restrict__ pcell,
-                        const int32_t* __restrict__ cell_start, int32_t* __restrict__ cursor,
-                        int32_t* __restrict__ perm) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int32_t c = pcell[i];
-  const int32_t s = cell_start[c] + atomicAdd(&cursor[c], 1);
-  perm[s] = int32_t(i);
-}
-
-// e runs over brick-order cell indices
-__global__ void k_sort_cells(int64_t n_cells, int64_t n, const int32_t* __restrict__ cell_start,
-                             int32_t* __restrict__ perm, int32_t* __restrict__ slot_of,
-                             int32_t* __restrict__ slot_cell, const double* __restrict__ x,
-                             double* __restrict__ xs, double4* __restrict__ x4) {
-  const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= n_cells) return;
-  const int32_t a = cell_start[e], b = cell_start[e + 1];
-  for (int32_t s = a + 1; s < b; ++s) {  // insertion sort by particle id
-    const int32_t v = perm[s];
-    int32_t t = s - 1;
-    while (t >= a && perm[t] > v) {
-      perm[t + 1] = perm[t];
-      --t;
-    }
-    perm[t + 1] = v;
+  __shared__ int32_t sh[kScanThreads / 64];
+  int32_t carry = 0;
+  if (scanned) {
+    carry = sums[blockIdx.x];
+  } else {
+    for (int t = int(threadIdx.x); t < int(blockIdx.x); t += kScanThreads) carry += sums[t];
+    carry = wave_sum(carry);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = carry;
+    __syncthreads();
+    carry = 0;
+#pragma unroll
+    for (int w = 0; w < kScanThreads / 64; ++w) carry += sh[w];
   }
-  for (int32_t s = a; s < b; ++s) {
-    const int32_t p = perm[s];
-    slot_of[p] = s;
-    slot_cell[s] = int32_t(e);
-    const double px = x[3 * int64_t(p)], py = x[3 * int64_t(p) + 1], pz = x[3 * int64_t(p) + 2];
-    xs[s] = px;
-    xs[n + s] = py;
-    xs[2 * n + s] = pz;
-    x4[s] = make_double4(px, py, pz, 0.0);
+  const int64_t base = int64_t(blockIdx.x) * kScanTile;
+#pragma unroll
+  for (int q = 0; q < kScanItems; ++q) {
+    const int64_t i = base + q * kScanThreads + threadIdx.x;
+    if (i < len) out[i] += carry;
   }
+  if (blockIdx.x == 0 && threadIdx.x == 0) out[len] = total_n;
 }
 
-// Forces (interleaved, particle order) -> slot SoA (FP64, FP32) and the
-// per-slot gather copies.
-__global__ void k_gather_forces(int64_t n, const int32_t* __restrict__ perm,
-                                const double* __restrict__ f, double* __restrict__ fs,
-                                float* __restrict__ fs32, float4* __restrict__ fg32,
-                                double4* __restrict__ fg64) {
-  const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  const int64_t p = perm[s];
+// Every particle into its cell's slot range, in arrival order
+__global__ void k_place(int64_t n, const int32_t* __restrict__ pcell, const int32_t* __restrict__ prank,
+                        const int32_t* __restrict__ cell_start, int32_t* __restrict__ arrived) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) arrived[cell_start[pcell[i]] + prank[i]] = int32_t(i);
+}
+
+// Forces of particle p (interleaved) to slot s: SoA and gather records
+__device__ __forceinline__ void slot_forces(int64_t n, int64_t s, int64_t p, const double* __restrict__ f,
+                                            double* __restrict__ fs, float4* __restrict__ fg32,
+                                            double4* __restrict__ fg64) {
   const double fx = f[3 * p], fy = f[3 * p + 1], fz = f[3 * p + 2];
   fs[s] = fx;
   fs[n + s] = fy;
   fs[2 * n + s] = fz;
-  fs32[s] = float(fx);
-  fs32[n + s] = float(fy);
-  fs32[2 * n + s] = float(fz);
   fg32[s] = make_float4(float(fx), float(fy), float(fz), 0.f);
   fg64[s] = make_double4(fx, fy, fz, 0.0);
+}
+
+// The slot arrays.  A particle's slot is its cell's first plus the cell's
+// particles of smaller id (counted, so the order does not depend on the
+// arrival); its thread writes all of the slot's records: one pass instead
+// of a sort per cell and a pass each for positions, FP32C records and
+// forces.  FP32C position record: the FP64 offset from the cell centre
+// rounded to FP32, the cell's (i, j, k) packed into the fourth word, so that
+// a pair displacement is (cell difference) h + (offset difference), all
+// terms small, in FP32.
+template <bool BATCH>
+__global__ void k_slots(Grid g, const SysGrid* __restrict__ sys, const int32_t* __restrict__ sys_part, int64_t n,
+                        const int32_t* __restrict__ arrived, const int32_t* __restrict__ pcell,
+                        const int32_t* __restrict__ cell_start, const double* __restrict__ x,
+                        const double* __restrict__ f, int32_t* __restrict__ perm, int32_t* __restrict__ slot_of,
+                        int32_t* __restrict__ slot_cell, int32_t* __restrict__ sys_slot, double4* __restrict__ x4,
+                        float4* __restrict__ pc, double* __restrict__ fs, float4* __restrict__ fg32,
+                        double4* __restrict__ fg64) {
+  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int32_t p = arrived[t];
+  const int32_t c = pcell[p];
+  const int32_t a = cell_start[c], b = cell_start[c + 1];
+  const double px = x[3 * int64_t(p)], py = x[3 * int64_t(p) + 1], pz = x[3 * int64_t(p) + 2];
+  int32_t s = a;
+  for (int32_t q = a; q < b; ++q) s += arrived[q] < p ? 1 : 0;
+  perm[s] = p;
+  slot_of[p] = s;
+  slot_cell[s] = c;
+  x4[s] = make_double4(px, py, pz, 0.0);
+  const SysView v = sys_view<BATCH>(g, nullptr, 0, nullptr, sys, sys_part, p);
+  if constexpr (BATCH) sys_slot[s] = sys_part[p];
+  int ci, cj, ck;
+  cell_ijk(v.g, c - v.coff, ci, cj, ck);
+  const double cx = v.g.bmin[0] + (double(ci) + 0.5) * v.g.h[0];
+  const double cy = v.g.bmin[1] + (double(cj) + 0.5) * v.g.h[1];
+  const double cz = v.g.bmin[2] + (double(ck) + 0.5) * v.g.h[2];
+  const uint32_t packed = uint32_t(ci) | (uint32_t(cj) << kCellBitsX) | (uint32_t(ck) << (kCellBitsX + kCellBitsY));
+  pc[s] = make_float4(float(px - cx), float(py - cy), float(pz - cz), __uint_as_float(packed));
+  slot_forces(n, s, p, f, fs, fg32, fg64);
+}
+
+// Forces (interleaved, particle order) -> slot SoA and gather records.
+__global__ void k_gather_forces(int64_t n, const int32_t* __restrict__ perm, const double* __restrict__ f,
+                                double* __restrict__ fs, float4* __restrict__ fg32, double4* __restrict__ fg64) {
+  const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (s < n) slot_forces(n, s, perm[s], f, fs, fg32, fg64);
 }
 
 // ---- per-brick list builds: the brick's box cells staged in LDS ----
@@ -294,8 +295,12 @@ struct BrickArgs {
   const int32_t* slot_cell;  // brick-order cell of each slot
   const SysGrid* sys;        // batched contexts (null: one system)
   const int32_t* sys_slot;
-  int32_t cells_cap;         // box cells the LDS tables hold
-  int32_t* recs;             // [n_bricks] particles in the box of each brick the count pass staged
+  int32_t cells_cap;         // box cells and stencil rows the LDS tables hold
+  int32_t rows_cap;
+  int32_t* cnt;              // [n] list lengths by slot
+  int64_t* box_cnt;          // census of the staged records (k_brick_count)
+  int64_t* box_ecnt;
+  int32_t* box_tgt;
   // slots whose list is the one their particle kept (GGEM_COMPAT_STALE_LISTS)
   const uint8_t* stale;      // [n] or null
   const int64_t* keep_off;   // kept lists by particle (reference order)
@@ -317,55 +322,103 @@ __device__ __forceinline__ bool brick_staged(const BrickArgs& a, const BoxGeom& 
   return B.nbc <= a.cells_cap && B.fits();
 }
 
-// Slot of every record of the box (record = particle of a box cell, in box
-// order) after stage_box_cells: a stencil run of box cells q0..q1 is then
-// records cst[q0] .. cst[q1 + 1] - 1.  False (nothing written) when the
-// box holds more than cap records.  Uniform over the block; ends with a
-// barrier when it writes.
-constexpr int kBrickRecCap = 2048;
+constexpr int kBoxSortMax = 2048;  // targets of a brick ordered in LDS
 
-__device__ __forceinline__ bool stage_box_slots(const BoxGeom& B, const int32_t* first, const int32_t* cst,
-                                                int32_t* rslot, int cap) {
-  if (cst[B.nbc] > cap) return false;
-  const int per = (B.nbc + kBrickThreads - 1) / kBrickThreads;
-  const int q0 = min(B.nbc, int(threadIdx.x) * per), q1 = min(B.nbc, q0 + per);
-  for (int q = q0; q < q1; ++q) {
-    const int f = first[q], r0 = cst[q];
-    for (int r = r0, e = cst[q + 1]; r < e; ++r) rslot[r] = f + (r - r0);
-  }
-  __syncthreads();
-  return true;
-}
-
-// List lengths of the brick's slots (own element + stencil, minus itself).
+// List lengths of the brick's slots (own element + stencil, minus itself),
+// and the census of the staged records: the records of the brick's box
+// (box_cnt, 0 where the brick is not staged: no targets, a box over the
+// packing or more than kBoxMaxRecs records), its targets longest lists first
+// (box_tgt, ties by slot; slot order in bricks that are not staged) and the
+// size of its entry layout (box_ecnt: 64 x the longest list of every wave of
+// that order).  Every brick writes its box_cnt and box_ecnt.
 template <bool BATCH>
-__global__ void __launch_bounds__(kBrickThreads) k_brick_count(BrickArgs a, int32_t* __restrict__ cnt) {
-  extern __shared__ int32_t cst[];  // [cells_cap + 1]
+__global__ void __launch_bounds__(kBrickThreads) k_brick_count(BrickArgs a) {
+  extern __shared__ int32_t cst[];  // [cells_cap + 1], then the stencil rows
   __shared__ int32_t s_w[kBrickThreads / 64];
+  __shared__ __attribute__((aligned(16))) int32_t keys[kBoxSortMax];  // list lengths in slot order
+  __shared__ int32_t skeys[kBoxSortMax];                              // the same, longest first
+  __shared__ int64_t s_e[kBrickThreads / 64];
   const int64_t brick = blockIdx.x;
   const int64_t c0 = brick * kBrickCells;
   const int32_t sb = a.cs[c0], se = a.cs[c0 + kBrickCells];
-  if (sb >= se) return;  // uniform over the block
+  const int nt = se - sb;
+  if (nt <= 0) {  // uniform over the block
+    if (threadIdx.x == 0) a.box_cnt[brick] = a.box_ecnt[brick] = 0;
+    return;
+  }
   BoxGeom B;
   const SysView v = brick_view<BATCH>(a, brick, sb, B);
-  if (brick_staged(a, B)) {
+  const bool order = nt <= kBoxSortMax;
+  int total = 0;
+  if (brick_staged(a, B) && v.nrows <= a.rows_cap) {
+    BoxRow* rt = reinterpret_cast<BoxRow*>(cst + ((a.cells_cap + 2) & ~1));
+    stage_box_rows(B, v.rows, v.nrows, rt);
     stage_box_cells<kBrickThreads>(B, a.cs, nullptr, cst, s_w);
-    if (threadIdx.x == 0) a.recs[brick] = cst[B.nbc];  // (the staged-record census reuses it)
-    for (int32_t s = sb + int32_t(threadIdx.x); s < se; s += kBrickThreads) {
+    total = cst[B.nbc];
+    const int nl = walk_lanes<kBrickThreads>(nt);  // lanes per slot, each a range of the rows
+    const int sub = int(threadIdx.x) & (nl - 1);
+    const int r0 = v.nrows * sub / nl, r1 = v.nrows * (sub + 1) / nl;
+    for (int i = int(threadIdx.x) / nl; i < nt; i += kBrickThreads / nl) {
       int ci, cj, ck;
-      cell_ijk(v.g, a.slot_cell[s] - v.coff, ci, cj, ck);
-      int c = -1;
-      box_walk(B, v.rows, v.nrows, ci, cj, ck, [&](int q0, int q1, uint32_t) { c += cst[q1 + 1] - cst[q0]; });
-      cnt[s] = c;
+      cell_ijk(v.g, a.slot_cell[sb + i] - v.coff, ci, cj, ck);
+      int c = 0;
+      box_walk_flat(rt, cst, r0, r1, B.box_cell(ci, cj, ck), [&](int p, int q) { c += q - p; });
+      c = group_sum(c, nl) - 1;
+      if (sub == 0) {
+        a.cnt[sb + i] = c;
+        if (order) keys[i] = c;
+      }
     }
   } else {
-    for (int32_t s = sb + int32_t(threadIdx.x); s < se; s += kBrickThreads) {
+    for (int i = int(threadIdx.x); i < nt; i += kBrickThreads) {
       int ci, cj, ck;
-      cell_ijk(v.g, a.slot_cell[s] - v.coff, ci, cj, ck);
+      cell_ijk(v.g, a.slot_cell[sb + i] - v.coff, ci, cj, ck);
       int c = -1;
       for_each_segment(v.g, v.rows, v.nrows, v.cs, ci, cj, ck, [&](int32_t p, int32_t q, uint32_t) { c += q - p; });
-      cnt[s] = c;
+      a.cnt[sb + i] = c;
+      if (order) keys[i] = c;
     }
+  }
+  const bool staged = total > 0 && total <= kBoxMaxRecs;
+  const bool sorted = staged && order;
+  if (order)
+    for (int i = nt + int(threadIdx.x); i < ((nt + 3) & ~3); i += kBrickThreads) keys[i] = -1;  // (kBoxSortMax is 4k)
+  __syncthreads();
+  if (sorted) {
+    const int4* k4 = reinterpret_cast<const int4*>(keys);
+    for (int i = int(threadIdx.x); i < nt; i += kBrickThreads) {
+      const int ki = keys[i];
+      int r = 0;  // lengths that come before: longer ones, and equal ones of smaller slot
+      for (int j = 0; j < nt; j += 4) {
+        const int4 k = k4[j >> 2];
+        r += (k.x > ki || (k.x == ki && j < i)) ? 1 : 0;
+        r += (k.y > ki || (k.y == ki && j + 1 < i)) ? 1 : 0;
+        r += (k.z > ki || (k.z == ki && j + 2 < i)) ? 1 : 0;
+        r += (k.w > ki || (k.w == ki && j + 3 < i)) ? 1 : 0;
+      }
+      skeys[r] = ki;
+      a.box_tgt[sb + r] = sb + i;
+    }
+    __syncthreads();
+  } else {
+    for (int i = int(threadIdx.x); i < nt; i += kBrickThreads) a.box_tgt[sb + i] = sb + i;
+  }
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int64_t esum = 0;
+  const int nw = (nt + 63) / 64;
+  for (int w = wv; w < nw; w += kBrickThreads / 64) {
+    const int i = 64 * w + lane;
+    const int c = i < nt ? (sorted ? skeys[i] : order ? keys[i] : a.cnt[sb + i]) : 0;
+    esum += 64 * int64_t(wave_max(c));
+  }
+  if (lane == 0) s_e[wv] = esum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int64_t e = 0;
+#pragma unroll
+    for (int w = 0; w < kBrickThreads / 64; ++w) e += s_e[w];
+    a.box_ecnt[brick] = e;
+    a.box_cnt[brick] = staged ? total : 0;
   }
 }
 
@@ -396,62 +449,92 @@ __global__ void __launch_bounds__(kSliceBlock) k_slice_len(const int32_t* __rest
   }
 }
 
-// The lists of the brick's slots in the sliced layout.
+// The lists of the brick's slots in the sliced layout.  In a staged brick a
+// list is its records in record order (rows in stencil order, x ascending
+// through the box, slots ascending within a cell).
 template <bool BATCH>
 __global__ void __launch_bounds__(kBrickThreads) k_brick_fill_ell(BrickArgs a, const int64_t* __restrict__ slice_off,
                                                                   uint32_t* __restrict__ ell) {
   extern __shared__ int32_t lds[];
   __shared__ int32_t s_w[kBrickThreads / 64];
-  int32_t* first = lds;                  // [cells_cap]
-  int32_t* cst = lds + a.cells_cap;      // [cells_cap + 1]
-  int32_t* rslot = cst + a.cells_cap + 1;  // [kBrickRecCap]
+  int32_t* first = lds;                                                 // [cells_cap]
+  int32_t* cst = lds + a.cells_cap;                                     // [cells_cap + 1]
+  uint32_t* rent = reinterpret_cast<uint32_t*>(cst + a.cells_cap + 1);  // [kBoxMaxRecs]
+  uint32_t* rcell = rent + kBoxMaxRecs;                                 // [kBoxMaxRecs]
+  BoxStencil st;
+  st.t = reinterpret_cast<uint16_t*>(rcell + kBoxMaxRecs);              // [kStencilTab]
   const int64_t brick = blockIdx.x;
   const int64_t c0 = brick * kBrickCells;
   const int32_t sb = a.cs[c0], se = a.cs[c0 + kBrickCells];
   if (sb >= se) return;
   BoxGeom B;
   const SysView v = brick_view<BATCH>(a, brick, sb, B);
-  const bool staged = brick_staged(a, B);
+  const bool waves = wave_walk(se - sb, v.nrows);
+  int i0, i1;
+  brick_share(se - sb, waves, i0, i1);
+  if (i0 >= i1) return;  // uniform over the block
   bool recs = false;
-  if (staged) {
+  if (brick_staged(a, B)) {
+    st.init(B, v.rows, v.nrows);
     stage_box_cells<kBrickThreads>(B, a.cs, first, cst, s_w);
-    recs = stage_box_slots(B, first, cst, rslot, kBrickRecCap);
+    recs = cst[B.nbc] <= kBoxMaxRecs;
+    if (recs) {
+      for (int q = int(threadIdx.x); q < B.nbc; q += kBrickThreads) {
+        const int r0 = cst[q], e = cst[q + 1];
+        if (r0 == e) continue;
+        int x, y, z;
+        B.xyz(q, x, y, z);
+        const uint32_t hi = B.shift_code(x, y, z) << kSlotBits, cell = box_pack(x, y, z);
+        for (int r = r0; r < e; ++r) {
+          rent[r] = uint32_t(first[q] + (r - r0)) | hi;
+          rcell[r] = cell;
+        }
+      }
+      __syncthreads();
+    }
   }
-  for (int32_t s = sb + int32_t(threadIdx.x); s < se; s += kBrickThreads) {
+  if (waves && recs && !a.stale && st.ok) {
+    // one wave per slot over the records of its z layers, 64 at a time
+    for (int i = i0 + int(threadIdx.x >> 6); i < i1; i += kBrickThreads / 64) {
+      const int32_t s = __builtin_amdgcn_readfirstlane(sb + i);
+      int ci, cj, ck;
+      cell_ijk(v.g, a.slot_cell[s] - v.coff, ci, cj, ck);
+      const int q = B.box_cell(ci, cj, ck), self = cst[q] + (s - first[q]);
+      const uint32_t kb = 0x808080u - box_pack(ci - B.ox, cj - B.oy, ck - B.oz);
+      uint32_t* out = ell + slice_off[s >> 6] + (s & 63);
+      wave_records(
+          B, st, cst, ck - B.oz, [&](int r) { return r != self && st.has(rcell[r] + kb); },
+          [&](int r, int k) { out[int64_t(k) * kSlice] = rent[r]; });
+    }
+    return;
+  }
+  for (int32_t s = sb + i0 + int32_t(threadIdx.x); s < sb + i1; s += kBrickThreads) {
     int ci, cj, ck;
     cell_ijk(v.g, a.slot_cell[s] - v.coff, ci, cj, ck);
     uint32_t* out = ell + slice_off[s >> 6] + (s & 63);
-    int64_t k = 0;
     if (a.stale && a.stale[s]) {  // the particle's kept list, slots by the current order
       const int32_t p = a.perm[s];
-      for (int64_t q = a.keep_off[p], e = a.keep_off[p + 1]; q < e; ++q, ++k)
-        out[k * kSlice] = uint32_t(a.slot_of[a.keep_ids[q]]);
+      for (int64_t q = a.keep_off[p], e = a.keep_off[p + 1]; q < e; ++q, out += kSlice)
+        *out = uint32_t(a.slot_of[a.keep_ids[q]]);
       continue;
     }
-    auto emit = [&](int32_t p, int32_t q, uint32_t code) {
-      const uint32_t hi = code << kSlotBits;
-      for (int32_t t = p; t < q; ++t) {
-        if (t == s) continue;
-        out[k * kSlice] = uint32_t(t) | hi;
-        ++k;
-      }
-    };
     if (recs) {
-      box_walk(B, v.rows, v.nrows, ci, cj, ck, [&](int q0, int q1, uint32_t code) {
-        const uint32_t hi = code << kSlotBits;
-        for (int r = cst[q0], e = cst[q1 + 1]; r < e; ++r) {
-          const int32_t t = rslot[r];
-          if (t == s) continue;
-          out[k * kSlice] = uint32_t(t) | hi;
-          ++k;
-        }
-      });
-    } else if (staged) {
-      box_walk(B, v.rows, v.nrows, ci, cj, ck, [&](int q0, int q1, uint32_t code) {
-        for (int q = q0; q <= q1; ++q) emit(first[q], first[q] + (cst[q + 1] - cst[q]), code);
+      const int q = B.box_cell(ci, cj, ck);
+      const int self = cst[q] + (s - first[q]);
+      box_walk_rec(B, v.rows, v.nrows, cst, q, [&](int r) {
+        if (r == self) return;
+        *out = rent[r];
+        out += kSlice;
       });
     } else {
-      for_each_segment(v.g, v.rows, v.nrows, v.cs, ci, cj, ck, emit);
+      for_each_segment(v.g, v.rows, v.nrows, v.cs, ci, cj, ck, [&](int32_t p, int32_t q, uint32_t code) {
+        const uint32_t hi = code << kSlotBits;
+        for (int32_t t = p; t < q; ++t) {
+          if (t == s) continue;
+          *out = uint32_t(t) | hi;
+          out += kSlice;
+        }
+      });
     }
   }
 }
@@ -460,19 +543,23 @@ __global__ void __launch_bounds__(kBrickThreads) k_brick_fill_ell(BrickArgs a, c
 // the own element is part of its stencil and nothing is excluded.  Every
 // brick has elements, particles or not.
 __global__ void __launch_bounds__(kBrickThreads) k_brick_elist_count(BrickArgs a, int64_t* __restrict__ cnt) {
-  extern __shared__ int32_t cst[];  // [cells_cap + 1]
+  extern __shared__ int32_t cst[];  // [cells_cap + 1], then the stencil rows
   __shared__ int32_t s_w[kBrickThreads / 64];
   BoxGeom B;
   B.init(a.g, 0, a.reach, blockIdx.x);
-  const bool staged = brick_staged(a, B);
-  if (staged) stage_box_cells<kBrickThreads>(B, a.cs, nullptr, cst, s_w);
+  const bool staged = brick_staged(a, B) && a.nrows <= a.rows_cap;
+  BoxRow* rt = reinterpret_cast<BoxRow*>(cst + ((a.cells_cap + 2) & ~1));
+  if (staged) {
+    stage_box_rows(B, a.rows, a.nrows, rt);
+    stage_box_cells<kBrickThreads>(B, a.cs, nullptr, cst, s_w);
+  }
   for (int l = int(threadIdx.x); l < kBrickCells; l += kBrickThreads) {
     int ci, cj, ck;
     int64_t e;
     if (!brick_elem(B, l, ci, cj, ck, e)) continue;
     int64_t c = 0;
     if (staged)
-      box_walk(B, a.rows, a.nrows, ci, cj, ck, [&](int q0, int q1, uint32_t) { c += cst[q1 + 1] - cst[q0]; });
+      box_walk_flat(rt, cst, 0, a.nrows, B.box_cell(ci, cj, ck), [&](int p, int q) { c += q - p; });
     else
       for_each_segment(a.g, a.rows, a.nrows, a.cs, ci, cj, ck, [&](int32_t p, int32_t q, uint32_t) { c += q - p; });
     cnt[e] = c;
@@ -578,6 +665,104 @@ __global__ void k_scan64_add(int64_t* __restrict__ out, int64_t len, const int64
   if (i == 0) out[len] = sums[ntiles];
 }
 
+// What a build leaves to the host, in one launch: block 0 scans the records
+// per brick, block 1 the entries per brick, block 2 the slice lengths (a
+// null input is left to launch_scan64), block 3 the maxima over the bricks
+// (records, targets, unstaged bricks with targets), the out-of-domain flag
+// and the pair count, which it clears for the next build.  The results go
+// straight to pinned host memory.
+constexpr int kSizesThreads = 1024;
+constexpr int kSizesItems = 4;
+constexpr int64_t kSizesMax = 65536;  // longest array one block scans (16 rounds)
+struct SizesArgs {
+  const int64_t* in[3];
+  int64_t* out[3];
+  int64_t len[3];
+  const int32_t* cs;
+  const int64_t* box_cnt;
+  int64_t nbricks;
+  int32_t* flag;
+  int64_t* pairs;
+  int64_t* host;  // [8] flag, pairs, records, entries, list slots, then the maxima
+};
+__global__ void __launch_bounds__(kSizesThreads) k_build_sizes(SizesArgs a) {
+  __shared__ int64_t sh[kSizesThreads / 64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  constexpr int NW = kSizesThreads / 64;
+  if (blockIdx.x < 3) {
+    const int64_t* __restrict__ in = a.in[blockIdx.x];
+    int64_t* __restrict__ out = a.out[blockIdx.x];
+    const int64_t len = a.len[blockIdx.x];
+    if (!in) return;
+    int64_t carry = 0;
+    for (int64_t c0 = 0; c0 < len; c0 += kSizesThreads * kSizesItems) {
+      const int64_t base = c0 + int64_t(threadIdx.x) * kSizesItems;
+      int64_t v[kSizesItems], mine = 0;
+#pragma unroll
+      for (int q = 0; q < kSizesItems; ++q) {
+        v[q] = base + q < len ? in[base + q] : 0;
+        mine += v[q];
+      }
+      int64_t incl = mine;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int64_t y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+      }
+      if (lane == 63) sh[wv] = incl;
+      __syncthreads();
+      int64_t run = carry + incl - mine, total = 0;
+      for (int w = 0; w < NW; ++w) {
+        if (w < wv) run += sh[w];
+        total += sh[w];
+      }
+      carry += total;
+#pragma unroll
+      for (int q = 0; q < kSizesItems; ++q) {
+        if (base + q < len) out[base + q] = run;
+        run += v[q];
+      }
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+      out[len] = carry;
+      a.host[2 + blockIdx.x] = carry;
+    }
+    return;
+  }
+  int mr = 0, mt = 0, nu = 0;
+  for (int64_t k = threadIdx.x; k < a.nbricks; k += kSizesThreads) {
+    const int nt = a.cs[(k + 1) * kBrickCells] - a.cs[k * kBrickCells];
+    const int nr = int(a.box_cnt[k]);
+    mr = max(mr, nr);
+    mt = max(mt, nt);
+    nu += nt > 0 && nr == 0 ? 1 : 0;
+  }
+  mr = wave_max(mr);
+  mt = wave_max(mt);
+  nu = wave_sum(nu);
+  __shared__ int32_t s_m[3][NW];
+  if (lane == 0) {
+    s_m[0][wv] = mr;
+    s_m[1][wv] = mt;
+    s_m[2][wv] = nu;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < NW; ++w) {
+      mr = max(mr, s_m[0][w]);
+      mt = max(mt, s_m[1][w]);
+      nu += s_m[2][w];
+    }
+    a.host[0] = *a.flag;
+    a.host[1] = *a.pairs;
+    a.host[5] = mr;
+    a.host[6] = mt;
+    a.host[7] = nu;
+    *a.flag = 0;
+    *a.pairs = 0;
+  }
+}
+
 // Neighbour count of every particle (own element + stencil, minus itself).
 __global__ void k_count_pairs(Grid g, const StencilRow* __restrict__ rows, int nrows,
                               const int32_t* __restrict__ cell_start,
@@ -674,7 +859,7 @@ __global__ void k_elem_point(Grid g, const StencilRow* __restrict__ rows, int nr
 // records are relative to the centre of the cell now holding the particle
 // (floor, clamped), the lists, elements and slot order stay.
 __global__ void k_update_slots(Grid g, int64_t n, const int32_t* __restrict__ perm, const double* __restrict__ x,
-                               double* __restrict__ xs, double4* __restrict__ x4, float4* __restrict__ pc) {
+                               double4* __restrict__ x4, float4* __restrict__ pc) {
   const int64_t s = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (s >= n) return;
   const int64_t p = perm[s];
@@ -687,7 +872,6 @@ __global__ void k_update_slots(Grid g, int64_t n, const int32_t* __restrict__ pe
     q = q < 0.0 ? 0.0 : (q > double(g.n[d] - 1) ? double(g.n[d] - 1) : q);
     c[d] = int(q);
     o[d] = float(v[d] - (g.bmin[d] + (q + 0.5) * g.h[d]));
-    xs[d * n + s] = v[d];
   }
   x4[s] = make_double4(v[0], v[1], v[2], 0.0);
   const uint32_t packed = uint32_t(c[0]) | (uint32_t(c[1]) << kCellBitsX) | (uint32_t(c[2]) << (kCellBitsX + kCellBitsY));
@@ -750,20 +934,23 @@ __global__ void k_locate(Grid g, int64_t m, const double* __restrict__ pts, int3
 
 }  // namespace
 
-hipError_t launch_bin(ggem_ctx* ctx, bool hysteresis) {
+hipError_t launch_clear_counters(ggem_ctx* ctx) {
   hipError_t e = hipMemsetAsync(ctx->cell_count, 0, sizeof(int32_t) * ctx->grid.n_cells, ctx->stream);
-  if (e != hipSuccess) return e;
-  e = hipMemsetAsync(ctx->flag, 0, sizeof(int32_t), ctx->stream);
-  if (e != hipSuccess) return e;
+  if (e == hipSuccess) e = hipMemsetAsync(ctx->flag, 0, sizeof(int32_t), ctx->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(ctx->pairs_d, 0, sizeof(int64_t), ctx->stream);
+  return e;
+}
+
+hipError_t launch_bin(ggem_ctx* ctx, bool hysteresis) {
   if (ctx->n == 0) return hipSuccess;
   ProfScope ps(ctx, "bin");
   if (ctx->nsys > 1)
     hipLaunchKernelGGL(k_bin<true>, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->grid,
                        ctx->sys_d, ctx->sys_part, ctx->n, ctx->x_in, ctx->elem, hysteresis ? 1 : 0,
-                       ctx->pcell, ctx->cell_count, ctx->flag);
+                       ctx->pcell, ctx->prank, ctx->cell_count, ctx->flag);
   else
     hipLaunchKernelGGL(k_bin<false>, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->grid,
-                       nullptr, nullptr, ctx->n, ctx->x_in, ctx->elem, hysteresis ? 1 : 0, ctx->pcell,
+                       nullptr, nullptr, ctx->n, ctx->x_in, ctx->elem, hysteresis ? 1 : 0, ctx->pcell, ctx->prank,
                        ctx->cell_count, ctx->flag);
   return hipGetLastError();
 }
@@ -774,32 +961,28 @@ hipError_t launch_scan(ggem_ctx* ctx) {
   ProfScope ps(ctx, "scan");
   hipLaunchKernelGGL(k_scan_tiles, dim3(unsigned(ntiles)), dim3(kScanThreads), 0, ctx->stream,
                      ctx->cell_count, len, ctx->cell_start, ctx->scan_tmp);
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanThreads), 0, ctx->stream, ctx->scan_tmp, ntiles);
-  hipLaunchKernelGGL(k_scan_add, dim3(blocks_for(len)), dim3(kBlock), 0, ctx->stream, ctx->cell_start,
-                     len, ctx->scan_tmp, int32_t(ctx->n));
+  const int scanned = ntiles > kScanSelfMax ? 1 : 0;
+  if (scanned)
+    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanThreads), 0, ctx->stream, ctx->scan_tmp, ntiles);
+  hipLaunchKernelGGL(k_scan_add, dim3(unsigned(ntiles)), dim3(kScanThreads), 0, ctx->stream, ctx->cell_start,
+                     len, ctx->scan_tmp, scanned, int32_t(ctx->n));
   return hipGetLastError();
 }
 
 hipError_t launch_place(ggem_ctx* ctx) {
-  hipError_t e = hipMemsetAsync(ctx->cell_count, 0, sizeof(int32_t) * ctx->grid.n_cells, ctx->stream);
-  if (e != hipSuccess) return e;
+  if (ctx->n == 0) return hipSuccess;
   ProfScope ps(ctx, "place_sort");
-  if (ctx->n > 0)
-    hipLaunchKernelGGL(k_place, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->n,
-                       ctx->pcell, ctx->cell_start, ctx->cell_count, ctx->perm);
-  hipLaunchKernelGGL(k_sort_cells, dim3(blocks_for(ctx->grid.n_cells)), dim3(kBlock), 0, ctx->stream,
-                     ctx->grid.n_cells, ctx->n, ctx->cell_start, ctx->perm, ctx->slot_of,
-                     ctx->slot_cell, ctx->x_in, ctx->xs, ctx->x4);
-  if (ctx->n == 0) return hipGetLastError();
-  if (ctx->nsys > 1) {
-    hipLaunchKernelGGL(k_slot_sys, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->n, ctx->perm,
-                       ctx->sys_part, ctx->sys_slot);
-    hipLaunchKernelGGL(k_cell_rel<true>, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->grid,
-                       ctx->sys_d, ctx->sys_slot, ctx->n, ctx->slot_cell, ctx->x4, ctx->pc32);
-  } else {
-    hipLaunchKernelGGL(k_cell_rel<false>, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->grid,
-                       nullptr, nullptr, ctx->n, ctx->slot_cell, ctx->x4, ctx->pc32);
-  }
+  hipLaunchKernelGGL(k_place, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->n, ctx->pcell, ctx->prank,
+                     ctx->cell_start, ctx->arrived);
+  if (ctx->nsys > 1)
+    hipLaunchKernelGGL(k_slots<true>, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->grid, ctx->sys_d,
+                       ctx->sys_part, ctx->n, ctx->arrived, ctx->pcell, ctx->cell_start, ctx->x_in, ctx->f_in,
+                       ctx->perm, ctx->slot_of, ctx->slot_cell, ctx->sys_slot, ctx->x4, ctx->pc32, ctx->fs, ctx->fg32,
+                       ctx->fg64);
+  else
+    hipLaunchKernelGGL(k_slots<false>, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->grid, nullptr,
+                       nullptr, ctx->n, ctx->arrived, ctx->pcell, ctx->cell_start, ctx->x_in, ctx->f_in, ctx->perm,
+                       ctx->slot_of, ctx->slot_cell, nullptr, ctx->x4, ctx->pc32, ctx->fs, ctx->fg32, ctx->fg64);
   return hipGetLastError();
 }
 
@@ -807,7 +990,7 @@ hipError_t launch_gather_forces(ggem_ctx* ctx) {
   if (ctx->n == 0) return hipSuccess;
   ProfScope ps(ctx, "gather_forces");
   hipLaunchKernelGGL(k_gather_forces, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->n,
-                     ctx->perm, ctx->f_in, ctx->fs, ctx->fs32, ctx->fg32, ctx->fg64);
+                     ctx->perm, ctx->f_in, ctx->fs, ctx->fg32, ctx->fg64);
   return hipGetLastError();
 }
 
@@ -828,7 +1011,11 @@ BrickArgs brick_args(const ggem_ctx* ctx) {
   int cap = cells(ctx->reach);
   for (int k = 0; k < ctx->nsys && ctx->nsys > 1; ++k) cap = std::max(cap, cells(ctx->sys_h[k].reach));
   a.cells_cap = std::min(cap, kBoxMaxCells);
-  a.recs = ctx->brick_recs;
+  a.rows_cap = box_rows_cap(ctx);
+  a.cnt = ctx->nbr_cnt;
+  a.box_cnt = ctx->box_cnt;
+  a.box_ecnt = ctx->box_ecnt;
+  a.box_tgt = ctx->box_tgt;
   a.stale = ctx->stale_lists ? ctx->stale_slot : nullptr;
   a.keep_off = ctx->keep_off;
   a.keep_ids = ctx->keep_ids;
@@ -839,21 +1026,50 @@ BrickArgs brick_args(const ggem_ctx* ctx) {
 
 unsigned brick_count(const ggem_ctx* ctx) { return unsigned(ctx->grid.n_cells >> (3 * kBrickBits)); }
 
+hipError_t launch_slice_len(ggem_ctx* ctx) {
+  hipLaunchKernelGGL(k_slice_len, dim3(blocks_for(ctx->n, kSliceBlock)), dim3(kSliceBlock), 0, ctx->stream,
+                     ctx->nbr_cnt, ctx->n, ctx->slice_len, reinterpret_cast<unsigned long long*>(ctx->pairs_d));
+  return hipGetLastError();
+}
+
 hipError_t launch_count_lists(ggem_ctx* ctx) {
-  hipError_t e = hipMemsetAsync(ctx->pairs_d, 0, sizeof(int64_t), ctx->stream);
-  if (e != hipSuccess || ctx->n == 0) return e;
   ProfScope ps(ctx, "count_lists");
   const BrickArgs a = brick_args(ctx);
-  const size_t lds = sizeof(int32_t) * (size_t(a.cells_cap) + 1);
+  const size_t lds = sizeof(int32_t) * size_t((a.cells_cap + 2) & ~1) + sizeof(BoxRow) * size_t(a.rows_cap);
   if (a.sys)
-    hipLaunchKernelGGL(k_brick_count<true>, dim3(brick_count(ctx)), dim3(kBrickThreads), lds, ctx->stream, a,
-                       ctx->nbr_cnt);
+    hipLaunchKernelGGL(k_brick_count<true>, dim3(brick_count(ctx)), dim3(kBrickThreads), lds, ctx->stream, a);
   else
-    hipLaunchKernelGGL(k_brick_count<false>, dim3(brick_count(ctx)), dim3(kBrickThreads), lds, ctx->stream, a,
-                       ctx->nbr_cnt);
-  hipLaunchKernelGGL(k_slice_len, dim3(blocks_for(ctx->n, kSliceBlock)), dim3(kSliceBlock), 0, ctx->stream,
-                     ctx->nbr_cnt, ctx->n,
-                     ctx->slice_len, reinterpret_cast<unsigned long long*>(ctx->pairs_d));
+    hipLaunchKernelGGL(k_brick_count<false>, dim3(brick_count(ctx)), dim3(kBrickThreads), lds, ctx->stream, a);
+  return ctx->n > 0 ? launch_slice_len(ctx) : hipGetLastError();
+}
+
+hipError_t launch_build_sizes(ggem_ctx* ctx, int64_t* host) {
+  const int64_t nb = int64_t(brick_count(ctx)), nsl = (ctx->n + kSlice - 1) / kSlice;
+  const int64_t* in[3] = {ctx->box_cnt, ctx->box_ecnt, ctx->slice_len};
+  int64_t* out[3] = {ctx->box_off, ctx->box_eoff, ctx->slice_off};
+  const int64_t len[3] = {nb, nb, nsl};
+  SizesArgs a;
+  for (int k = 0; k < 3; ++k) {
+    a.in[k] = len[k] <= kSizesMax ? in[k] : nullptr;
+    a.out[k] = out[k];
+    a.len[k] = len[k];
+    if (len[k] == 0) {  // no particles: no slices
+      a.in[k] = nullptr;
+      host[2 + k] = 0;
+    } else if (!a.in[k]) {
+      const hipError_t e = launch_scan64(ctx, in[k], len[k], out[k]);
+      if (e != hipSuccess) return e;
+      host[2 + k] = -1;  // read back by the caller
+    }
+  }
+  a.cs = ctx->cell_start;
+  a.box_cnt = ctx->box_cnt;
+  a.nbricks = nb;
+  a.flag = ctx->flag;
+  a.pairs = ctx->pairs_d;
+  a.host = host;
+  ProfScope ps(ctx, "build_sizes");
+  hipLaunchKernelGGL(k_build_sizes, dim3(4), dim3(kSizesThreads), 0, ctx->stream, a);
   return hipGetLastError();
 }
 
@@ -875,12 +1091,14 @@ hipError_t launch_fill_ell(ggem_ctx* ctx) {
   if (ctx->n == 0) return hipSuccess;
   ProfScope ps(ctx, "fill_ell");
   const BrickArgs a = brick_args(ctx);
-  const size_t lds = sizeof(int32_t) * (2 * size_t(a.cells_cap) + 1 + kBrickRecCap);
+  const size_t lds =
+      sizeof(int32_t) * (2 * size_t(a.cells_cap) + 1 + 2 * size_t(kBoxMaxRecs)) + sizeof(uint16_t) * kStencilTab;
+  const unsigned split = brick_split(ctx);
   if (a.sys)
-    hipLaunchKernelGGL(k_brick_fill_ell<true>, dim3(brick_count(ctx)), dim3(kBrickThreads), lds, ctx->stream, a,
+    hipLaunchKernelGGL(k_brick_fill_ell<true>, dim3(brick_count(ctx), split), dim3(kBrickThreads), lds, ctx->stream, a,
                        ctx->slice_off, ctx->ell);
   else
-    hipLaunchKernelGGL(k_brick_fill_ell<false>, dim3(brick_count(ctx)), dim3(kBrickThreads), lds, ctx->stream,
+    hipLaunchKernelGGL(k_brick_fill_ell<false>, dim3(brick_count(ctx), split), dim3(kBrickThreads), lds, ctx->stream,
                        a, ctx->slice_off, ctx->ell);
   return hipGetLastError();
 }
@@ -895,7 +1113,7 @@ hipError_t launch_part_sys(ggem_ctx* ctx) {
 hipError_t launch_elist_count(ggem_ctx* ctx) {
   ProfScope ps(ctx, "elist_count");
   const BrickArgs a = brick_args(ctx);
-  const size_t lds = sizeof(int32_t) * (size_t(a.cells_cap) + 1);
+  const size_t lds = sizeof(int32_t) * size_t((a.cells_cap + 2) & ~1) + sizeof(BoxRow) * size_t(a.rows_cap);
   hipLaunchKernelGGL(k_brick_elist_count, dim3(brick_count(ctx)), dim3(kBrickThreads), lds, ctx->stream, a,
                      ctx->elist_off);
   return hipGetLastError();
@@ -909,6 +1127,7 @@ hipError_t launch_elist_fill(ggem_ctx* ctx) {
 }
 
 hipError_t launch_count_pairs(ggem_ctx* ctx, int64_t* counts_d) {
+  ctx->counters_clear = false;
   hipError_t e = hipMemsetAsync(ctx->pairs_d, 0, sizeof(int64_t), ctx->stream);
   if (e != hipSuccess || ctx->n == 0) return e;
   hipLaunchKernelGGL(k_count_pairs, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->grid,
@@ -939,20 +1158,19 @@ hipError_t launch_update_slots(ggem_ctx* ctx) {
   if (ctx->n == 0) return hipSuccess;
   ProfScope ps(ctx, "update_slots");
   hipLaunchKernelGGL(k_update_slots, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->grid, ctx->n,
-                     ctx->perm, ctx->x_in, ctx->xs, ctx->x4, ctx->pc32);
+                     ctx->perm, ctx->x_in, ctx->x4, ctx->pc32);
   return hipGetLastError();
 }
 
 hipError_t launch_stale_patch(ggem_ctx* ctx, bool have_kept) {
+  ctx->counters_clear = false;
   hipError_t e = hipMemsetAsync(ctx->flag, 0, sizeof(int32_t), ctx->stream);
   if (e == hipSuccess) e = hipMemsetAsync(ctx->pairs_d, 0, sizeof(int64_t), ctx->stream);
   if (e != hipSuccess || ctx->n == 0) return e;
   ProfScope ps(ctx, "stale_lists");
   hipLaunchKernelGGL(k_stale_patch, dim3(blocks_for(ctx->n)), dim3(kBlock), 0, ctx->stream, ctx->n, ctx->perm,
                      have_kept ? ctx->keep_off : nullptr, ctx->nbr_cnt, ctx->stale_slot, ctx->flag);
-  hipLaunchKernelGGL(k_slice_len, dim3(blocks_for(ctx->n, kSliceBlock)), dim3(kSliceBlock), 0, ctx->stream,
-                     ctx->nbr_cnt, ctx->n, ctx->slice_len, reinterpret_cast<unsigned long long*>(ctx->pairs_d));
-  return hipGetLastError();
+  return launch_slice_len(ctx);
 }
 
 hipError_t launch_counts_by_particle(ggem_ctx* ctx, int64_t* out) {

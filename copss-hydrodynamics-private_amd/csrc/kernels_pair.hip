@@ -183,6 +183,10 @@ struct V4<double> {
 };
 
 // FP64 pair tensors of all list entries: (A, w) with G = A I + sgn w w^T.
+// gridDim.y threads share a slot's entries (every gridDim.y-th one each):
+// one entry is a chain of a gather, two erf and two exp, so a few thousand
+// slots with one thread each left the chip idle (3,001 beads: 65 us, with
+// eight threads a slot 12.5 us).
 template <bool EXACT, bool BATCH, int BLK>
 __global__ void __launch_bounds__(BLK) k_tensors(PairArgs a, double4* __restrict__ c64) {
   const int64_t s = block_index(a.xcd) * BLK + threadIdx.x;
@@ -192,16 +196,17 @@ __global__ void __launch_bounds__(BLK) k_tensors(PairArgs a, double4* __restrict
   const int64_t base = a.slice_off[s >> 6] + (s & 63);
   const uint32_t* lst = a.ell + base;
   const double4 xs = a.x4[s];
-  const int last = cnt > 0 ? cnt - 1 : 0;
-  uint32_t e1 = cnt > 0 ? lst[0] : 0u;
-  uint32_t e2 = cnt > 1 ? lst[kSlice] : e1;
+  const int k0 = int(blockIdx.y), dk = int(gridDim.y), last = cnt - 1;
+  if (k0 > last) return;
+  uint32_t e1 = lst[uint32_t(k0) * uint32_t(kSlice)];
+  uint32_t e2 = lst[uint32_t(min(k0 + dk, last)) * uint32_t(kSlice)];
   double4 xa = a.x4[e1 & kSlotMask];
-  for (int k = 0; k < cnt; ++k) {
+  for (int k = k0; k < cnt; k += dk) {
     const uint32_t e = e1;
     const double4 xt = xa;
     e1 = e2;
     xa = a.x4[e1 & kSlotMask];
-    e2 = lst[uint32_t(min(k + 2, last)) * uint32_t(kSlice)];
+    e2 = lst[uint32_t(min(k + 2 * dk, last)) * uint32_t(kSlice)];
     double dx, dy, dz;
     pair_disp<EXACT>(g, xs, xt, e >> kSlotBits, dx, dy, dz);
     const int64_t o = base + int64_t(k) * kSlice;
@@ -506,7 +511,6 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
 // A brick whose box holds more than kBoxMaxRecs records reads its list and
 // gathers the neighbours' records from global memory.
 constexpr int kBoxThreads = 256;
-constexpr int kBoxMaxRecs = 2048;   // records of a staged brick (64 KiB of LDS)
 // A target's packed entry base: the offset of its entry 0 (below 2^40), its
 // own record number (12 bits) and, in staged bricks, its count of stored
 // (kept) entries (12 bits; a staged box holds at most kBoxMaxRecs records).
@@ -518,13 +522,9 @@ constexpr uint64_t kField12 = 0xFFFu;
 struct BoxArgs {
   const int32_t* cs;     // cell starts, brick order
   int32_t reach[3];      // stencil reach of a plain context
-  int64_t* cnt;          // [n_bricks] records of each staged brick (k_box_count)
-  int64_t* ecnt;         // [n_bricks] entries of each brick's layout (k_box_count)
-  int32_t* maxrec;       // [3] largest staged record count, most targets of a brick, unstaged bricks
-  const int32_t* recs;   // [n_bricks] particles in each brick's box (from the list count pass)
   const int64_t* off;    // [n_bricks + 1] first record of each brick
   const int64_t* eoff;   // [n_bricks + 1] first entry of each brick
-  int32_t* tgt;          // [n] slots of each brick, longest lists first (staged bricks)
+  const int32_t* tgt;    // [n] slots of each brick, longest lists first (staged bricks)
   int64_t* base;         // [n] entry 0 of the target at each position of tgt (low kBaseBits),
                          // its own record in a staged brick (above)
   uint32_t* slot;        // [records] slot of each record
@@ -558,7 +558,6 @@ struct BoxView {
 // wave w.  Staged bricks order their targets by list length, longest first
 // (ties by slot), so the lanes of a wave do similar work.
 constexpr int kBoxMaxWaves = kBoxMaxTargets / 64;  // waves of one brick
-constexpr int kBoxSortMax = 2048;   // targets of a brick ordered in LDS
 
 // Box of the brick holding first_slot (the slot picks the system of a
 // batched context).
@@ -572,97 +571,6 @@ __device__ __forceinline__ void box_init(BoxGeom& B, const PairArgs& a, const in
   }
 }
 
-// Records of every brick's box (a brick is staged when it has targets, its
-// box fits the packing and holds at most kBoxMaxRecs records), the order of
-// its targets and the size of its entry layout.
-__global__ void __launch_bounds__(kBoxThreads) k_box_count(PairArgs a, BoxArgs b) {
-  __shared__ int32_t keys[kBoxSortMax];   // list lengths in slot order
-  __shared__ int32_t skeys[kBoxSortMax];  // the same, longest first
-  __shared__ int64_t s_e[kBoxThreads / 64];
-  const int64_t brick = blockIdx.x;
-  const int64_t c0 = brick * kBrickCells;
-  const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
-  const int nt = se - sb;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  int total = 0;
-  if (nt > 0) {  // uniform over the block
-    BoxGeom B;
-    box_init(B, a, b.reach, brick, sb);
-    // the list count pass staged exactly the boxes that fit and counted
-    // their particles
-    if (B.fits()) total = b.recs[brick];
-  }
-  const bool staged = total > 0 && total <= kBoxMaxRecs;
-  const bool sorted = staged && nt <= kBoxSortMax;
-  if (sorted) {
-    for (int i = int(threadIdx.x); i < nt; i += kBoxThreads) keys[i] = a.cnt[sb + i];
-    __syncthreads();
-    for (int i = int(threadIdx.x); i < nt; i += kBoxThreads) {
-      const int ki = keys[i];
-      int r = 0;
-      for (int j = 0; j < nt; ++j) {
-        const int kj = keys[j];
-        r += (kj > ki || (kj == ki && j < i)) ? 1 : 0;
-      }
-      skeys[r] = ki;
-      b.tgt[sb + r] = sb + i;
-    }
-    __syncthreads();
-  } else {
-    for (int i = int(threadIdx.x); i < nt; i += kBoxThreads) b.tgt[sb + i] = sb + i;
-  }
-  // entries: 64 x the longest list of every wave of the order
-  int64_t esum = 0;
-  const int nw = (nt + 63) / 64;
-  for (int w = wv; w < nw; w += kBoxThreads / 64) {
-    const int i = 64 * w + lane;
-    const int c = i < nt ? (sorted ? skeys[i] : a.cnt[sb + i]) : 0;
-    esum += 64 * int64_t(wave_max(c));
-  }
-  if (lane == 0) s_e[wv] = esum;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int64_t e = 0;
-#pragma unroll
-    for (int w = 0; w < kBoxThreads / 64; ++w) e += s_e[w];
-    b.ecnt[brick] = e;
-    b.cnt[brick] = staged ? total : 0;
-  }
-}
-
-// Largest staged record count and most targets of any brick (one block; a
-// reduction instead of an atomic per brick on the same two words).
-constexpr int kMaxThreads = 1024;
-__global__ void __launch_bounds__(kMaxThreads) k_box_max(BoxArgs b, int64_t nbricks) {
-  __shared__ int32_t s_m[3][kMaxThreads / 64];
-  int mr = 0, mt = 0, nu = 0;  // nu: bricks with targets that are not staged
-  for (int64_t k = threadIdx.x; k < nbricks; k += kMaxThreads) {
-    const int nt = b.cs[(k + 1) * kBrickCells] - b.cs[k * kBrickCells];
-    mr = max(mr, int(b.cnt[k]));
-    mt = max(mt, nt);
-    nu += nt > 0 && b.cnt[k] == 0 ? 1 : 0;
-  }
-  mr = wave_max(mr);
-  mt = wave_max(mt);
-  nu = wave_sum(nu);
-  if ((threadIdx.x & 63) == 0) {
-    s_m[0][threadIdx.x >> 6] = mr;
-    s_m[1][threadIdx.x >> 6] = mt;
-    s_m[2][threadIdx.x >> 6] = nu;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kMaxThreads / 64; ++w) {
-      mr = max(mr, s_m[0][w]);
-      mt = max(mt, s_m[1][w]);
-      nu += s_m[2][w];
-    }
-    b.maxrec[0] = mr;
-    b.maxrec[1] = mt;
-    b.maxrec[2] = nu;
-  }
-}
-
 // Records of staged bricks, the entry layout of every brick's targets, and
 // in staged bricks each entry's neighbour record number.
 template <bool BATCH>
@@ -673,17 +581,33 @@ __global__ void __launch_bounds__(kBoxThreads) k_box_fill(PairArgs a, BoxArgs b)
   int32_t* cst = cfirst + b.cells_cap;                                 // [cells_cap + 1] record start of each box cell
   int32_t* wpre = cst + b.cells_cap + 1;                               // [waves_cap + 1] entry rows before each wave
   __shared__ int32_t s_w[kBoxThreads / 64];
+  __shared__ uint16_t s_st[kStencilTab];
   const int64_t brick = blockIdx.x;
   const int64_t c0 = brick * kBrickCells;
   const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
   if (sb >= se) return;
   const int nt = se - sb;
+  const StencilRow* rows = b.rows;
+  int nrows = b.nrows;
+  if constexpr (BATCH) {
+    const SysGrid& S = a.sys[a.sys_slot[sb]];
+    rows += S.row_off;
+    nrows = S.nrows;
+  }
+  const bool waves = wave_walk(nt, nrows);
+  int t0, t1;  // this block's share of the targets
+  brick_share(nt, waves, t0, t1);
+  if (t0 >= t1) return;  // uniform over the block
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int64_t r0 = b.off[brick];
   const int nrec = int(b.off[brick + 1] - r0);
   BoxGeom B;
   box_init(B, a, b.reach, brick, sb);
+  BoxStencil st;
+  st.t = s_st;
+  st.ok = false;
   if (nrec > 0) {
+    st.init(B, rows, nrows);
     // (1) first slots and record starts of the box cells (the total is nrec),
     // (2) the records: record i lies in the last box cell whose start is <= i
     stage_box_cells<kBoxThreads>(B, b.cs, cfirst, cst, s_w);
@@ -718,8 +642,10 @@ __global__ void __launch_bounds__(kBoxThreads) k_box_fill(PairArgs a, BoxArgs b)
         B.xyz(lo[u], x, y, z);
         const uint32_t packed = box_pack(x, y, z);
         const float4 rec = make_float4(p[u].x, p[u].y, p[u].z, __uint_as_float(packed));
-        b.slot[r0 + i] = uint32_t(t[u]);
-        b.pos[r0 + i] = rec;
+        if (t0 == 0) {
+          b.slot[r0 + i] = uint32_t(t[u]);
+          b.pos[r0 + i] = rec;
+        }
         rpos[i] = rec;
       }
     }
@@ -742,75 +668,77 @@ __global__ void __launch_bounds__(kBoxThreads) k_box_fill(PairArgs a, BoxArgs b)
     }
   }
   __syncthreads();
-  // (4) the entries of the staged bricks' targets: the neighbour's record
-  // number of every kept pair (outside the table's zero interval at the
-  // FP32C displacement, formed exactly as the list-order kernel forms it),
-  // walking the stencil through the box records in LDS (list order,
-  // box_walk); the targets of other bricks keep their entry offset only.
+  // (4) the entries of the staged bricks' targets, in record order: the
+  // neighbour's record number of every kept pair (outside the table's zero
+  // interval at the FP32C displacement, formed exactly as the list-order
+  // kernel forms it); FP64: of every pair, at its position in the lists'
+  // slice layout.  The targets of other bricks keep their entry offset only.
   const float hx = B.h[0], hy = B.h[1], hz = B.h[2];
-  const StencilRow* rows = b.rows;
-  int nrows = b.nrows;
-  if constexpr (BATCH) {
-    const SysGrid& S = a.sys[a.sys_slot[sb]];
-    rows += S.row_off;
-    nrows = S.nrows;
+  const bool all = b.fp64 != 0;
+  struct Target {
+    float4 po;
+    uint32_t kb;
+    int q, z, self;
+  };
+  auto target = [&](int64_t s) {
+    Target T;
+    T.po = a.pc32[s];
+    const uint32_t co = __float_as_uint(T.po.w);
+    const int x = int(co & ((1u << kCellBitsX) - 1)) - B.ox;
+    const int y = int((co >> kCellBitsX) & ((1u << kCellBitsY) - 1)) - B.oy;
+    T.z = int(co >> (kCellBitsX + kCellBitsY)) - B.oz;
+    T.kb = 0x808080u - box_pack(x, y, T.z);
+    T.q = (T.z * B.ey + y) * B.ex + x;
+    T.self = cst[T.q] + int(s - cfirst[T.q]);  // the target's own record
+    return T;
+  };
+  auto keeps = [&](const Target& T, const float4& pt) {
+    float di, dj, dk;
+    box_diff(__float_as_uint(pt.w), T.kb, di, dj, dk);
+    const float dx = __builtin_fmaf(di, hx, pt.x - T.po.x);
+    const float dy = __builtin_fmaf(dj, hy, pt.y - T.po.y);
+    const float dz = __builtin_fmaf(dk, hz, pt.z - T.po.z);
+    float y;
+    return fp32c_kept(a.ct, fp32c_interval(a.ct, fp32c_r2(dx, dy, dz), y));
+  };
+  auto entries = [&](int64_t s, int64_t bb) { return b.idx + (all ? a.slice_off[s >> 6] + (s & 63) : bb); };
+  auto packed = [&](const Target& T, int64_t bb, int kept) {
+    return all ? bb : bb | (int64_t(T.self) << kSelfShift) | (int64_t(kept) << kKeptShift);
+  };
+  if (waves && nrec > 0 && st.ok) {
+    for (int i = t0 + wv; i < t1; i += kBoxThreads / 64) {  // one wave per target
+      const int32_t s = __builtin_amdgcn_readfirstlane(b.tgt[sb + i]);
+      const int64_t bb = b.eoff[brick] + 64 * int64_t(wpre[i >> 6]) + (i & 63);
+      const Target T = target(s);
+      uint16_t* __restrict__ out = entries(s, bb);
+      const int kept = wave_records(
+          B, st, cst, T.z,
+          [&](int r) {
+            const float4 pt = rpos[r];
+            return r != T.self && st.has(__float_as_uint(pt.w) + T.kb) && (all || keeps(T, pt));
+          },
+          [&](int r, int k) { out[int64_t(k) * kSlice] = uint16_t(r); });
+      if (lane == 0) b.base[sb + i] = packed(T, bb, kept);
+    }
+    return;
   }
-  for (int i = int(threadIdx.x); i < nt; i += kBoxThreads) {
+  for (int i = t0 + int(threadIdx.x); i < t1; i += kBoxThreads) {
     const int64_t s = b.tgt[sb + i];
     const int64_t bb = b.eoff[brick] + 64 * int64_t(wpre[i >> 6]) + (i & 63);
-    const float4 po = a.pc32[s];
-    const uint32_t co = __float_as_uint(po.w);
-    const int io = int(co & ((1u << kCellBitsX) - 1));
-    const int jo = int((co >> kCellBitsX) & ((1u << kCellBitsY) - 1));
-    const int ko = int(co >> (kCellBitsX + kCellBitsY));
-    // staged bricks: the target's own record, packed above the entry offset
-    const int bx = io - B.ox, by = jo - B.oy, bz = ko - B.oz;
-    const uint32_t kb = 0x808080u - box_pack(bx, by, bz);
-    int self = 0;
-    if (nrec > 0) {
-      const int qs = (bz * B.ey + by) * B.ex + bx;
-      self = cst[qs] + int(s - cfirst[qs]);
-    }
-    const int cnt = a.cnt[s];
-    if (nrec > 0 && b.fp64) {
-      // FP64: every pair, at its position in the lists' slice layout
-      int64_t o = a.slice_off[s >> 6] + (s & 63);
-      if (cnt > 0)
-        box_walk(B, rows, nrows, io, jo, ko, [&](int q0, int q1, uint32_t) {
-          for (int r = cst[q0], re = cst[q1 + 1]; r < re; ++r) {
-            if (r == self) continue;
-            b.idx[o] = uint16_t(r);
-            o += kSlice;
-          }
-        });
-      b.base[sb + i] = bb;
+    if (nrec == 0) {
+      b.base[sb + i] = bb;  // unstaged brick: the pair sum reads its list
       continue;
     }
-    if (nrec > 0) {
-      // only the kept pairs (not in the table's zero interval) are stored
-      int64_t o = bb;
-      int kept = 0;
-      if (cnt > 0)
-        box_walk(B, rows, nrows, io, jo, ko, [&](int q0, int q1, uint32_t) {
-          for (int r = cst[q0], re = cst[q1 + 1]; r < re; ++r) {
-            if (r == self) continue;
-            const float4 pt = rpos[r];
-            float di, dj, dk;
-            box_diff(__float_as_uint(pt.w), kb, di, dj, dk);
-            const float dx = __builtin_fmaf(di, hx, pt.x - po.x);
-            const float dy = __builtin_fmaf(dj, hy, pt.y - po.y);
-            const float dz = __builtin_fmaf(dk, hz, pt.z - po.z);
-            float y;
-            if (!fp32c_kept(a.ct, fp32c_interval(a.ct, fp32c_r2(dx, dy, dz), y))) continue;
-            b.idx[o] = uint16_t(r);
-            o += kSlice;
-            ++kept;
-          }
-        });
-      b.base[sb + i] = bb | (int64_t(self) << kSelfShift) | (int64_t(kept) << kKeptShift);
-      continue;
-    }
-    b.base[sb + i] = bb;  // unstaged brick: the pair sum reads its list
+    const Target T = target(s);
+    uint16_t* out = entries(s, bb);
+    int kept = 0;
+    box_walk_rec(B, rows, nrows, cst, T.q, [&](int r) {
+      if (r == T.self || !(all || keeps(T, rpos[r]))) return;
+      *out = uint16_t(r);
+      out += kSlice;
+      ++kept;
+    });
+    b.base[sb + i] = packed(T, bb, kept);
   }
 }
 
@@ -1322,10 +1250,6 @@ BoxArgs box_args(const ggem_ctx* ctx) {
   b.rows = ctx->rows_d;
   b.nrows = ctx->n_rows;
   b.cells_cap = b.waves_cap = b.recs_cap = 0;
-  b.cnt = ctx->box_cnt;
-  b.ecnt = ctx->box_ecnt;
-  b.maxrec = ctx->box_max_d;
-  b.recs = ctx->brick_recs;
   b.off = ctx->box_off;
   b.eoff = ctx->box_eoff;
   b.tgt = ctx->box_tgt;
@@ -1460,7 +1384,9 @@ hipError_t launch_cheb_nr(ggem_ctx* ctx, const PairArgs& a, int c, int nr, const
 
 template <bool E, bool B, int BLK>
 void launch_tb(ggem_ctx* ctx, const PairArgs& a) {
-  hipLaunchKernelGGL((k_tensors<E, B, BLK>), dim3(blocks_for(a.n, BLK)), dim3(BLK), 0, ctx->stream, a,
+  // threads per slot: 2^18 threads fill the chip
+  const unsigned split = unsigned(std::min<int64_t>(8, std::max<int64_t>(1, (int64_t(1) << 18) / a.n)));
+  hipLaunchKernelGGL((k_tensors<E, B, BLK>), dim3(blocks_for(a.n, BLK), split), dim3(BLK), 0, ctx->stream, a,
                      ctx->coef64);
 }
 
@@ -1498,15 +1424,7 @@ hipError_t launch_pair_tensors(ggem_ctx* ctx, int precision) {
 
 bool box_supported(const ggem_ctx* ctx) { return ctx->n > 0 && !explicit_minimg(ctx); }
 
-hipError_t launch_box_count(ggem_ctx* ctx) {
-  ProfScope ps(ctx, "box_count");
-  const BoxArgs b = box_args(ctx);
-  hipLaunchKernelGGL(k_box_count, dim3(n_bricks(ctx)), dim3(kBoxThreads), 0, ctx->stream, make_args(ctx), b);
-  hipLaunchKernelGGL(k_box_max, dim3(1), dim3(kMaxThreads), 0, ctx->stream, b, int64_t(n_bricks(ctx)));
-  return hipGetLastError();
-}
-
-hipError_t launch_box_fill(ggem_ctx* ctx, int32_t max_records, int32_t max_targets) {
+hipError_t launch_box_fill(ggem_ctx* ctx) {
   ProfScope ps(ctx, "box_fill");
   BoxArgs b = box_args(ctx);
   // LDS tables sized for the largest box and the most crowded brick
@@ -1516,15 +1434,16 @@ hipError_t launch_box_fill(ggem_ctx* ctx, int32_t max_records, int32_t max_targe
   int cap = cells(ctx->reach);
   for (int k = 0; k < ctx->nsys && ctx->nsys > 1; ++k) cap = std::max(cap, cells(ctx->sys_h[k].reach));
   b.cells_cap = std::min(cap, kBoxMaxCells);
-  b.waves_cap = (max_targets + 63) / 64;
-  b.recs_cap = max_records;
-  if (b.waves_cap > kBoxMaxWaves || max_records > kBoxMaxRecs) return hipErrorInvalidValue;
+  b.waves_cap = (ctx->max_targets + 63) / 64;
+  b.recs_cap = ctx->max_recs;
+  if (b.waves_cap > kBoxMaxWaves || b.recs_cap > kBoxMaxRecs) return hipErrorInvalidValue;
+  const unsigned split = brick_split(ctx);
   const size_t lds = sizeof(float4) * size_t(b.recs_cap) + sizeof(int32_t) * (2 * size_t(b.cells_cap) + b.waves_cap + 2);
   if (ctx->nsys > 1)
-    hipLaunchKernelGGL(k_box_fill<true>, dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream, make_args(ctx),
+    hipLaunchKernelGGL(k_box_fill<true>, dim3(n_bricks(ctx), split), dim3(kBoxThreads), lds, ctx->stream, make_args(ctx),
                        b);
   else
-    hipLaunchKernelGGL(k_box_fill<false>, dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream,
+    hipLaunchKernelGGL(k_box_fill<false>, dim3(n_bricks(ctx), split), dim3(kBoxThreads), lds, ctx->stream,
                        make_args(ctx), b);
   return hipGetLastError();
 }
