@@ -302,15 +302,6 @@ double tridiag_eig(const std::vector<double>& a, const std::vector<double>& b, i
   return 0.5 * (lo + hi);
 }
 
-// one dot product into a device scalar (no readback)
-int dot_dev(ggem_ctx* ctx, const double* a, const double* b, double* out_d) {
-  Pools& P = pools(ctx);
-  int rc = ensure(ctx, &P.red, &P.red_cap, size_t(513));
-  if (rc) return rc;
-  hipError_t e = launch_dot(ctx, 1, a, b, out_d, P.red);
-  return e == hipSuccess ? GGEM_OK : hip_fail(ctx, e, "dot");
-}
-
 }  // namespace
 
 extern "C" int ggem_cheb_brownian(ggem_ctx* ctx, const ggem_op* op, int32_t N, double eig_min,
@@ -383,54 +374,32 @@ extern "C" int ggem_cheb_brownian(ggem_ctx* ctx, const ggem_op* op, int32_t N, d
     // at a time; the device's own operator decides where to stop on the
     // device, a host operator on the host
     if (!op) {
+      const int64_t nb = apply_ref_blocks(ctx);
       if ((rc = ensure(ctx, &P.cref, &P.cref_cap, size_t(8 * nrhs)))) return rc;
-      if ((rc = ensure(ctx, &P.red, &P.red_cap, size_t(513 + 3 * 512)))) return rc;
-      if ((rc = ensure(ctx, &P.cstop, &P.cstop_cap, size_t(nrhs)))) return rc;
+      if ((rc = ensure(ctx, &P.red, &P.red_cap, size_t(3 * nb)))) return rc;
+      if ((rc = ensure(ctx, &P.cstop, &P.cstop_cap, size_t(nrhs + 1)))) return rc;
     }
     for (int r = 0; r < nrhs && !op; ++r) {
       SlotVec a0 = offset(x0, r, n), a1 = offset(x1, r, n);
       const SlotVec ay = offset(yv, r, n), am = offset(dwm, r, n);
       double* st = P.cref + 8 * r;
-      int32_t* stop = P.cstop + r;
-      double* px = P.red + 513;  // partials: x . x, then (M y).(M y) and y . y
-      double* pmy = px + 512;
-      if ((e = launch_cheb_ref_init(ctx, st, stop)) != hipSuccess) return hip_fail(ctx, e, "chebyshev");
-      if ((rc = apply(1, a0, a1, plain))) return rc;  // x1 = M x0
-      if ((rc = dot_dev(ctx, a1.soa, a0.soa, st + 0))) return rc;
-      if ((e = launch_axpby(ctx, len, db, a0.soa, da, a1.soa)) != hipSuccess) return hip_fail(ctx, e, "axpby");
-      if ((rc = refresh(ctx, 1, a1))) return rc;
-      if ((e = launch_fill(ctx, len, 0.0, ay.soa)) != hipSuccess) return hip_fail(ctx, e, "fill");
-      if ((e = launch_axpby(ctx, len, X[0], a0.soa, 1.0, ay.soa)) != hipSuccess) return hip_fail(ctx, e, "axpy");
-      if ((rc = dot_dev(ctx, ay.soa, ay.soa, st + 1))) return rc;
-      if ((e = launch_axpby(ctx, len, X[1], a1.soa, 1.0, ay.soa)) != hipSuccess) return hip_fail(ctx, e, "axpy");
-      if ((e = launch_dot_partial(ctx, a1.soa, a1.soa, px)) != hipSuccess) return hip_fail(ctx, e, "dot");
-      if ((rc = refresh(ctx, 1, ay))) return rc;
-      if ((rc = apply(1, ay, am, plain))) return rc;
-      if ((e = launch_dot2_partial(ctx, am.soa, am.soa, ay.soa, ay.soa, pmy)) != hipSuccess ||
-          (e = launch_cheb_ref_term(ctx, st, stop, px, pmy, std::fabs(X[1]), tol, 1, 0)) != hipSuccess)
-        return hip_fail(ctx, e, "chebyshev");
-      ChebEpi skip_plain = plain;
-      skip_plain.skip = stop;
-      // terms are launched up to two past the last call's stop; one small
+      int32_t *stop = P.cstop + 1 + r, *ticket = P.cstop;
+      if ((e = launch_cheb_ref_init(ctx, st, stop, ticket)) != hipSuccess) return hip_fail(ctx, e, "chebyshev");
+      // terms are launched up to one past the last call's stop; one small
       // readback then tells whether the rest are needed (terms launched after
       // the stop return at entry, so the results do not depend on the guess)
-      const int guess = std::min(N, std::max(2, ctx->cheb_terms + 2));
-      for (int i = 1; i < N; ++i) {
-        if (i == guess) {
+      const int guess = std::max(2, ctx->cheb_terms + 2);
+      for (int k = 0; k <= N; ++k) {
+        if (k == guess) {
           int64_t stopped = 0;
           if ((rc = peek(ctx, {{stop, 4}}, &stopped))) return rc;
           if (stopped) break;
         }
-        // y . y before the term is in st[1] (from the previous term)
-        ChebEpi stp{2, da, db, X[i + 1], a0, ay.soa};
-        stp.skip = stop;
-        if ((rc = apply(1, a1, a0, stp))) return rc;  // a0 <- x_{k+1}; y += c x_{k+1}
-        if ((e = launch_dot_partial(ctx, a0.soa, a0.soa, px)) != hipSuccess) return hip_fail(ctx, e, "dot");
-        if ((rc = refresh(ctx, 1, ay))) return rc;
-        if ((rc = apply(1, ay, am, skip_plain))) return rc;
-        if ((e = launch_dot2_partial(ctx, am.soa, am.soa, ay.soa, ay.soa, pmy)) != hipSuccess ||
-            (e = launch_cheb_ref_term(ctx, st, stop, px, pmy, std::fabs(X[i + 1]), tol, i + 1, 1)) != hipSuccess)
-          return hip_fail(ctx, e, "chebyshev");
+        // term k: y += c_k x_k, x_{k+1} into x_{k-1}'s storage
+        ChebEpi t{2, da, db, 0.0, k ? a1 : none, ay.soa};
+        t.skip = stop;
+        t.ref = RefEpi{X[k], am.soa, P.red, ticket, st, stop, tol, k, k >= 2 ? 1 : 0};
+        if ((e = launch_apply_ref(ctx, prec, a0, a1, t)) != hipSuccess) return hip_fail(ctx, e, "apply");
         std::swap(a0, a1);
       }
     }

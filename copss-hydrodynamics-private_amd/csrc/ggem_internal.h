@@ -472,6 +472,23 @@ enum Epi : int {
   EPI_LOCAL = 0,     // out[3p+c] = U_loc  (p = particle id, interleaved)
   EPI_MOBILITY = 1,  // out[3p+c] = U_glob + U_loc - coeff_1 f + f (type rules)
   EPI_CHEB = 2,      // Chebyshev step on slot vectors (ChebEpi)
+  EPI_REF = 3,       // ... of the reference mode, with its estimators (RefEpi)
+};
+// The reference mode's term k (one operand): m = M x_k gives y += c_k x_k,
+// M y += c_k m and x_{k+1}, so the estimators of term k need no application
+// of their own (M y is the same combination of the M x_j as y is of the
+// x_j).  Every block of the pair sum leaves its part of three dot products
+// and the last block to finish adds them in block order, forms the
+// estimators and decides (brownian_system.C:1030-1155).
+struct RefEpi {
+  double c;         // c_k
+  double* my;       // [3][n] M y so far
+  double* part;     // [3][blocks] each block's part of (M y).(M y) (term 0: (M x0).x0), y.y and x_k.x_k
+  int32_t* ticket;  // blocks done (zero between launches)
+  double* st;       // [8] (M x0).x0, y.y of the last term, -, -, err1, err2, terms, converged
+  int32_t* stop;
+  double tol;
+  int32_t term, check;
 };
 struct ChebEpi {
   int kind;            // 0: v = M x; 1: v = db x + da M x; 2: v = 2db x + 2da M x - x_{k-1}, y += c v
@@ -495,6 +512,7 @@ struct ChebEpi {
   // non-null: the launch does nothing while *skip is set (the reference
   // mode's recurrence after its stopping rule fired on the device)
   const int32_t* skip = nullptr;
+  RefEpi ref{};  // EPI_REF
 };
 // pair tensors of every list entry for the given precision
 hipError_t launch_pair_tensors(ggem_ctx* ctx, int precision);
@@ -506,6 +524,10 @@ hipError_t launch_pair_beads(ggem_ctx* ctx, int precision, int epi, const double
                              double* out);
 hipError_t launch_pair_points(ggem_ctx* ctx, int precision, int64_t m, const double* pts,
                               const int32_t* elem, double* u);
+// one term of the reference mode (EPI_REF) for one slot vector, and the
+// most blocks any launch shape of it has (the length of RefEpi::part / 3)
+hipError_t launch_apply_ref(ggem_ctx* ctx, int precision, const SlotVec& x, const SlotVec& v, const ChebEpi& epi);
+int64_t apply_ref_blocks(const ggem_ctx* ctx);
 // v = M x (+ epilogue) for nrhs slot vectors (x, v: nrhs consecutive SlotVecs
 // of stride 3n / n)
 hipError_t launch_apply(ggem_ctx* ctx, int precision, int nrhs, const SlotVec& x, const SlotVec& v,
@@ -546,15 +568,8 @@ hipError_t launch_cheb_init_y(ggem_ctx* ctx, int nrhs, const double* x0, const d
 hipError_t launch_dot(ggem_ctx* ctx, int nrhs, const double* a, const double* b, double* out_d,
                       double* partials);
 hipError_t launch_axpby(ggem_ctx* ctx, int64_t len, double a, const double* x, double b, double* y);
-// partials of one dot product of 3n slot vectors (512 doubles) or of two
-// (1024), and the reference mode's per-term estimators and stopping rule
-// over them (state st[8] and stop flag per right-hand side)
-hipError_t launch_dot_partial(ggem_ctx* ctx, const double* a, const double* b, double* partials);
-hipError_t launch_dot2_partial(ggem_ctx* ctx, const double* a1, const double* b1, const double* a2, const double* b2,
-                               double* partials);
-hipError_t launch_cheb_ref_init(ggem_ctx* ctx, double* st, int32_t* stop);
-hipError_t launch_cheb_ref_term(ggem_ctx* ctx, double* st, int32_t* stop, const double* px, const double* pmy,
-                                double xabs, double tol, int term, int check);
+// clears the reference mode's state (st[8], stop flag, block ticket)
+hipError_t launch_cheb_ref_init(ggem_ctx* ctx, double* st, int32_t* stop, int32_t* ticket);
 // batched contexts: out_d[k] = a . b over system k's slots ([3][n] vectors)
 hipError_t launch_seg_dot(ggem_ctx* ctx, const double* a, const double* b, double* out_d);
 // w -= ca[k] x + cb[k] y, out = sc[k] x on the slots of system k

@@ -222,8 +222,40 @@ template <int NR, int EPI>
 __device__ __forceinline__ void apply_epilogue(const PairArgs& a, int64_t s, const double (&acc)[NR][3],
                                                const double* __restrict__ xsoa, const SlotVec& v,
                                                const ChebEpi& epi, const double* __restrict__ u_glob,
-                                               double* __restrict__ out) {
+                                               double* __restrict__ out, double (&dots)[3]) {
   const int64_t n = a.n;
+  if constexpr (EPI == EPI_REF) {
+    static_assert(NR == 1, "the reference mode takes one vector at a time");
+    const RefEpi& R = epi.ref;
+    double nv[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int64_t idx = int64_t(q) * n + s;
+      const double xv = xsoa[idx];
+      double m = acc[0][q];
+      if (a.k.point_type == GGEM_POLYMER_BEAD) m = m - a.k.coeff_1 * xv + xv;
+      else if (a.k.point_type == GGEM_LAGRANGIAN_POINT) m = m + a.k.coeff_2 * xv;
+      else m = 0.0;
+      double y = R.c * xv, my = R.c * m;
+      if (R.term == 0) {
+        nv[q] = epi.db * xv + epi.da * m;
+        dots[0] += m * xv;
+      } else {
+        y += epi.y[idx];
+        my += R.my[idx];
+        nv[q] = 2. * epi.db * xv + 2. * epi.da * m - epi.xm1.soa[idx];
+        dots[0] += my * my;
+      }
+      dots[1] += y * y;
+      dots[2] += xv * xv;
+      epi.y[idx] = y;
+      R.my[idx] = my;
+      v.soa[idx] = nv[q];
+    }
+    if (v.g32) v.g32[s] = make_float4(float(nv[0]), float(nv[1]), float(nv[2]), 0.f);
+    if (v.g64) v.g64[s] = make_double4(nv[0], nv[1], nv[2], 0.0);
+    return;
+  }
   if (EPI == EPI_LOCAL || EPI == EPI_MOBILITY) {
     // forces are the operand: own force from the FP64 store
     const double fo[3] = {a.fs[s], a.fs[n + s], a.fs[2 * n + s]};
@@ -293,6 +325,69 @@ __device__ __forceinline__ void apply_epilogue(const PairArgs& a, int64_t s, con
   }
 }
 
+__device__ __forceinline__ double block_add(double v, double* sh) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = 0.0;
+  for (int w = 0; w < int(blockDim.x >> 6); ++w) t += sh[w];
+  __syncthreads();
+  return t;
+}
+
+// End of a reference-mode launch, the whole block with its parts of the
+// three dot products: they go to memory past the XCD's L2 (agent scope), and
+// the block that draws the last ticket adds all blocks' parts (in block
+// order, whichever block that is) and applies the stopping rule.  One launch
+// per term instead of six: per-term dot products, gather records and the
+// deciding kernel were 16 us of the 66 us a term took for 25,600 chain beads.
+__device__ __forceinline__ void ref_finish(const ChebEpi& epi, const double (&dots)[3]) {
+  __shared__ double sh[16];
+  __shared__ int s_last;
+  const RefEpi& R = epi.ref;
+  const int nb = int(gridDim.x);
+  double t[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) t[q] = block_add(dots[q], sh);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      __hip_atomic_store(R.part + int64_t(q) * nb + blockIdx.x, t[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = __hip_atomic_fetch_add(R.ticket, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+  }
+  __syncthreads();
+  if (!s_last) return;  // uniform over the block
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    double sum = 0.0;
+    for (int b = int(threadIdx.x); b < nb; b += int(blockDim.x))
+      sum += __hip_atomic_load(R.part + int64_t(q) * nb + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    t[q] = block_add(sum, sh);
+  }
+  if (threadIdx.x != 0) return;
+  *R.ticket = 0;
+  if (R.term == 0) {
+    R.st[0] = t[0];
+  } else {
+    const double aux2 = R.st[0], aux4 = sqrt(R.st[1]), aux3 = sqrt(t[2]) * fabs(R.c), aux1 = t[0];
+    double err1 = R.st[4], err2 = R.st[5];
+    if (aux2 != 0.0) err1 = sqrt(fabs(aux1 - aux2) / aux2);
+    if (aux4 != 0.0) err2 = aux3 / aux4;
+    R.st[4] = err1;
+    R.st[5] = err2;
+    R.st[6] = double(R.term);
+    if (R.check) {
+      if (err1 <= R.tol) {
+        R.st[7] = 1.0;
+        *R.stop = 1;
+      } else if (err2 <= 1E-9) {
+        *R.stop = 1;
+      }
+    }
+  }
+  R.st[1] = t[1];
+}
+
 // Output of one target: m = sum over its list of G_ij x_j for NR operand
 // vectors, then the epilogue.
 template <int P, int NR, int EPI, int BLK>
@@ -314,7 +409,8 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
     __syncthreads();
     tab = s_tab;
   }
-  if (s >= a.n) return;
+  double dots[3] = {0.0, 0.0, 0.0};
+  auto body = [&]() {
   const int64_t n = a.n;
   const int cnt = a.cnt[s];
   const int64_t base = a.slice_off[s >> 6] + (s & 63);
@@ -486,7 +582,10 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
       }
   }
 
-  apply_epilogue<NR, EPI>(a, s, acc, xsoa, v, epi, u_glob, out);
+  apply_epilogue<NR, EPI>(a, s, acc, xsoa, v, epi, u_glob, out, dots);
+  };
+  if (s < a.n) body();
+  if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
 }
 
 
@@ -804,7 +903,11 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box(PairArgs a, BoxView b
   const int64_t brick = block_index(a.xcd);
   const int64_t c0 = brick * kBrickCells;
   const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
-  if (sb >= se) return;  // no targets (uniform over the block)
+  double dots[3] = {0.0, 0.0, 0.0};
+  if (sb >= se) {  // no targets (uniform over the block)
+    if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
+    return;
+  }
   const int64_t r0 = b.off[brick];
   const int nrec = int(b.off[brick + 1] - r0);
   const int nt = se - sb;
@@ -818,8 +921,9 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box(PairArgs a, BoxView b
       const int64_t s = b.tgt[sb + i];
       double acc[1][3];
       fp32c_pairs_global(a, s, s_tab, xg, acc);
-      apply_epilogue<1, EPI>(a, s, acc, xsoa, v, epi, u_glob, out);
+      apply_epilogue<1, EPI>(a, s, acc, xsoa, v, epi, u_glob, out, dots);
     }
+    if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
     return;
   }
   {
@@ -931,8 +1035,9 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box(PairArgs a, BoxView b
       kh[q].add(ps[q]);
       acc[0][q] = kh[q].value();
     }
-    apply_epilogue<1, EPI>(a, s, acc, xsoa, v, epi, u_glob, out);
+    apply_epilogue<1, EPI>(a, s, acc, xsoa, v, epi, u_glob, out, dots);
   }
+  if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
 }
 
 
@@ -1063,7 +1168,8 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box_nr(PairArgs a, BoxVie
         kh[r][q].add(ps[r][q]);
         acc[r][q] = kh[r][q].value();
       }
-    apply_epilogue<NR, EPI>(a, s, acc, xsoa, v, epi, u_glob, out);
+    double dots[3];
+    apply_epilogue<NR, EPI>(a, s, acc, xsoa, v, epi, u_glob, out, dots);
   }
 }
 
@@ -1084,7 +1190,11 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box64(PairArgs a, BoxView
   const int64_t brick = block_index(a.xcd);
   const int64_t c0 = brick * kBrickCells;
   const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
-  if (sb >= se) return;  // no targets (uniform over the block)
+  double dots[3] = {0.0, 0.0, 0.0};
+  if (sb >= se) {  // no targets (uniform over the block)
+    if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
+    return;
+  }
   const int64_t r0 = b.off[brick];
   const int nrec = int(b.off[brick + 1] - r0);
   const int nt = se - sb;
@@ -1142,8 +1252,9 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box64(PairArgs a, BoxView
         fp64_acc(cf[int64_t(k) * kSlice], sg, xg[lst[int64_t(k) * kSlice] & kSlotMask], ps[0], ps[1], ps[2]);
     }
     const double acc[1][3] = {{ps[0], ps[1], ps[2]}};
-    apply_epilogue<1, EPI>(a, s, acc, xsoa, v, epi, u_glob, out);
+    apply_epilogue<1, EPI>(a, s, acc, xsoa, v, epi, u_glob, out, dots);
   }
+  if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
 }
 
 // Field points: sum over the element's particle list, own element
@@ -1483,6 +1594,21 @@ hipError_t launch_pair_points(ggem_ctx* ctx, int precision, int64_t m, const dou
     hipLaunchKernelGGL(k_pair_points<GGEM_FP32C>, dim3(blocks_for(m)), dim3(kBlock), 0, ctx->stream, a,
                        ctx->rows_d, ctx->n_rows, ctx->cell_start, ctx->fg32, ctx->fg64, m, pts, elem, u);
   return hipGetLastError();
+}
+
+int64_t apply_ref_blocks(const ggem_ctx* ctx) {
+  return std::max<int64_t>(blocks_for(ctx->n, 64), n_bricks(ctx));
+}
+
+hipError_t launch_apply_ref(ggem_ctx* ctx, int precision, const SlotVec& x, const SlotVec& v, const ChebEpi& epi) {
+  if (ctx->n == 0) return hipSuccess;
+  const PairArgs a = make_args(ctx);
+  // (the term updates y in place: the pick of plain applications serves)
+  const int c = tune_lookup(ctx, tune_key("apply", precision, 1, ctx->n), apply_default(ctx, precision, 1));
+  ProfScope ps(ctx, precision == GGEM_FP64 ? "apply_fp64" : "apply_fp32c");
+  return precision == GGEM_FP64
+             ? launch_k<GGEM_FP64, 1, EPI_REF>(ctx, a, c, x.g64, x.g32, x.soa, v, epi, nullptr, nullptr)
+             : launch_k<GGEM_FP32C, 1, EPI_REF>(ctx, a, c, x.g64, x.g32, x.soa, v, epi, nullptr, nullptr);
 }
 
 hipError_t launch_apply(ggem_ctx* ctx, int precision, int nrhs, const SlotVec& x, const SlotVec& v,
