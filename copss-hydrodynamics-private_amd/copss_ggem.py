@@ -387,6 +387,9 @@ def hex20_box_mesh(cfg):
 class Context:
     """One GGEM context on one HIP device (PointMesh + GGEMStokes + BrownianSystem state).
 
+    Output arrays are allocated unset: a call that returns has filled them
+    (zeroing 26 MB of fresh pages first cost 0.6 ms).
+
     cfg: one workload dict, or a list of them for a batch of independent
     suspensions in one context (see BatchContext)."""
 
@@ -464,7 +467,7 @@ class Context:
         self._c(lib().ggem_update_positions(self._h, _p(x), _p(ff)))
 
     def elem_ids(self):
-        e = np.zeros(self.n, np.int32)
+        e = np.empty(self.n, np.int32)
         self._c(lib().ggem_get_elem_ids(self._h, _p(e)))
         return e
 
@@ -474,38 +477,38 @@ class Context:
         return v.value
 
     def neighbor_csr(self):
-        off = np.zeros(self.n + 1, np.int64)
+        off = np.empty(self.n + 1, np.int64)
         self._c(lib().ggem_get_neighbor_csr(self._h, _p(off), None))
-        ids = np.zeros(max(int(off[-1]), 1), np.int32)
+        ids = np.empty(max(int(off[-1]), 1), np.int32)
         self._c(lib().ggem_get_neighbor_csr(self._h, _p(off), _p(ids)))
         return off, ids[: int(off[-1])]
 
     def elem_point_csr(self, e0=0, ne=None):
         ne = self.n_elem - e0 if ne is None else ne
-        off = np.zeros(ne + 1, np.int64)
+        off = np.empty(ne + 1, np.int64)
         self._c(lib().ggem_get_elem_point_csr(self._h, e0, ne, _p(off), None))
-        ids = np.zeros(max(int(off[-1]), 1), np.int32)
+        ids = np.empty(max(int(off[-1]), 1), np.int32)
         self._c(lib().ggem_get_elem_point_csr(self._h, e0, ne, _p(off), _p(ids)))
         return off, ids[: int(off[-1])]
 
     def elem_point_pairs(self):
         """sum over elements of the element-point list length (spreading pairs / nqp)."""
-        off = np.zeros(self.n_elem + 1, np.int64)
+        off = np.empty(self.n_elem + 1, np.int64)
         self._c(lib().ggem_get_elem_point_csr(self._h, 0, self.n_elem, _p(off), None))
         return int(off[-1])
 
     def local_velocity_beads(self, out=True):
-        u = np.zeros((self.n, 3)) if out else None
+        u = np.empty((self.n, 3)) if out else None
         self._c(lib().ggem_local_velocity_beads(self._h, _p(u)))
         return u
 
     def global_self_exclusion(self):
-        u = np.zeros((self.n, 3))
+        u = np.empty((self.n, 3))
         self._c(lib().ggem_global_self_exclusion(self._h, _p(u)))
         return u
 
     def combine_velocity(self, u_glob=None, out=True):
-        U = np.zeros((self.n, 3)) if out else None
+        U = np.empty((self.n, 3)) if out else None
         ug = None if u_glob is None else _f64(u_glob, (-1, 3))
         self._c(lib().ggem_combine_velocity(self._h, _p(ug), _p(U)))
         return U
@@ -518,14 +521,14 @@ class Context:
     def global_velocity_beads(self, node_u):
         """U_glob of every bead from the nodal velocity node_u[n_nodes, 3]."""
         nu = _f64(node_u, (-1, 3))
-        u = np.zeros((self.n, 3))
+        u = np.empty((self.n, 3))
         self._c(lib().ggem_global_velocity_beads(self._h, _p(nu), _p(u)))
         return u
 
     def combine_velocity_fe(self, node_u, out=True):
         """combine_velocity with U_glob interpolated on the device from node_u."""
         nu = _f64(node_u, (-1, 3))
-        U = np.zeros((self.n, 3)) if out else None
+        U = np.empty((self.n, 3)) if out else None
         self._c(lib().ggem_combine_velocity_fe(self._h, _p(nu), _p(U)))
         return U
 
@@ -533,7 +536,7 @@ class Context:
                    rcut=2.0 ** (1.0 / 6.0), out=True):
         """FENE chains + LJ slit walls from the current positions; they become the context's forces."""
         fp = FixParams(int(chain_beads), int(bool(walls)), k, b_max, eps, sigma, rcut)
-        f = np.zeros((self.n, 3)) if out else None
+        f = np.empty((self.n, 3)) if out else None
         self._c(lib().ggem_fix_forces(self._h, C.byref(fp), _p(f)))
         return f
 
@@ -556,14 +559,14 @@ class Context:
             arr[i].type = int(typ)
             for k, v in enumerate(p):
                 arr[i].p[k] = float(v)
-        f = np.zeros((self.n, 3)) if out else None
+        f = np.empty((self.n, 3)) if out else None
         self._c(lib().ggem_apply_fixes(self._h, len(fixes), arr, _p(f)))
         return f
 
     def spread_nodes(self, nqp_1d, IF, n_nodes):
         """Spreading summed into one force per node of the velocity mesh: [n_nodes, 3]."""
         IF = _f64(IF).ravel()
-        F = np.zeros((int(n_nodes), 3))
+        F = np.empty((int(n_nodes), 3))
         self._c(lib().ggem_spread_nodes(self._h, nqp_1d, _p(IF), _p(F)))
         return F
 
@@ -571,7 +574,7 @@ class Context:
         """Element vectors Fe[n_elem, 3, 20] after the spreading (or inlet
         traction) and the wall penalty rows; opts from rhs_opts()."""
         IF = None if IF is None else _f64(IF).ravel()
-        Fe = np.zeros((self.n_elem, 3, 20))
+        Fe = np.empty((self.n_elem, 3, 20))
         self._c(lib().ggem_assemble_elem_rhs(self._h, nqp_1d, _p(IF), C.byref(opts), _p(Fe)))
         return Fe
 
@@ -580,14 +583,14 @@ class Context:
         mesh, periodic images condensed onto the min faces when condense
         (out=False: kept on the device)."""
         IF = None if IF is None else _f64(IF).ravel()
-        F = np.zeros((int(n_nodes), 3)) if out else None
+        F = np.empty((int(n_nodes), 3)) if out else None
         self._c(lib().ggem_assemble_rhs(self._h, nqp_1d, _p(IF), C.byref(opts), int(bool(condense)), _p(F)))
         return F
 
     def local_velocity_points(self, pts, elem=None):
         pts = _f64(pts, (-1, 3))
         el = None if elem is None else np.ascontiguousarray(elem, dtype=np.int32)
-        u = np.zeros_like(pts)
+        u = np.empty_like(pts)
         self._c(lib().ggem_local_velocity_points(self._h, pts.shape[0], _p(pts), _p(el), _p(u)))
         return u
 
@@ -596,7 +599,7 @@ class Context:
         device allocation; at most 65536 points)."""
         pts = _f64(pts, (-1, 3))
         el = None if elem is None else np.ascontiguousarray(elem, dtype=np.int32)
-        u = np.zeros_like(pts)
+        u = np.empty_like(pts)
         self._c(lib().ggem_local_velocity_points_noalloc(self._h, pts.shape[0], _p(pts), _p(el), _p(u)))
         return u
 
@@ -604,15 +607,15 @@ class Context:
         nqp = nqp_1d ** 3
         IF = _f64(IF).ravel()
         n_u = IF.size // nqp
-        rho = np.zeros((self.n_elem, nqp, 3)) if want_rho else None
-        Fe = np.zeros((self.n_elem, 3, n_u)) if want_fe else None
+        rho = np.empty((self.n_elem, nqp, 3)) if want_rho else None
+        Fe = np.empty((self.n_elem, 3, n_u)) if want_fe else None
         self._c(lib().ggem_spread(self._h, nqp_1d, n_u, _p(IF), _p(rho), _p(Fe)))
         return rho, Fe
 
     def mobility_apply(self, f):
         """u = M f; f None: the context's current forces."""
         f = None if f is None else _f64(f, (-1, 3))
-        u = np.zeros((self.n, 3))
+        u = np.empty((self.n, 3))
         self._c(lib().ggem_mobility_apply(self._h, _p(f), _p(u)))
         return u
 
@@ -632,8 +635,8 @@ class Context:
             nrhs = dw.size // (3 * self.n)
             dw = dw.reshape(nrhs, self.n, 3)
         shape = (nrhs, self.n, 3)
-        y = np.zeros(shape) if want_y else None
-        disp = np.zeros(shape) if want_disp else None
+        y = np.empty(shape) if want_y else None
+        disp = np.empty(shape) if want_disp else None
         info = (ChebInfo * nrhs)()
         opp = None
         if op is not None:
@@ -648,15 +651,15 @@ class Context:
     def get_brownian(self):
         """(y, disp) kept by cheb_brownian(..., keep=True) / displacement_apply: [nrhs, n, 3] each."""
         nrhs = max(int(getattr(self, "_keep_nrhs", 1)), 1)
-        y = np.zeros((nrhs, self.n, 3))
-        d = np.zeros((nrhs, self.n, 3))
+        y = np.empty((nrhs, self.n, 3))
+        d = np.empty((nrhs, self.n, 3))
         self._c(lib().ggem_get_brownian(self._h, _p(y), _p(d)))
         return y, d
 
     def displacement_apply(self, out=True):
         """disp = M y with the kept y at the current positions (hi_ewald at the mid-point)."""
         nrhs = max(int(getattr(self, "_keep_nrhs", 1)), 1)
-        d = np.zeros((nrhs, self.n, 3)) if out else None
+        d = np.empty((nrhs, self.n, 3)) if out else None
         self._c(lib().ggem_displacement_apply(self._h, _p(d)))
         return d
 
@@ -669,13 +672,13 @@ class Context:
 
     def noise_draw(self, dt, out=True):
         """Next sqrt(2) N(0, sqrt(dt)) vector; it becomes the device noise (nrhs 1)."""
-        dw = np.zeros((self.n, 3)) if out else None
+        dw = np.empty((self.n, 3)) if out else None
         self._c(lib().ggem_noise_draw(self._h, dt, _p(dw)))
         self._noise_nrhs = 1
         return dw
 
     def get_noise(self):
-        dw = np.zeros((int(getattr(self, "_noise_nrhs", 1)), self.n, 3))
+        dw = np.empty((int(getattr(self, "_noise_nrhs", 1)), self.n, 3))
         self._c(lib().ggem_get_noise(self._h, _p(dw)))
         return dw
 
@@ -695,9 +698,9 @@ class Context:
 
     def get_positions(self):
         """(positions, unwrapped positions, image counts) [n, 3] each."""
-        x = np.zeros((self.n, 3))
-        r = np.zeros((self.n, 3))
-        im = np.zeros((self.n, 3), np.int32)
+        x = np.empty((self.n, 3))
+        r = np.empty((self.n, 3))
+        im = np.empty((self.n, 3), np.int32)
         self._c(lib().ggem_get_positions(self._h, _p(x), _p(r), _p(im)))
         return x, r, im
 
@@ -809,8 +812,8 @@ class BatchContext(Context):
         lo = _f64(np.broadcast_to(np.asarray(eig_min, dtype=np.float64), (self.nsys,)).copy())
         hi = _f64(np.broadcast_to(np.asarray(eig_max, dtype=np.float64), (self.nsys,)).copy())
         shape = (nrhs, self.n, 3)
-        y = np.zeros(shape) if want_y else None
-        disp = np.zeros(shape) if want_disp else None
+        y = np.empty(shape) if want_y else None
+        disp = np.empty(shape) if want_disp else None
         self._c(lib().ggem_batch_cheb_brownian(self._h, N, _p(lo), _p(hi), nrhs, _p(dw), _p(y), _p(disp)))
         return y, disp
 

@@ -419,6 +419,12 @@ void free_all(ggem_ctx* ctx) {
   ctx->peek_h = nullptr;
   if (ctx->par_ev) (void)hipEventDestroy(ctx->par_ev);
   ctx->par_ev = nullptr;
+  if (ctx->read_h) (void)hipHostFree(ctx->read_h);
+  ctx->read_h = nullptr;
+  for (hipEvent_t& ev : ctx->read_ev) {
+    if (ev) (void)hipEventDestroy(ev);
+    ev = nullptr;
+  }
   if (ctx->cheb_exec) (void)hipGraphExecDestroy(ctx->cheb_exec);
   ctx->cheb_exec = nullptr;
   if (ctx->scratch) {
@@ -460,6 +466,47 @@ int grow_scan64(ggem_ctx* ctx, int64_t len) {
 }
 
 }  // namespace
+
+int ggem::d2h(ggem_ctx* ctx, void* host, const void* dev, size_t bytes) {
+  static_assert(kReadBufs == sizeof(ctx->read_ev) / sizeof(ctx->read_ev[0]), "an event per buffer");
+  if (bytes == 0) return sync(ctx);
+  const size_t want = bytes <= kReadChunk ? bytes : kReadChunk * kReadBufs;
+  if (ctx->read_cap < want) {
+    if (ctx->read_h) GGEM_HIP(ctx, hipHostFree(ctx->read_h));
+    ctx->read_h = nullptr;
+    ctx->read_cap = 0;
+    const size_t cap = std::min(kReadChunk * kReadBufs, std::max(want, size_t(1) << 16));
+    GGEM_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->read_h), cap));
+    ctx->read_cap = cap;
+  }
+  char* const to = static_cast<char*>(host);
+  const char* const from = static_cast<const char*>(dev);
+  if (bytes <= kReadChunk) {
+    GGEM_HIP(ctx, hipMemcpyAsync(ctx->read_h, from, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    const int rc = sync(ctx);
+    if (!rc) std::memcpy(to, ctx->read_h, bytes);
+    return rc;
+  }
+  for (hipEvent_t& ev : ctx->read_ev)
+    if (!ev) GGEM_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  const size_t n = (bytes + kReadChunk - 1) / kReadChunk;
+  auto part = [&](size_t i) { return std::min(kReadChunk, bytes - i * kReadChunk); };
+  auto fetch = [&](size_t i) {
+    hipError_t e = hipMemcpyAsync(ctx->read_h + (i % kReadBufs) * kReadChunk, from + i * kReadChunk, part(i),
+                                  hipMemcpyDeviceToHost, ctx->stream);
+    return e != hipSuccess ? e : hipEventRecord(ctx->read_ev[i % kReadBufs], ctx->stream);
+  };
+  hipError_t e = hipSuccess;
+  for (size_t i = 0; i < size_t(kReadBufs) && i < n && e == hipSuccess; ++i) e = fetch(i);
+  for (size_t i = 0; i < n && e == hipSuccess; ++i) {
+    if ((e = hipEventSynchronize(ctx->read_ev[i % kReadBufs])) != hipSuccess) break;
+    std::memcpy(to + i * kReadChunk, ctx->read_h + (i % kReadBufs) * kReadChunk, part(i));
+    if (i + kReadBufs < n) e = fetch(i + kReadBufs);
+  }
+  if (e == hipSuccess) return GGEM_OK;
+  (void)hipStreamSynchronize(ctx->stream);  // nothing may still write the buffers
+  return hip_fail(ctx, e, "device-to-host copy");
+}
 
 int ggem::peek(ggem_ctx* ctx, std::initializer_list<std::pair<const void*, int32_t>> items, int64_t* out) {
   if (items.size() > size_t(kPeekMax)) return fail(ctx, GGEM_ERR_INVALID_ARG, "too many values to read back");

@@ -96,10 +96,14 @@ inline int sync(ggem_ctx* ctx) {
   return GGEM_OK;
 }
 
-inline int d2h(ggem_ctx* ctx, void* host, const void* dev, size_t bytes) {
-  GGEM_HIP(ctx, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
-  return sync(ctx);
-}
+// Device to host.  The caller's array is pageable: the runtime's own copy
+// of 26 MB into it took 1.5 to 1.9 ms, a copy into pinned memory 0.46 ms and
+// one thread's memcpy from there 0.35 to 0.49 ms.  So the bytes go through
+// kReadBufs pinned buffers of the context, the copy engine filling the next
+// ones while the host empties one.
+constexpr size_t kReadChunk = size_t(512) << 10;
+constexpr int kReadBufs = 3;
+int d2h(ggem_ctx* ctx, void* host, const void* dev, size_t bytes);
 
 inline int h2d(ggem_ctx* ctx, void* dev, const void* host, size_t bytes) {
   GGEM_HIP(ctx, hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, ctx->stream));

@@ -9,12 +9,12 @@
 #include <functional>
 #include <initializer_list>
 #include <map>
-#include <random>
 #include <string>
 #include <utility>
 #include <vector>
 
 #include "copss_ggem.h"
+#include "noise_engine.h"
 
 namespace ggem {
 
@@ -251,7 +251,7 @@ struct ggem_ctx {
   int64_t noise_cap = 0;
   int32_t noise_nrhs = 0;
   // the reference's noise engine, one for the whole run (host; sequential)
-  std::default_random_engine noise_gen;
+  ggem::NoiseEngine noise_gen;
   std::vector<double> noise_h;
 
   // Brownian vectors kept on the device (GGEM_CHEB_KEEP): y and the
@@ -295,6 +295,9 @@ struct ggem_ctx {
   int32_t cheb_terms = 1 << 30;      // terms of the last reference-mode Chebyshev call (its statistics read)
   size_t par_cap = 0;
   hipEvent_t par_ev = nullptr;
+  char* read_h = nullptr;            // pinned buffers of the device-to-host copies (d2h)
+  size_t read_cap = 0;
+  hipEvent_t read_ev[3] = {nullptr, nullptr, nullptr};
 
   // force-field fixes: bonds (incidences by bead, bond order), constant
   // forces and discretized wall particles

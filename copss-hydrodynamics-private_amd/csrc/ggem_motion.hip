@@ -281,7 +281,7 @@ extern "C" {
 
 int ggem_noise_seed(ggem_ctx* ctx, uint64_t seed) {
   if (!ctx) return fail(nullptr, GGEM_ERR_INVALID_ARG, "null context");
-  ctx->noise_gen.seed(static_cast<std::default_random_engine::result_type>(seed));
+  ctx->noise_gen.seed(seed);
   return GGEM_OK;
 }
 
@@ -291,11 +291,7 @@ int ggem_noise_skip(ggem_ctx* ctx, int64_t n_vectors) {
   if (!ctx) return fail(nullptr, GGEM_ERR_INVALID_ARG, "null context");
   if (n_vectors < 0) return fail(ctx, GGEM_ERR_INVALID_ARG, "negative vector count");
   const int64_t len = 3 * ctx->n;
-  for (int64_t v = 0; v < n_vectors; ++v) {
-    std::normal_distribution<double> d(0.0, 1.0);
-    d.reset();
-    for (int64_t i = 0; i < len; ++i) (void)d(ctx->noise_gen);
-  }
+  for (int64_t v = 0; v < n_vectors; ++v) ctx->noise_gen.skip(len);
   return GGEM_OK;
 }
 
@@ -305,11 +301,9 @@ int ggem_noise_draw(ggem_ctx* ctx, double dt, double* dw) {
   const int64_t len = 3 * ctx->n;
   ctx->noise_h.resize(size_t(len));
   // random_vector_normal (random_generator.C:43-67) then VecScale(dw, sqrt 2)
-  std::normal_distribution<double> dist(0.0, std::sqrt(dt));
-  dist.reset();
-  for (int64_t i = 0; i < len; ++i) ctx->noise_h[size_t(i)] = dist(ctx->noise_gen);
-  const double s2 = std::sqrt(2.0);
-  for (auto& v : ctx->noise_h) v *= s2;
+  const double sd = std::sqrt(dt), s2 = std::sqrt(2.0);
+  double* const h = ctx->noise_h.data();
+  ctx->noise_gen.normals(len, [=](int64_t i, double v) { h[i] = v * sd * s2; });
   if (dw && len) std::copy(ctx->noise_h.begin(), ctx->noise_h.end(), dw);
   if (len == 0) return GGEM_OK;
   GGEM_HIP(ctx, hipSetDevice(ctx->device));
