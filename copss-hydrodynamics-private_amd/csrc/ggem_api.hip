@@ -198,10 +198,10 @@ int ensure_tensors(ggem_ctx* ctx, int nrhs) {
     if ((rc = prepare_box(ctx))) return rc;
     ctx->box_built = true;
   }
-  // the list-order kernels read the lists: several operands, no staged
-  // bricks (or some unstaged), and the autotuner, which times every shape
-  if (nrhs > 1 || !ctx->box_valid || ctx->box_unstaged || ctx->tune.on) return ensure_ell(ctx);
-  return GGEM_OK;
+  // the list-order kernels read the lists: no staged bricks (or some
+  // unstaged), operands whose records do not fit the LDS, and the autotuner,
+  // which times every shape
+  return apply_reads_lists(ctx, GGEM_FP32C, nrhs) ? ensure_ell(ctx) : GGEM_OK;
 }
 
 }  // namespace ggem
@@ -371,6 +371,7 @@ void free_all(ggem_ctx* ctx) {
   f(ctx->tab32);
   f(ctx->box_cnt);
   f(ctx->box_tgt);
+  f(ctx->quad_work);
   f(ctx->box_base);
   f(ctx->box_slot);
   f(ctx->box_pos);
@@ -894,6 +895,8 @@ int ensure_build(ggem_ctx* ctx) {
   ctx->box_eoff = ctx->box_cnt + 3 * ctx->box_brick_cap;
   int rc = grow_scan64(ctx, int64_t(nb) + 1);
   if (!rc) rc = ensure(ctx, &ctx->box_tgt, &ctx->box_tgt_cap, size_t(std::max<int64_t>(ctx->n, 1)));
+  // (a brick's shares are at most one more than its 64ths of the targets)
+  if (!rc) rc = ensure(ctx, &ctx->quad_work, &ctx->quad_work_cap, size_t(ctx->n / 64) + nb + 1);
   return rc;
 }
 
@@ -982,6 +985,8 @@ int ggem_build_neighbors(ggem_ctx* ctx) {
   ctx->max_recs = int32_t(v[5]);
   ctx->max_targets = int32_t(v[6]);
   ctx->unstaged = int32_t(v[7]);
+  ctx->full_bricks = int32_t(v[8]);
+  ctx->quad_items = v[9];
   if (ctx->box_recs < 0 || ctx->box_entries < 0 || ctx->ell_len < 0) {  // arrays longer than one block scans
     const int64_t nb = ctx->grid.n_cells >> (3 * kBrickBits), nsl = (ctx->n + kSlice - 1) / kSlice;
     int64_t w[3];

@@ -79,8 +79,14 @@ int ensure_keep(ggem_ctx* ctx, int nrhs) {
 }
 
 int refresh(ggem_ctx* ctx, int nrhs, const SlotVec& v) {
-  hipError_t e = launch_make_gather(ctx, nrhs, v.soa, v.g32, v.g64);
-  return e == hipSuccess ? GGEM_OK : hip_fail(ctx, e, "gather records");
+  for (int done = 0; done < nrhs;) {
+    const int nr = apply_chunk(ctx, ctx->p.precision, nrhs - done);
+    const SlotVec c = offset(v, done, ctx->n);
+    hipError_t e = launch_make_gather(ctx, nr, c.soa, c.g32, c.g64);
+    if (e != hipSuccess) return hip_fail(ctx, e, "gather records");
+    done += nr;
+  }
+  return GGEM_OK;
 }
 
 // v = M x (+ epilogue), on the device or through a host operator.
@@ -226,7 +232,8 @@ int run_fixed_graph(ggem_ctx* ctx, Applier& apply, FixedStep s) {
       uintptr_t(s.dw_dev), uintptr_t(s.dpar), uintptr_t(P.vec), uintptr_t(P.g32), uintptr_t(P.g64),
       uintptr_t(ctx->x4), uintptr_t(ctx->nbr_cnt), uintptr_t(ctx->slice_off), uintptr_t(ctx->ell),
       uintptr_t(ctx->perm), uintptr_t(ctx->fs), uintptr_t(ctx->tab32), uintptr_t(ctx->coef64),
-      uintptr_t(ctx->box_valid), uintptr_t(ctx->box_max), uintptr_t(ctx->box_cnt), uintptr_t(ctx->box_slot),
+      uintptr_t(ctx->box_valid), uintptr_t(ctx->box_unstaged), uintptr_t(ctx->box_max), uintptr_t(ctx->quad_items), uintptr_t(ctx->quad_work),
+      uintptr_t(ctx->full_bricks), uintptr_t(ctx->box_cnt), uintptr_t(ctx->box_slot),
       uintptr_t(ctx->box_pos), uintptr_t(ctx->box_idx), uintptr_t(ctx->cell_start),
       uintptr_t(ctx->box_tgt), uintptr_t(ctx->box_base),
       uintptr_t(s.sys), uintptr_t(ctx->nsys)};
@@ -369,7 +376,8 @@ extern "C" int ggem_cheb_brownian(ggem_ctx* ctx, const ggem_op* op, int32_t N, d
   } else {
     e = launch_permute_in(ctx, nrhs, dw_dev, x0.soa);
     if (e != hipSuccess) return hip_fail(ctx, e, "permute");
-    if ((rc = refresh(ctx, nrhs, x0))) return rc;
+    for (int r = 0; r < nrhs; ++r)
+      if ((rc = refresh(ctx, 1, offset(x0, r, n)))) return rc;
     // reference-compatible (brownian_system.C:1030-1155), one right-hand side
     // at a time; the device's own operator decides where to stop on the
     // device, a host operator on the host
@@ -377,13 +385,13 @@ extern "C" int ggem_cheb_brownian(ggem_ctx* ctx, const ggem_op* op, int32_t N, d
       const int64_t nb = apply_ref_blocks(ctx);
       if ((rc = ensure(ctx, &P.cref, &P.cref_cap, size_t(8 * nrhs)))) return rc;
       if ((rc = ensure(ctx, &P.red, &P.red_cap, size_t(3 * nb)))) return rc;
-      if ((rc = ensure(ctx, &P.cstop, &P.cstop_cap, size_t(nrhs + 1)))) return rc;
+      if ((rc = ensure(ctx, &P.cstop, &P.cstop_cap, size_t(nrhs + 1 + kRefGroups)))) return rc;
     }
     for (int r = 0; r < nrhs && !op; ++r) {
       SlotVec a0 = offset(x0, r, n), a1 = offset(x1, r, n);
       const SlotVec ay = offset(yv, r, n), am = offset(dwm, r, n);
       double* st = P.cref + 8 * r;
-      int32_t *stop = P.cstop + 1 + r, *ticket = P.cstop;
+      int32_t *stop = P.cstop + 1 + kRefGroups + r, *ticket = P.cstop;
       if ((e = launch_cheb_ref_init(ctx, st, stop, ticket)) != hipSuccess) return hip_fail(ctx, e, "chebyshev");
       // terms are launched up to one past the last call's stop; one small
       // readback then tells whether the rest are needed (terms launched after

@@ -92,6 +92,9 @@ __device__ __forceinline__ int wrap_axis(int x, int n) {
 __device__ __forceinline__ int div_small(int q, float inv_d) { return int((float(q) + 0.5f) * inv_d); }
 
 constexpr int kBrickCells = 1 << (3 * kBrickBits);
+// blocks that share a brick's targets in the quad pair sums
+constexpr int kQuadShare = 64, kQuadShares = 4;
+__device__ __forceinline__ int quad_shares(int nt) { return min(kQuadShares, (nt + kQuadShare - 1) / kQuadShare); }
 constexpr int kBoxMaxCells = 8192;  // box cells whose tables a brick kernel keeps in LDS
 constexpr int kBoxBits = 6;         // box coordinates: below 2^6 per axis
 constexpr int kBoxField = 8;        // ... packed one byte per axis (x, y, z from the low byte)

@@ -231,6 +231,10 @@ struct ggem_ctx {
   int32_t max_recs = 0;           // largest record count of a staged brick
   int32_t max_targets = 0;        // most targets of a brick
   int32_t unstaged = 0;           // bricks with targets that are not staged
+  int32_t full_bricks = 0;        // bricks with targets
+  uint32_t* quad_work = nullptr;  // [quad_items] brick and share of every block of the quad pair sums
+  size_t quad_work_cap = 0;
+  int64_t quad_items = 0;
   uint8_t* spread_unstaged = nullptr;  // [bricks] the brick spreading's boxes over its record table
   size_t spread_unstaged_cap = 0;
   int32_t box_max = 0;            // same on the host; 0 when no brick is staged
@@ -422,10 +426,11 @@ hipError_t launch_clear_counters(ggem_ctx* ctx);
 // per-slot counts, per-slice lengths, the total pair count and the census
 // of the staged records
 hipError_t launch_count_lists(ggem_ctx* ctx);
-// record, entry and slice offsets and the sizes a build reads back: host[8]
-// (pinned) = flag, pairs, records, entries, list slots (-1: the total at the
-// end of the scanned array), largest record count, most targets of a
-// brick, unstaged bricks
+// record, entry and slice offsets, the work list of the quad pair sums and
+// the sizes a build reads back: host[10] (pinned) = flag, pairs, records,
+// entries, list slots (-1: the total at the end of the scanned array),
+// largest record count, most targets of a brick, unstaged bricks, bricks
+// with targets, work items
 hipError_t launch_build_sizes(ggem_ctx* ctx, int64_t* host);
 // exclusive scan of int64 values; out[len] receives the total
 hipError_t launch_scan64(ggem_ctx* ctx, const int64_t* in, int64_t len, int64_t* out);
@@ -463,7 +468,9 @@ hipError_t launch_fix_forces(ggem_ctx* ctx, int32_t chain, double k, double b, i
 
 // ---- launchers (kernels_pair.hip) ----
 // A vector operand of the pair sum: FP64 SoA by slot for the element-wise
-// algebra plus a one-record-per-slot copy for the neighbour gathers.
+// algebra plus a one-record-per-slot copy for the neighbour gathers.  Of
+// several operands, each launch's (apply_chunk) lie together by slot, record
+// (s, r) of nr at s nr + r: a neighbour is one run of memory.
 struct SlotVec {
   double* soa;    // [3][n]
   float4* g32;    // [n]
@@ -483,11 +490,12 @@ enum Epi : int {
 // x_j).  Every block of the pair sum leaves its part of three dot products
 // and the last block to finish adds them in block order, forms the
 // estimators and decides (brownian_system.C:1030-1155).
+constexpr int kRefGroups = 32;
 struct RefEpi {
   double c;         // c_k
   double* my;       // [3][n] M y so far
   double* part;     // [3][blocks] each block's part of (M y).(M y) (term 0: (M x0).x0), y.y and x_k.x_k
-  int32_t* ticket;  // blocks done (zero between launches)
+  int32_t* ticket;  // [1 + kRefGroups] blocks done (zero between launches)
   double* st;       // [8] (M x0).x0, y.y of the last term, -, -, err1, err2, terms, converged
   int32_t* stop;
   double tol;
@@ -531,6 +539,10 @@ hipError_t launch_pair_points(ggem_ctx* ctx, int precision, int64_t m, const dou
 // most blocks any launch shape of it has (the length of RefEpi::part / 3)
 hipError_t launch_apply_ref(ggem_ctx* ctx, int precision, const SlotVec& x, const SlotVec& v, const ChebEpi& epi);
 int64_t apply_ref_blocks(const ggem_ctx* ctx);
+// operands of the next launch of `left`
+int apply_chunk(const ggem_ctx* ctx, int precision, int left);
+// whether some pair sum of nrhs operands reads the sliced lists (after prepare_box)
+bool apply_reads_lists(const ggem_ctx* ctx, int precision, int nrhs);
 // v = M x (+ epilogue) for nrhs slot vectors (x, v: nrhs consecutive SlotVecs
 // of stride 3n / n)
 hipError_t launch_apply(ggem_ctx* ctx, int precision, int nrhs, const SlotVec& x, const SlotVec& v,
@@ -540,7 +552,7 @@ hipError_t launch_apply(ggem_ctx* ctx, int precision, int nrhs, const SlotVec& x
 // Fe[e][j][l] (node_major: Fe[e][l][j])
 // Small device values (int32 or int64 each) written to pinned host memory
 // by one kernel, then one synchronisation; out gets them as int64.
-constexpr int kPeekMax = 8;
+constexpr int kPeekMax = 10;
 struct PeekArgs {
   const void* src[kPeekMax];
   int32_t bytes[kPeekMax];  // 4 or 8
@@ -560,7 +572,7 @@ int spread_brick_mode(ggem_ctx* ctx, int precision, int nqp_1d);
 // ---- launchers (kernels_vec.hip) ----
 hipError_t launch_permute_in(ggem_ctx* ctx, int nrhs, const double* in_interleaved, double* out_slots);
 hipError_t launch_permute_out(ggem_ctx* ctx, int nrhs, const double* in_slots, double* out_interleaved);
-// gather copies of nrhs slot SoA vectors
+// gather records of nrhs slot SoA vectors of one launch
 hipError_t launch_make_gather(ggem_ctx* ctx, int nrhs, const double* soa, float4* g32, double4* g64);
 // dpar[off .. off+cnt) = vals (kernel arguments, so safe inside a stream or graph)
 hipError_t launch_set_params(ggem_ctx* ctx, double* dpar, int64_t off, const double* vals, int cnt);

@@ -668,9 +668,10 @@ __global__ void k_scan64_add(int64_t* __restrict__ out, int64_t len, const int64
 // What a build leaves to the host, in one launch: block 0 scans the records
 // per brick, block 1 the entries per brick, block 2 the slice lengths (a
 // null input is left to launch_scan64), block 3 the maxima over the bricks
-// (records, targets, unstaged bricks with targets), the out-of-domain flag
-// and the pair count, which it clears for the next build.  The results go
-// straight to pinned host memory.
+// (records, targets, unstaged bricks with targets, bricks with targets), the
+// out-of-domain flag and the pair count, which it clears for the next build;
+// block 4 lists the quad pair sums' blocks.  The results go straight to
+// pinned host memory.
 constexpr int kSizesThreads = 1024;
 constexpr int kSizesItems = 4;
 constexpr int64_t kSizesMax = 65536;  // longest array one block scans (16 rounds)
@@ -683,12 +684,37 @@ struct SizesArgs {
   int64_t nbricks;
   int32_t* flag;
   int64_t* pairs;
-  int64_t* host;  // [8] flag, pairs, records, entries, list slots, then the maxima
+  uint32_t* work;
+  int64_t* host;  // [10] flag, pairs, records, entries, list slots, the maxima (4), work items
 };
 __global__ void __launch_bounds__(kSizesThreads) k_build_sizes(SizesArgs a) {
   __shared__ int64_t sh[kSizesThreads / 64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   constexpr int NW = kSizesThreads / 64;
+  if (blockIdx.x == 4) {
+    __shared__ int32_t s_n[NW];
+    int carry = 0;
+    for (int64_t c0 = 0; c0 < a.nbricks; c0 += kSizesThreads) {
+      const int64_t k = c0 + threadIdx.x;
+      const int m = k < a.nbricks ? quad_shares(a.cs[(k + 1) * kBrickCells] - a.cs[k * kBrickCells]) : 0;
+      int incl = m;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+      }
+      if (lane == 63) s_n[wv] = incl;
+      __syncthreads();
+      int at = carry + incl - m;
+      for (int w = 0; w < NW; ++w) {
+        if (w < wv) at += s_n[w];
+        carry += s_n[w];
+      }
+      for (int y = 0; y < m; ++y) a.work[at + y] = uint32_t(k) * kQuadShares + uint32_t(y);
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) a.host[9] = carry;
+    return;
+  }
   if (blockIdx.x < 3) {
     const int64_t* __restrict__ in = a.in[blockIdx.x];
     int64_t* __restrict__ out = a.out[blockIdx.x];
@@ -729,22 +755,25 @@ __global__ void __launch_bounds__(kSizesThreads) k_build_sizes(SizesArgs a) {
     }
     return;
   }
-  int mr = 0, mt = 0, nu = 0;
+  int mr = 0, mt = 0, nu = 0, nf = 0;
   for (int64_t k = threadIdx.x; k < a.nbricks; k += kSizesThreads) {
     const int nt = a.cs[(k + 1) * kBrickCells] - a.cs[k * kBrickCells];
     const int nr = int(a.box_cnt[k]);
     mr = max(mr, nr);
     mt = max(mt, nt);
     nu += nt > 0 && nr == 0 ? 1 : 0;
+    nf += nt > 0 ? 1 : 0;
   }
   mr = wave_max(mr);
   mt = wave_max(mt);
   nu = wave_sum(nu);
-  __shared__ int32_t s_m[3][NW];
+  nf = wave_sum(nf);
+  __shared__ int32_t s_m[4][NW];
   if (lane == 0) {
     s_m[0][wv] = mr;
     s_m[1][wv] = mt;
     s_m[2][wv] = nu;
+    s_m[3][wv] = nf;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -752,12 +781,14 @@ __global__ void __launch_bounds__(kSizesThreads) k_build_sizes(SizesArgs a) {
       mr = max(mr, s_m[0][w]);
       mt = max(mt, s_m[1][w]);
       nu += s_m[2][w];
+      nf += s_m[3][w];
     }
     a.host[0] = *a.flag;
     a.host[1] = *a.pairs;
     a.host[5] = mr;
     a.host[6] = mt;
     a.host[7] = nu;
+    a.host[8] = nf;
     *a.flag = 0;
     *a.pairs = 0;
   }
@@ -1067,9 +1098,10 @@ hipError_t launch_build_sizes(ggem_ctx* ctx, int64_t* host) {
   a.nbricks = nb;
   a.flag = ctx->flag;
   a.pairs = ctx->pairs_d;
+  a.work = ctx->quad_work;
   a.host = host;
   ProfScope ps(ctx, "build_sizes");
-  hipLaunchKernelGGL(k_build_sizes, dim3(4), dim3(kSizesThreads), 0, ctx->stream, a);
+  hipLaunchKernelGGL(k_build_sizes, dim3(5), dim3(kSizesThreads), 0, ctx->stream, a);
   return hipGetLastError();
 }
 

@@ -17,9 +17,10 @@
 // entry) in list order and k_apply streams them, gathering one operand
 // record per neighbour.  FP32C, one operand: per brick of cells the
 // neighbours' records are staged in LDS and the entries stream a 2-byte
-// record number and the 8-byte (A, Bx) (k_box_fill, k_apply_box, below).
-// FP32C, several operands or the explicit minimum image: k_apply evaluates
-// (A, Bx) per pair from the coefficient table in LDS.  Blocks are
+// record number (k_box_fill, k_apply_box, k_apply_quad, below).  FP32C,
+// several operands: k_apply_quad, four lanes per target.  The explicit
+// minimum image, bricks that are not staged: k_apply evaluates (A, Bx) per
+// pair from the coefficient table in LDS.  Blocks are
 // renumbered per XCD so a chip partition keeps a contiguous stretch of
 // cells and their neighbours in its L2.
 //
@@ -30,6 +31,7 @@
 // (combination, recurrence) runs in FP64.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "ggem_device.h"
@@ -217,155 +219,225 @@ __global__ void __launch_bounds__(BLK) k_tensors(PairArgs a, double4* __restrict
   }
 }
 
-// Epilogue of the pair sum of target slot s, m = acc (see Epi).
-template <int NR, int EPI>
-__device__ __forceinline__ void apply_epilogue(const PairArgs& a, int64_t s, const double (&acc)[NR][3],
-                                               const double* __restrict__ xsoa, const SlotVec& v,
-                                               const ChebEpi& epi, const double* __restrict__ u_glob,
-                                               double* __restrict__ out, double (&dots)[3]) {
+// What the epilogue of a target slot reads once for all its components.
+struct EpiTarget {
+  double da, db, ck, cm1, c0;  // EPI_CHEB
+  int64_t p;                   // EPI_LOCAL, EPI_MOBILITY: particle of the slot
+};
+template <int EPI>
+__device__ __forceinline__ EpiTarget epi_target(const PairArgs& a, int64_t s, const ChebEpi& epi) {
+  EpiTarget T{epi.da, epi.db, epi.c, epi.cm1, epi.c0, 0};
+  if (EPI == EPI_LOCAL || EPI == EPI_MOBILITY) T.p = a.perm[s];
+  if (EPI == EPI_CHEB && epi.dpar) {
+    const double* pp = epi.dpar + int64_t(epi.sys ? epi.sys[s] : 0) * epi.pstride;
+    T.da = pp[0];
+    T.db = pp[1];
+    T.ck = pp[2 + epi.term];
+    if (epi.ymask & 1) T.cm1 = pp[epi.term];
+    if (epi.ymask & 2) T.c0 = pp[1 + epi.term];
+  }
+  return T;
+}
+
+// Epilogue of component q of the pair sum of target slot s for operand r, m
+// the sum (see Epi); the value of the new vector (EPI_CHEB, EPI_REF), whose
+// gather record is left to epi_record.
+template <int EPI>
+__device__ __forceinline__ double epi_component(const PairArgs& a, const EpiTarget& T, int64_t s, int r, int q, double m,
+                                                const double* __restrict__ xsoa, const SlotVec& v, const ChebEpi& epi,
+                                                const double* __restrict__ u_glob, double* __restrict__ out,
+                                                double (&dots)[3]) {
   const int64_t n = a.n;
-  if constexpr (EPI == EPI_REF) {
-    static_assert(NR == 1, "the reference mode takes one vector at a time");
-    const RefEpi& R = epi.ref;
-    double nv[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int64_t idx = int64_t(q) * n + s;
-      const double xv = xsoa[idx];
-      double m = acc[0][q];
-      if (a.k.point_type == GGEM_POLYMER_BEAD) m = m - a.k.coeff_1 * xv + xv;
-      else if (a.k.point_type == GGEM_LAGRANGIAN_POINT) m = m + a.k.coeff_2 * xv;
-      else m = 0.0;
+  if constexpr (EPI == EPI_LOCAL || EPI == EPI_MOBILITY) {
+    // forces are the operand: own force from the FP64 store
+    const double fo = a.fs[q * n + s];
+    double u = m;
+    if (a.k.point_type == GGEM_LAGRANGIAN_POINT) u += a.k.coeff_2 * fo;  // self term
+    if (EPI == EPI_MOBILITY) {
+      const double ug = u_glob ? u_glob[3 * T.p + q] : 0.0;
+      if (a.k.point_type == GGEM_POLYMER_BEAD) u = ug + u - a.k.coeff_1 * fo + fo;
+      else if (a.k.point_type == GGEM_LAGRANGIAN_POINT) u = ug + u;
+      else u = 0.0;
+    }
+    out[3 * T.p + q] = u;
+    return u;
+  } else {
+    const int64_t idx = int64_t(r) * 3 * n + int64_t(q) * n + s;
+    const double xv = xsoa[idx];
+    if (a.k.point_type == GGEM_POLYMER_BEAD) m = m - a.k.coeff_1 * xv + xv;
+    else if (a.k.point_type == GGEM_LAGRANGIAN_POINT) m = m + a.k.coeff_2 * xv;
+    else m = 0.0;
+    double nv;
+    if constexpr (EPI == EPI_REF) {
+      const RefEpi& R = epi.ref;
       double y = R.c * xv, my = R.c * m;
       if (R.term == 0) {
-        nv[q] = epi.db * xv + epi.da * m;
+        nv = T.db * xv + T.da * m;
         dots[0] += m * xv;
       } else {
         y += epi.y[idx];
         my += R.my[idx];
-        nv[q] = 2. * epi.db * xv + 2. * epi.da * m - epi.xm1.soa[idx];
+        nv = 2. * T.db * xv + 2. * T.da * m - epi.xm1.soa[idx];
         dots[0] += my * my;
       }
       dots[1] += y * y;
       dots[2] += xv * xv;
       epi.y[idx] = y;
       R.my[idx] = my;
-      v.soa[idx] = nv[q];
+    } else if (epi.kind == 0) {
+      nv = m;
+    } else if (epi.kind == 1) {
+      nv = T.db * xv + T.da * m;
+    } else {
+      const double xm = epi.xm1.soa[idx];
+      nv = 2. * T.db * xv + 2. * T.da * m;
+      nv += -1.0 * xm;
+      if (epi.ymask == 4) {
+        epi.y[idx] += T.ck * nv;
+      } else if (epi.ymask) {  // x_{k-1}, x_k and x_{k+1} terms in one update of y
+        double add = 0.0;
+        if (epi.ymask & 1) add += T.cm1 * xm;
+        if (epi.ymask & 2) add += T.c0 * xv;
+        if (epi.ymask & 4) add += T.ck * nv;
+        epi.y[idx] += add;
+      }
     }
-    if (v.g32) v.g32[s] = make_float4(float(nv[0]), float(nv[1]), float(nv[2]), 0.f);
-    if (v.g64) v.g64[s] = make_double4(nv[0], nv[1], nv[2], 0.0);
-    return;
+    v.soa[idx] = nv;
+    return nv;
   }
-  if (EPI == EPI_LOCAL || EPI == EPI_MOBILITY) {
-    // forces are the operand: own force from the FP64 store
-    const double fo[3] = {a.fs[s], a.fs[n + s], a.fs[2 * n + s]};
-    double u[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      u[q] = acc[0][q];
-      if (a.k.point_type == GGEM_LAGRANGIAN_POINT) u[q] += a.k.coeff_2 * fo[q];  // self term
-    }
-    const int64_t p = a.perm[s];
-    if (EPI == EPI_MOBILITY) {
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const double ug = u_glob ? u_glob[3 * p + q] : 0.0;
-        if (a.k.point_type == GGEM_POLYMER_BEAD) u[q] = ug + u[q] - a.k.coeff_1 * fo[q] + fo[q];
-        else if (a.k.point_type == GGEM_LAGRANGIAN_POINT) u[q] = ug + u[q];
-        else u[q] = 0.0;
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) out[3 * p + q] = u[q];
-  } else {
-    double da = epi.da, db = epi.db, ck = epi.c, cm1 = epi.cm1, c0 = epi.c0;
-    if (epi.dpar) {
-      const double* pp = epi.dpar + int64_t(epi.sys ? epi.sys[s] : 0) * epi.pstride;
-      da = pp[0];
-      db = pp[1];
-      ck = pp[2 + epi.term];
-      if (epi.ymask & 1) cm1 = pp[epi.term];
-      if (epi.ymask & 2) c0 = pp[1 + epi.term];
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      double nv[3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const int64_t idx = int64_t(r) * 3 * n + int64_t(q) * n + s;
-        const double xv = xsoa[idx];
-        double m = acc[r][q];
-        if (a.k.point_type == GGEM_POLYMER_BEAD) m = m - a.k.coeff_1 * xv + xv;
-        else if (a.k.point_type == GGEM_LAGRANGIAN_POINT) m = m + a.k.coeff_2 * xv;
-        else m = 0.0;
-        if (epi.kind == 0) {
-          nv[q] = m;
-        } else if (epi.kind == 1) {
-          nv[q] = db * xv + da * m;
-        } else {
-          const double xm = epi.xm1.soa[idx];
-          double tv = 2. * db * xv + 2. * da * m;
-          tv += -1.0 * xm;
-          nv[q] = tv;
-          if (epi.ymask == 4) {
-            epi.y[idx] += ck * tv;
-          } else if (epi.ymask) {  // x_{k-1}, x_k and x_{k+1} terms in one update of y
-            double add = 0.0;
-            if (epi.ymask & 1) add += cm1 * xm;
-            if (epi.ymask & 2) add += c0 * xv;
-            if (epi.ymask & 4) add += ck * tv;
-            epi.y[idx] += add;
-          }
-        }
-        v.soa[idx] = nv[q];
-      }
-      if (v.g32) v.g32[r * n + s] = make_float4(float(nv[0]), float(nv[1]), float(nv[2]), 0.f);
-      if (v.g64) v.g64[r * n + s] = make_double4(nv[0], nv[1], nv[2], 0.0);
-    }
+}
+// gather record of the new vector, operand r of NR
+template <int NR, int EPI>
+__device__ __forceinline__ void epi_record(int64_t s, int r, double x, double y, double z,
+                                           const SlotVec& v) {
+  if constexpr (EPI == EPI_CHEB || EPI == EPI_REF) {
+    if (v.g32) v.g32[s * NR + r] = make_float4(float(x), float(y), float(z), 0.f);
+    if (v.g64) v.g64[s * NR + r] = make_double4(x, y, z, 0.0);
   }
 }
 
-__device__ __forceinline__ double block_add(double v, double* sh) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+// Epilogue of the pair sums of target slot s, one thread
+template <int NR, int EPI>
+__device__ __forceinline__ void apply_epilogue(const PairArgs& a, int64_t s, const double (&acc)[NR][3],
+                                               const double* __restrict__ xsoa, const SlotVec& v,
+                                               const ChebEpi& epi, const double* __restrict__ u_glob,
+                                               double* __restrict__ out, double (&dots)[3]) {
+  const EpiTarget T = epi_target<EPI>(a, s, epi);
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    double nv[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      nv[q] = epi_component<EPI>(a, T, s, r, q, acc[r][q], xsoa, v, epi, u_glob, out, dots);
+    epi_record<NR, EPI>(s, r, nv[0], nv[1], nv[2], v);
+  }
+}
+
+// value of v in lane M of the lane's quad (four consecutive lanes)
+template <int M>
+__device__ __forceinline__ int quad_get(int v) {
+  return __builtin_amdgcn_mov_dpp(v, M * 0x55, 0xf, 0xf, true);
+}
+template <int M>
+__device__ __forceinline__ float quad_get(float v) {
+  return __int_as_float(quad_get<M>(__float_as_int(v)));
+}
+template <int M>
+__device__ __forceinline__ double quad_get(double v) {
+  return __hiloint2double(quad_get<M>(__double2hiint(v)), quad_get<M>(__double2loint(v)));
+}
+// p + v of lane 0 + .. + v of lane 3 of the quad, in that order
+template <class T>
+__device__ __forceinline__ T quad_add(T p, T v) {
+  p += quad_get<0>(v);
+  p += quad_get<1>(v);
+  p += quad_get<2>(v);
+  p += quad_get<3>(v);
+  return p;
+}
+
+// Epilogue of the pair sum of target slot s of a quad whose lanes all hold
+// it: lane c < 3 takes component c
+template <int EPI>
+__device__ __forceinline__ void quad_epilogue(const PairArgs& a, int64_t s, int c, double m0, double m1, double m2,
+                                              const double* __restrict__ xsoa, const SlotVec& v, const ChebEpi& epi,
+                                              const double* __restrict__ u_glob, double* __restrict__ out,
+                                              double (&dots)[3]) {
+  double nv = 0.0;
+  if (c < 3) {
+    const EpiTarget T = epi_target<EPI>(a, s, epi);
+    nv = epi_component<EPI>(a, T, s, 0, c, c == 0 ? m0 : (c == 1 ? m1 : m2), xsoa, v, epi, u_glob, out, dots);
+  }
+  const double x = quad_get<0>(nv), y = quad_get<1>(nv), z = quad_get<2>(nv);
+  if (c == 0) epi_record<1, EPI>(s, 0, x, y, z, v);
+}
+
+// the block's sums of three values, on every thread (one barrier pair)
+__device__ __forceinline__ void block_add3(double (&t)[3]) {
+  __shared__ double sh[3][16];
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+    for (int o = 32; o > 0; o >>= 1) t[q] += __shfl_down(t[q], o, 64);
+  const int nw = int(blockDim.x >> 6);
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) sh[q][threadIdx.x >> 6] = t[q];
   __syncthreads();
-  double t = 0.0;
-  for (int w = 0; w < int(blockDim.x >> 6); ++w) t += sh[w];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    t[q] = 0.0;
+    for (int w = 0; w < nw; ++w) t[q] += sh[q][w];
+  }
   __syncthreads();
-  return t;
 }
 
 // End of a reference-mode launch, the whole block with its parts of the
 // three dot products: they go to memory past the XCD's L2 (agent scope), and
-// the block that draws the last ticket adds all blocks' parts (in block
-// order, whichever block that is) and applies the stopping rule.  One launch
-// per term instead of six: per-term dot products, gather records and the
-// deciding kernel were 16 us of the 66 us a term took for 25,600 chain beads.
+// the last block to finish adds all blocks' parts (in block order, whichever
+// block that is) and applies the stopping rule.  Tickets are drawn in
+// kRefGroups groups, a group's last block drawing one of the top: a single
+// ticket's atomics follow one another at 11 ns each (700 blocks: 8 us).
+// One launch per term instead of six: per-term dot products, gather records
+// and the deciding kernel were 16 us of the 66 us a term took for 25,600
+// chain beads.
 __device__ __forceinline__ void ref_finish(const ChebEpi& epi, const double (&dots)[3]) {
-  __shared__ double sh[16];
   __shared__ int s_last;
   const RefEpi& R = epi.ref;
-  const int nb = int(gridDim.x);
-  double t[3];
-#pragma unroll
-  for (int q = 0; q < 3; ++q) t[q] = block_add(dots[q], sh);
+  const int nb = int(gridDim.x), id = int(blockIdx.x);
+  double t[3] = {dots[0], dots[1], dots[2]};
+  block_add3(t);
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int q = 0; q < 3; ++q)
-      __hip_atomic_store(R.part + int64_t(q) * nb + blockIdx.x, t[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = __hip_atomic_fetch_add(R.ticket, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+      __hip_atomic_store(R.part + int64_t(q) * nb + id, t[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int g = id % kRefGroups, groups = min(nb, kRefGroups), in_group = (nb - g + kRefGroups - 1) / kRefGroups;
+    bool last = __hip_atomic_fetch_add(R.ticket + 1 + g, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == in_group - 1;
+    if (last) last = __hip_atomic_fetch_add(R.ticket, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
+    s_last = last;
   }
   __syncthreads();
   if (!s_last) return;  // uniform over the block
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    double sum = 0.0;
-    for (int b = int(threadIdx.x); b < nb; b += int(blockDim.x))
-      sum += __hip_atomic_load(R.part + int64_t(q) * nb + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    t[q] = block_add(sum, sh);
+  for (int q = 0; q < 3; ++q) t[q] = 0.0;
+  constexpr int U = 4;  // parts in flight per thread and product
+  for (int b = int(threadIdx.x); b < nb; b += U * int(blockDim.x)) {
+    double w[U][3];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int bu = min(b + u * int(blockDim.x), nb - 1);
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        w[u][q] = __hip_atomic_load(R.part + int64_t(q) * nb + bu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (b + u * int(blockDim.x) < nb)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) t[q] += w[u][q];
   }
+  block_add3(t);
+  if (threadIdx.x <= kRefGroups) R.ticket[threadIdx.x] = 0;  // (blocks have 64 threads or more)
   if (threadIdx.x != 0) return;
-  *R.ticket = 0;
   if (R.term == 0) {
     R.st[0] = t[0];
   } else {
@@ -411,7 +483,6 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
   }
   double dots[3] = {0.0, 0.0, 0.0};
   auto body = [&]() {
-  const int64_t n = a.n;
   const int cnt = a.cnt[s];
   const int64_t base = a.slice_off[s >> 6] + (s & 63);
   const uint32_t* lst = a.ell + base;
@@ -452,7 +523,7 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
 #pragma unroll
       for (int i = 0; i < U; ++i)
 #pragma unroll
-        for (int r = 0; r < NR; ++r) f[i][r] = xg[r * n + (e[i] & kSlotMask)];
+        for (int r = 0; r < NR; ++r) f[i][r] = xg[int64_t(e[i] & kSlotMask) * NR + r];
 #pragma unroll
       for (int i = 0; i < U; ++i) pair_acc(c[i], f[i]);
     }
@@ -461,7 +532,7 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
       if (k + i < cnt) {  // entries en[0 .. cnt - k)
         double4 f[NR];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) f[r] = xg[r * n + (en[i] & kSlotMask)];
+        for (int r = 0; r < NR; ++r) f[r] = xg[int64_t(en[i] & kSlotMask) * NR + r];
         pair_acc(cf[int64_t(k + i) * kSlice], f);
       }
     }
@@ -558,7 +629,7 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
         const uint32_t t = c[i] & kSlotMask;
         pt[i] = pc[t];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) f[i][r] = xg[r * n + t];
+        for (int r = 0; r < NR; ++r) f[i][r] = xg[int64_t(t) * NR + r];
       }
 #pragma unroll
       for (int i = 0; i < U; ++i) pair_acc(c[i], pt[i], f[i]);
@@ -569,7 +640,7 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
         const uint32_t t = en[i] & kSlotMask;
         float4 f[NR];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) f[r] = xg[r * n + t];
+        for (int r = 0; r < NR; ++r) f[r] = xg[int64_t(t) * NR + r];
         pair_acc(en[i], pc[t], f);
       }
     }
@@ -649,6 +720,7 @@ struct BoxView {
   const uint32_t* slot;
   const float4* pos;
   const uint16_t* idx;
+  const uint32_t* work;  // k_apply_quad: brick * kQuadShares + share of every block
 };
 
 // Entry layout of a brick: its targets in the order tgt, in waves of 64;
@@ -1041,136 +1113,273 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box(PairArgs a, BoxView b
 }
 
 
-// k_apply_box for NR > 1 operands (the fixed-order step of several noise
-// vectors): the box's positions and the NR operands' records staged in LDS
-// ([NR][records] after the positions), each kept pair's table evaluated
-// once for all NR; per operand the sums, their merge points and the
-// epilogue are k_apply's for NR operands.  Every brick with targets is
-// staged (the host launches it only then).
+// The staged pair sum with four lanes (a quad) per target, for NR operands.
+// One operand: lane c takes entries c, c + 4, ...; the four terms of a step
+// are added in list order by every lane (quad_add).  Several operands: lane c
+// forms the displacement and the tensor of its entry, then the quad goes
+// through the four entries together and lane c sums operands c, c + 4, ...
+// (NR = 2: c mod 2).  Sums, merge points and epilogue are k_apply's for NR
+// operands, bit for bit.  A block takes one item of the work list, a brick's share
+// of about kQuadShare targets.
+// A lane per target leaves most of a block idle in bricks with few targets
+// (20,000 beads: 39 of 256 lanes) and walks each list alone: one operand 9.1
+// -> 6.6 us per application there, 30 -> 21 us for chains in a slit (25,600
+// beads).  Several operands used to gather from global memory, a lane per
+// target: eight of 20,000 beads 34.8 -> 12.9 us, four of 272,000 beads in 64
+// suspensions 176 -> 131 us (bound by staging 16 records per target).
 template <int EPI, bool ONE, int NR>
-__global__ void __launch_bounds__(kBoxThreads) k_apply_box_nr(PairArgs a, BoxView b, const float4* __restrict__ xg,
-                                                             const double* __restrict__ xsoa, SlotVec v, ChebEpi epi,
-                                                             const double* __restrict__ u_glob,
-                                                             double* __restrict__ out) {
-  static_assert(NR > 1, "one operand: k_apply_box");
+__global__ void __launch_bounds__(kBoxThreads) k_apply_quad(PairArgs a, BoxView b, const float4* __restrict__ xg,
+                                                           const double* __restrict__ xsoa, SlotVec v, ChebEpi epi,
+                                                           const double* __restrict__ u_glob,
+                                                           double* __restrict__ out) {
   extern __shared__ float4 lds[];
   if (epi.skip && *epi.skip) return;  // uniform over the grid
-  const int64_t brick = block_index(a.xcd);
+  const uint32_t item = b.work[block_index(a.xcd)];
+  const int64_t brick = item / kQuadShares;
   const int64_t c0 = brick * kBrickCells;
   const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
-  if (sb >= se) return;  // no targets (uniform over the block)
+  const int nt = se - sb, shares = quad_shares(nt), y = int(item % kQuadShares);
+  const int t0 = nt * y / shares, t1 = nt * (y + 1) / shares;
+  double dots[3] = {0.0, 0.0, 0.0};
   const int64_t r0 = b.off[brick];
   const int nrec = int(b.off[brick + 1] - r0);
-  const int nt = se - sb;
-  if (nrec == 0) return;  // not staged: never launched so (uniform over the block)
-  const int64_t n = a.n;
+  const int c = int(threadIdx.x) & 3;
+  int i = t0 + (int(threadIdx.x) >> 2);
+  // the first target's words are on their way while the records are staged
+  int32_t s = 0;
+  int64_t bpk = 0;
+  if (i < t1) {
+    s = b.tgt[sb + i];
+    bpk = b.base[sb + i];
+  }
   float4* s_tab = lds;                       // coefficient table
   float4* rpos = lds + kTabStride * a.ct.n;  // [nrec] offset xyz, packed box cell
-  float4* rval = rpos + nrec;                // [NR][nrec] operands
+  float4* rval = rpos + nrec;                // [nrec][NR] operands
   load_tab(s_tab, a);
-  for (int i = int(threadIdx.x); i < nrec; i += kBoxThreads) {
-    const uint32_t t = b.slot[r0 + i];
-    rpos[i] = b.pos[r0 + i];
+  if (nrec == 0) {  // not staged (one operand only)
+    __syncthreads();
+    if constexpr (NR == 1)
+      for (int j = t0 + int(threadIdx.x); j < t1; j += kBoxThreads) {
+        const int64_t sj = b.tgt[sb + j];
+        double acc[1][3];
+        fp32c_pairs_global(a, sj, s_tab, xg, acc);
+        apply_epilogue<1, EPI>(a, sj, acc, xsoa, v, epi, u_glob, out, dots);
+      }
+    if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
+    return;
+  }
+  for (int j = int(threadIdx.x); j < nrec; j += kBoxThreads) {
+    const uint32_t t = b.slot[r0 + j];
+    rpos[j] = b.pos[r0 + j];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) rval[r * nrec + i] = xg[r * n + t];
+    for (int r = 0; r < NR; ++r) rval[j * NR + r] = xg[int64_t(t) * NR + r];
   }
   __syncthreads();
   BoxGeom B;
   box_init(B, a, b.reach, brick, sb);
   const float hx = B.h[0], hy = B.h[1], hz = B.h[2];
-  constexpr int U = 2;  // entries per group, the next group's record numbers loaded one ahead
-  for (int i = int(threadIdx.x); i < nt; i += kBoxThreads) {
-    const int64_t s = b.tgt[sb + i];
-    const int64_t bpk = b.base[sb + i];
-    const int64_t base = bpk & kBaseMask;
+  constexpr int PER = NR <= 4 ? 1 : NR / 4;  // operands per lane
+  const int op = NR == 1 ? 0 : (NR == 2 ? (c & 1) : c);
+  while (i < t1) {
+    const uint16_t* __restrict__ ci = b.idx + (bpk & kBaseMask);
     const float4 po = rpos[int((uint64_t(bpk) >> kSelfShift) & kField12)];  // the target's own record
     const uint32_t kb = 0x808080u - __float_as_uint(po.w);
-    const int cnt = int((uint64_t(bpk) >> kKeptShift) & kField12);  // stored (kept) entries
-    float ps[NR][3];
-    KahanF kh[NR][3];
+    const int cnt = int((uint64_t(bpk) >> kKeptShift) & kField12), last = cnt - 1;  // stored (kept) entries
+    float ps[PER][3];
+    KahanF kh[PER][3];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) ps[r][0] = ps[r][1] = ps[r][2] = 0.f;
-    auto disp = [&](const float4& pt, float& dx, float& dy, float& dz, float& y) {
-      float di, dj, dk;
+    for (int r = 0; r < PER; ++r) ps[r][0] = ps[r][1] = ps[r][2] = 0.f;
+    auto merge = [&]() {
+#pragma unroll
+      for (int r = 0; r < PER; ++r)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          kh[r][q].add(ps[r][q]);
+          ps[r][q] = 0.f;
+        }
+    };
+    struct Geo {
+      float dx, dy, dz, A, Bx;
+    };
+    auto geometry = [&](const float4& pt) {
+      Geo g;
+      float di, dj, dk, y;
       box_diff(__float_as_uint(pt.w), kb, di, dj, dk);
-      dx = __builtin_fmaf(di, hx, pt.x - po.x);
-      dy = __builtin_fmaf(dj, hy, pt.y - po.y);
-      dz = __builtin_fmaf(dk, hz, pt.z - po.z);
-      return ONE ? fp32c_interval1(a.ct, fp32c_r2(dx, dy, dz), y) : fp32c_interval(a.ct, fp32c_r2(dx, dy, dz), y);
+      g.dx = __builtin_fmaf(di, hx, pt.x - po.x);
+      g.dy = __builtin_fmaf(dj, hy, pt.y - po.y);
+      g.dz = __builtin_fmaf(dk, hz, pt.z - po.z);
+      const float r2 = fp32c_r2(g.dx, g.dy, g.dz);
+      const int it = ONE ? fp32c_interval1(a.ct, r2, y) : fp32c_interval(a.ct, r2, y);
+      fp32c_eval(s_tab, it, y, g.A, g.Bx);
+      return g;
     };
-    auto merge = [&](int k) {
-      if ((k & (kMergeEvery - 1)) == kMergeEvery - 1) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-#pragma unroll
-          for (int q = 0; q < 3; ++q) {
-            kh[r][q].add(ps[r][q]);
-            ps[r][q] = 0.f;
-          }
+    static_assert(kMergeEvery == 8, "a merge every two steps of the quad");
+    if constexpr (NR == 1) {
+      auto term = [&](const Geo& g, const float4& f, bool in, float& x, float& y, float& z) {
+        x = y = z = 0.f;
+        fp32c_acc(g.A, g.Bx, g.dx, g.dy, g.dz, f.x, f.y, f.z, x, y, z);
+        if (!in) x = y = z = 0.f;
+      };
+      // two steps (eight entries) at a time, their record numbers loaded one ahead
+      uint32_t e0 = 0, e1 = 0;
+      if (cnt > 0) {
+        e0 = ci[int64_t(min(c, last)) * kSlice];
+        e1 = ci[int64_t(min(c + 4, last)) * kSlice];
       }
-    };
-    auto one = [&](uint32_t rec, int k) {
-      const float4 pt = rpos[rec];
-      float dx, dy, dz, y, A, Bx;
-      const int it = disp(pt, dx, dy, dz, y);
-      fp32c_eval(s_tab, it, y, A, Bx);
-#pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        const float4 f = rval[r * nrec + rec];
-        fp32c_acc(A, Bx, dx, dy, dz, f.x, f.y, f.z, ps[r][0], ps[r][1], ps[r][2]);
-      }
-      merge(k);
-    };
-    if (cnt > 0) {
-      const uint16_t* __restrict__ ci = b.idx + base;
-      const int last = cnt - 1;
-      uint32_t en[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) en[u] = ci[int64_t(min(u, last)) * kSlice];
       int k = 0;
-      for (; k + U <= cnt; k += U) {
-        uint32_t c[U];
+      auto steps = [&](bool in0, bool in1) {
+        const float4 p0 = rpos[e0], p1 = rpos[e1], f0 = rval[e0], f1 = rval[e1];
+        e0 = ci[int64_t(min(k + 8 + c, last)) * kSlice];
+        e1 = ci[int64_t(min(k + 12 + c, last)) * kSlice];
+        const Geo g0 = geometry(p0), g1 = geometry(p1);
+        float x0, y0_, z0, x1, y1_, z1;
+        term(g0, f0, in0, x0, y0_, z0);
+        term(g1, f1, in1, x1, y1_, z1);
+        ps[0][0] = quad_add(quad_add(ps[0][0], x0), x1);
+        ps[0][1] = quad_add(quad_add(ps[0][1], y0_), y1_);
+        ps[0][2] = quad_add(quad_add(ps[0][2], z0), z1);
+        merge();
+      };
+      for (; k + 8 <= cnt; k += 8) steps(true, true);
+      if (k < cnt) steps(k + c < cnt, k + 4 + c < cnt);
+    } else {
+      uint32_t en = cnt > 0 ? ci[int64_t(min(c, last)) * kSlice] : 0u;
+      for (int k = 0; k < cnt; k += 4) {
+        const int e = int(en);
+        en = ci[int64_t(min(k + 4 + c, last)) * kSlice];
+        const Geo g = geometry(rpos[e]);
+        auto entry = [&](auto M) {
+          constexpr int m = decltype(M)::value;
+          if (k + m < cnt) {  // uniform over the quad
+            const int em = quad_get<m>(e);
+            const Geo gm{quad_get<m>(g.dx), quad_get<m>(g.dy), quad_get<m>(g.dz), quad_get<m>(g.A),
+                         quad_get<m>(g.Bx)};
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          c[u] = en[u];
-          en[u] = ci[int64_t(min(k + U + u, last)) * kSlice];
-        }
-        float4 pt[U], f[U][NR];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          pt[u] = rpos[c[u]];
-#pragma unroll
-          for (int r = 0; r < NR; ++r) f[u][r] = rval[r * nrec + c[u]];
-        }
-        float dx[U], dy[U], dz[U], y[U];
-        int it[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) it[u] = disp(pt[u], dx[u], dy[u], dz[u], y[u]);
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          float A, Bx;
-          fp32c_eval(s_tab, it[u], y[u], A, Bx);
-#pragma unroll
-          for (int r = 0; r < NR; ++r)
-            fp32c_acc(A, Bx, dx[u], dy[u], dz[u], f[u][r].x, f[u][r].y, f[u][r].z, ps[r][0], ps[r][1], ps[r][2]);
-          merge(k + u);
-        }
+            for (int r = 0; r < PER; ++r) {
+              const float4 f = rval[em * NR + op + 4 * r];
+              fp32c_acc(gm.A, gm.Bx, gm.dx, gm.dy, gm.dz, f.x, f.y, f.z, ps[r][0], ps[r][1], ps[r][2]);
+            }
+          }
+        };
+        entry(std::integral_constant<int, 0>{});
+        entry(std::integral_constant<int, 1>{});
+        entry(std::integral_constant<int, 2>{});
+        entry(std::integral_constant<int, 3>{});
+        if ((k & 4) && k + 4 <= cnt) merge();
       }
-#pragma unroll
-      for (int u = 0; u < U - 1; ++u)
-        if (k + u < cnt) one(en[u], k + u);
     }
-    double acc[NR][3];
+    double acc[PER][3];
 #pragma unroll
-    for (int r = 0; r < NR; ++r)
+    for (int r = 0; r < PER; ++r)
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         kh[r][q].add(ps[r][q]);
         acc[r][q] = kh[r][q].value();
       }
-    double dots[3];
-    apply_epilogue<NR, EPI>(a, s, acc, xsoa, v, epi, u_glob, out, dots);
+    if constexpr (NR == 1) {
+      quad_epilogue<EPI>(a, s, c, acc[0][0], acc[0][1], acc[0][2], xsoa, v, epi, u_glob, out, dots);
+    } else if (c < NR) {
+      const EpiTarget T = epi_target<EPI>(a, s, epi);
+#pragma unroll
+      for (int r = 0; r < PER; ++r) {
+        double nv[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          nv[q] = epi_component<EPI>(a, T, s, op + 4 * r, q, acc[r][q], xsoa, v, epi, u_glob, out, dots);
+        epi_record<NR, EPI>(s, op + 4 * r, nv[0], nv[1], nv[2], v);
+      }
+    }
+    i += kBoxThreads / 4;
+    if (i < t1) {
+      s = b.tgt[sb + i];
+      bpk = b.base[sb + i];
+    }
   }
+  if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
+}
+
+// k_apply_box64 (below) with four lanes per target: lane c takes entries c,
+// c + 4, ...; the four terms of a step are added in list order by every lane.
+template <int EPI>
+__global__ void __launch_bounds__(kBoxThreads) k_apply_quad64(PairArgs a, BoxView b, const double4* __restrict__ c64,
+                                                             const double4* __restrict__ xg,
+                                                             const double* __restrict__ xsoa, SlotVec v, ChebEpi epi,
+                                                             const double* __restrict__ u_glob,
+                                                             double* __restrict__ out) {
+  extern __shared__ double4 lds64[];
+  if (epi.skip && *epi.skip) return;  // uniform over the grid
+  const uint32_t item = b.work[block_index(a.xcd)];
+  const int64_t brick = item / kQuadShares;
+  const int64_t c0 = brick * kBrickCells;
+  const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
+  const int nt = se - sb, shares = quad_shares(nt), y = int(item % kQuadShares);
+  const int t0 = nt * y / shares, t1 = nt * (y + 1) / shares;
+  double dots[3] = {0.0, 0.0, 0.0};
+  const int64_t r0 = b.off[brick];
+  const int nrec = int(b.off[brick + 1] - r0);
+  double4* rval = lds64;  // [nrec] operand
+  const double sg = a.bsign;
+  const int c = int(threadIdx.x) & 3;
+  // the first target's words are on their way while the records are staged
+  int i = t0 + (int(threadIdx.x) >> 2);
+  int cnt = 0;
+  int64_t base = 0;
+  auto words = [&]() {
+    const int64_t s = sb + i;
+    cnt = a.cnt[s];
+    base = a.slice_off[s >> 6] + (s & 63);
+  };
+  if (i < t1) words();
+  for (int j = int(threadIdx.x); j < nrec; j += kBoxThreads) rval[j] = xg[b.slot[r0 + j]];
+  __syncthreads();
+  constexpr int U = 2;  // steps per group, the next group's tensors and record numbers loaded one ahead
+  while (i < t1) {
+    const int64_t s = sb + i;
+    const int last = cnt - 1;
+    double ps[3] = {0.0, 0.0, 0.0};
+    const double4* __restrict__ cf = c64 + base;
+    auto sum = [&](const double4& t, const double4& f, bool in) {
+      double x = 0.0, y = 0.0, z = 0.0;
+      fp64_acc(t, sg, f, x, y, z);
+      if (!in) x = y = z = 0.0;
+      ps[0] = quad_add(ps[0], x);
+      ps[1] = quad_add(ps[1], y);
+      ps[2] = quad_add(ps[2], z);
+    };
+    if (nrec > 0 && cnt > 0) {
+      const uint16_t* __restrict__ ci = b.idx + base;
+      double4 tn[U];
+      uint32_t en[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t e = int64_t(min(4 * u + c, last)) * kSlice;
+        en[u] = ci[e];
+        tn[u] = cf[e];
+      }
+      for (int k = 0; k < cnt; k += 4 * U) {
+        double4 t[U], f[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          t[u] = tn[u];
+          f[u] = rval[en[u]];
+          const int64_t e = int64_t(min(k + 4 * (U + u) + c, last)) * kSlice;
+          en[u] = ci[e];
+          tn[u] = cf[e];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) sum(t[u], f[u], k + 4 * u + c < cnt);
+      }
+    } else {
+      for (int k = 0; k < cnt; k += 4) {
+        const int64_t e = int64_t(min(k + c, last)) * kSlice;
+        sum(cf[e], xg[a.ell[base + e] & kSlotMask], k + c < cnt);
+      }
+    }
+    quad_epilogue<EPI>(a, s, c, ps[0], ps[1], ps[2], xsoa, v, epi, u_glob, out, dots);
+    i += kBoxThreads / 4;
+    if (i < t1) words();
+  }
+  if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
 }
 
 // FP64 pair sum with the operand records staged in LDS: one workgroup per
@@ -1382,10 +1591,42 @@ BoxView box_view(const ggem_ctx* ctx) {
   b.slot = ctx->box_slot;
   b.pos = ctx->box_pos;
   b.idx = ctx->box_idx;
+  b.work = ctx->quad_work;
   return b;
 }
 
 unsigned n_bricks(const ggem_ctx* ctx) { return unsigned(ctx->grid.n_cells >> (3 * kBrickBits)); }
+
+// Four lanes per target (k_apply_quad, k_apply_quad64) or one (k_apply_box,
+// k_apply_box64), by the mean number of targets of the bricks that have
+// any.  One operand, one lane -> four, us per application:
+//   targets a brick     13 (h = 2)  20         33 (h = 2)  59          117         176         244
+//   FP32C               13.2->10.0  9.3->7.7   15.1->9.5   10.7->9.0   13.6->11.8  16.1->16.5  26.2->25.4
+//   FP64                10.9->10.3  8.3->7.3   10.6->9.8   9.6->9.8    16.6->17.0  24.3->26.3  43.9->45.7
+// and 87 -> 122 us at 1M beads (244, FP32C): there the lanes are busy either
+// way and the sums on every lane of a quad only cost.  FP64 streams its
+// tensors and gains by the split only where the blocks leave CUs idle.
+bool quad_lanes(const ggem_ctx* ctx, int precision) {
+  if (precision == GGEM_FP32C) return ctx->n <= 150 * int64_t(ctx->full_bricks);
+  return ctx->n <= 40 * int64_t(ctx->full_bricks) || ctx->quad_items <= 256;
+}
+
+size_t box_lds(const ggem_ctx* ctx, int nr) {
+  return sizeof(float4) * (kTabStride * size_t(ctx->tab.n) + size_t(ctx->box_max) * size_t(1 + nr));
+}
+
+template <int EPI, int NR>
+hipError_t launch_quad(ggem_ctx* ctx, PairArgs a, const float4* xg, const double* soa, const SlotVec& v,
+                       const ChebEpi& epi, const double* u_glob, double* out) {
+  const dim3 grid(unsigned(ctx->quad_items));
+  if (ctx->tab.n2 == 0)
+    hipLaunchKernelGGL((k_apply_quad<EPI, true, NR>), grid, dim3(kBoxThreads), box_lds(ctx, NR), ctx->stream, a,
+                       box_view(ctx), xg, soa, v, epi, u_glob, out);
+  else
+    hipLaunchKernelGGL((k_apply_quad<EPI, false, NR>), grid, dim3(kBoxThreads), box_lds(ctx, NR), ctx->stream, a,
+                       box_view(ctx), xg, soa, v, epi, u_glob, out);
+  return hipGetLastError();
+}
 
 template <int EPI>
 hipError_t launch_box(ggem_ctx* ctx, PairArgs a, const float4* xg, const double* soa, const SlotVec& v,
@@ -1393,7 +1634,8 @@ hipError_t launch_box(ggem_ctx* ctx, PairArgs a, const float4* xg, const double*
   if (!ctx->box_valid || ctx->box_fp64 || ctx->box_max <= 0 || ctx->box_max > kBoxMaxRecs)
     return hipErrorInvalidConfiguration;
   a.xcd = 1;
-  const size_t lds = sizeof(float4) * (kTabStride * size_t(ctx->tab.n) + size_t(ctx->box_max) * 2);
+  if (quad_lanes(ctx, GGEM_FP32C)) return launch_quad<EPI, 1>(ctx, a, xg, soa, v, epi, u_glob, out);
+  const size_t lds = box_lds(ctx, 1);
   if (ctx->tab.n2 == 0)
     hipLaunchKernelGGL((k_apply_box<EPI, true>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream, a,
                        box_view(ctx), xg, soa, v, epi, u_glob, out);
@@ -1406,12 +1648,9 @@ hipError_t launch_box(ggem_ctx* ctx, PairArgs a, const float4* xg, const double*
 // staged FP32C pair sum of NR > 1 operands: every brick with targets staged
 // and the box's positions and NR operand tables within the block's LDS
 constexpr size_t kBoxNrLds = 81920;  // two blocks per CU
-size_t box_nr_lds(const ggem_ctx* ctx, int nr) {
-  return sizeof(float4) * (kTabStride * size_t(ctx->tab.n) + size_t(ctx->box_max) * size_t(1 + nr));
-}
 bool box_nr_ready(const ggem_ctx* ctx, int nr) {
-  return nr > 1 && nr <= 4 && ctx->box_valid && !ctx->box_fp64 && !ctx->box_unstaged && ctx->box_max > 0 &&
-         ctx->box_max <= kBoxMaxRecs && box_nr_lds(ctx, nr) <= kBoxNrLds;
+  return (nr == 2 || nr == 4 || nr == 8) && ctx->box_valid && !ctx->box_fp64 && !ctx->box_unstaged &&
+         ctx->box_max > 0 && ctx->box_max <= kBoxMaxRecs && box_lds(ctx, nr) <= kBoxNrLds;
 }
 
 template <int EPI, int NR>
@@ -1419,14 +1658,7 @@ hipError_t launch_box_nr(ggem_ctx* ctx, PairArgs a, const float4* xg, const doub
                          const ChebEpi& epi, const double* u_glob, double* out) {
   if (!box_nr_ready(ctx, NR)) return hipErrorInvalidConfiguration;
   a.xcd = 1;
-  const size_t lds = box_nr_lds(ctx, NR);
-  if (ctx->tab.n2 == 0)
-    hipLaunchKernelGGL((k_apply_box_nr<EPI, true, NR>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream, a,
-                       box_view(ctx), xg, soa, v, epi, u_glob, out);
-  else
-    hipLaunchKernelGGL((k_apply_box_nr<EPI, false, NR>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream,
-                       a, box_view(ctx), xg, soa, v, epi, u_glob, out);
-  return hipGetLastError();
+  return launch_quad<EPI, NR>(ctx, a, xg, soa, v, epi, u_glob, out);
 }
 
 template <int EPI>
@@ -1436,8 +1668,12 @@ hipError_t launch_box64(ggem_ctx* ctx, PairArgs a, const double4* xg, const doub
     return hipErrorInvalidConfiguration;
   a.xcd = 1;
   const size_t lds = size_t(ctx->box_max) * sizeof(double4);
-  hipLaunchKernelGGL((k_apply_box64<EPI>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream, a,
-                     box_view(ctx), ctx->coef64, xg, soa, v, epi, u_glob, out);
+  if (quad_lanes(ctx, GGEM_FP64))
+    hipLaunchKernelGGL((k_apply_quad64<EPI>), dim3(unsigned(ctx->quad_items)), dim3(kBoxThreads), lds, ctx->stream, a,
+                       box_view(ctx), ctx->coef64, xg, soa, v, epi, u_glob, out);
+  else
+    hipLaunchKernelGGL((k_apply_box64<EPI>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream, a,
+                       box_view(ctx), ctx->coef64, xg, soa, v, epi, u_glob, out);
   return hipGetLastError();
 }
 
@@ -1449,11 +1685,9 @@ bool box_ready(const ggem_ctx* ctx, int precision, int nr) {
   if (!ctx->box_valid || ctx->box_max <= 0) return false;
   return precision == GGEM_FP32C ? !ctx->box_fp64 : (ctx->box_fp64 && ctx->coef64_valid);
 }
-// the staged kernel by default for one operand; for two or four it is an
-// autotuner candidate only (256 systems x 16 operands in chunks of 4:
-// 3.53 ms per apply against 2.25 ms for the list-order kernel in chunks of 8)
+// the staged kernel by default wherever it applies
 int apply_default(const ggem_ctx* ctx, int precision, int nr) {
-  return nr == 1 && box_ready(ctx, precision, nr) ? kBoxShape : 0;
+  return box_ready(ctx, precision, nr) ? kBoxShape : 0;
 }
 int apply_candidates(const ggem_ctx* ctx, int precision, int nr) {
   return box_ready(ctx, precision, nr) ? kNApply + 1 : kNApply;
@@ -1465,7 +1699,7 @@ hipError_t launch_k(ggem_ctx* ctx, PairArgs a, int c, const double4* g64, const 
                     const SlotVec& v, const ChebEpi& epi, const double* u_glob, double* out) {
   if (c == kBoxShape) {
     if constexpr (P == GGEM_FP32C && NR == 1) return launch_box<EPI>(ctx, a, g32, soa, v, epi, u_glob, out);
-    if constexpr (P == GGEM_FP32C && (NR == 2 || NR == 4))
+    if constexpr (P == GGEM_FP32C && NR > 1)
       return launch_box_nr<EPI, NR>(ctx, a, g32, soa, v, epi, u_glob, out);
     if constexpr (P == GGEM_FP64 && NR == 1) return launch_box64<EPI>(ctx, a, g64, soa, v, epi, u_glob, out);
     return hipErrorInvalidConfiguration;
@@ -1597,7 +1831,26 @@ hipError_t launch_pair_points(ggem_ctx* ctx, int precision, int64_t m, const dou
 }
 
 int64_t apply_ref_blocks(const ggem_ctx* ctx) {
-  return std::max<int64_t>(blocks_for(ctx->n, 64), n_bricks(ctx));
+  return std::max<int64_t>(blocks_for(ctx->n, 64), std::max<int64_t>(n_bricks(ctx), ctx->quad_items));
+}
+
+// operands of the next launch of `left`: the largest power of two up to 8,
+// halved while only a smaller one fits the staged kernel's LDS
+int apply_chunk(const ggem_ctx* ctx, int precision, int left) {
+  int nr = left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1;
+  if (precision == GGEM_FP32C)
+    for (int m = nr; m > 1; m /= 2)
+      if (box_nr_ready(ctx, m)) return m;
+  return nr;
+}
+bool apply_reads_lists(const ggem_ctx* ctx, int precision, int nrhs) {
+  if (ctx->tune.on) return true;
+  for (int left = nrhs; left > 0;) {
+    const int nr = apply_chunk(ctx, precision, left);
+    if (!box_ready(ctx, precision, nr) || ctx->box_unstaged) return true;
+    left -= nr;
+  }
+  return false;
 }
 
 hipError_t launch_apply_ref(ggem_ctx* ctx, int precision, const SlotVec& x, const SlotVec& v, const ChebEpi& epi) {
@@ -1626,8 +1879,7 @@ hipError_t launch_apply(ggem_ctx* ctx, int precision, int nrhs, const SlotVec& x
   };
   std::vector<Chunk> chunks;
   for (int done = 0; done < nrhs;) {
-    const int left = nrhs - done;
-    const int nr = left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1;
+    const int nr = apply_chunk(ctx, precision, nrhs - done);
     ChebEpi e = epi;
     if (e.xm1.soa) e.xm1.soa += done * stride;
     if (e.y) e.y += done * stride;
