@@ -129,6 +129,8 @@ int tune_pick(ggem_ctx* ctx, const std::string& key, int ncand, const std::funct
 
 // Staged neighbour records of the lists (per brick of cells): records and
 // record numbers, with the sizes of the build's census.
+static int reserve_ell(ggem_ctx* ctx);
+
 int prepare_box(ggem_ctx* ctx) {
   ctx->box_valid = false;
   ctx->box_unstaged = false;
@@ -146,18 +148,22 @@ int prepare_box(ggem_ctx* ctx) {
   if ((rc = ensure(ctx, &ctx->box_pos, &ctx->box_pos_cap, size_t(ctx->box_recs)))) return rc;
   const size_t ne = size_t(std::max<int64_t>(ctx->box_fp64 ? ctx->ell_len : ctx->box_entries, 1));
   if ((rc = ensure(ctx, &ctx->box_idx, &ctx->box_idx_cap, ne))) return rc;
-  // bricks that are not staged fill their tensors from the lists
+  // bricks that are not staged read the lists; FP64 needs them for its
+  // tensors, and the record fill writes them along where it covers every brick
   ctx->box_unstaged = ctx->unstaged > 0;
   if (ctx->box_unstaged && (rc = ensure_ell(ctx))) return rc;
-  const hipError_t e = launch_box_fill(ctx);
+  const bool lists = ctx->box_fp64 && !ctx->ell_valid;
+  if (lists && (rc = reserve_ell(ctx))) return rc;
+  const hipError_t e = launch_box_fill(ctx, lists);
   if (e != hipSuccess) return hip_fail(ctx, e, "box_fill");
+  if (lists) ctx->ell_valid = true;
   ctx->box_max = ctx->max_recs;
   ctx->box_valid = true;
   return GGEM_OK;
 }
 
-int ensure_ell(ggem_ctx* ctx) {
-  if (ctx->ell_valid) return GGEM_OK;
+// room for the sliced lists of the current build
+static int reserve_ell(ggem_ctx* ctx) {
   hipError_t e = hipSuccess;
   int rc = GGEM_OK;
   if (ctx->ell_len < 0) {  // the lengths changed since the build (kept lists): scan them again
@@ -168,7 +174,15 @@ int ensure_ell(ggem_ctx* ctx) {
   size_t cap = size_t(ctx->ell_cap);
   if ((rc = ensure(ctx, &ctx->ell, &cap, size_t(std::max<int64_t>(ctx->ell_len, 1))))) return rc;
   ctx->ell_cap = int64_t(cap);
-  if ((e = launch_fill_ell(ctx)) != hipSuccess) return hip_fail(ctx, e, "fill_ell");
+  return GGEM_OK;
+}
+
+int ensure_ell(ggem_ctx* ctx) {
+  if (ctx->ell_valid) return GGEM_OK;
+  const int rc = reserve_ell(ctx);
+  if (rc) return rc;
+  const hipError_t e = launch_fill_ell(ctx);
+  if (e != hipSuccess) return hip_fail(ctx, e, "fill_ell");
   ctx->ell_valid = true;
   return GGEM_OK;
 }
@@ -176,6 +190,12 @@ int ensure_ell(ggem_ctx* ctx) {
 int ensure_tensors(ggem_ctx* ctx, int nrhs) {
   int rc;
   if (ctx->p.precision == GGEM_FP64) {
+    // the staged-record kernel serves one right-hand side; its records come
+    // with the lists
+    if (!ctx->box_built) {
+      if ((rc = prepare_box(ctx))) return rc;
+      ctx->box_built = true;
+    }
     if ((rc = ensure_ell(ctx))) return rc;
     if (!ctx->coef64_valid) {
       size_t cap = size_t(ctx->coef64_cap);
@@ -184,11 +204,6 @@ int ensure_tensors(ggem_ctx* ctx, int nrhs) {
       hipError_t e = launch_pair_tensors(ctx, GGEM_FP64);
       if (e != hipSuccess) return hip_fail(ctx, e, "pair tensors");
       ctx->coef64_valid = true;
-    }
-    // the staged-record kernel serves one right-hand side
-    if (!ctx->box_built) {
-      if ((rc = prepare_box(ctx))) return rc;
-      ctx->box_built = true;
     }
     return GGEM_OK;
   }
@@ -471,18 +486,18 @@ int grow_scan64(ggem_ctx* ctx, int64_t len) {
 int ggem::d2h(ggem_ctx* ctx, void* host, const void* dev, size_t bytes) {
   static_assert(kReadBufs == sizeof(ctx->read_ev) / sizeof(ctx->read_ev[0]), "an event per buffer");
   if (bytes == 0) return sync(ctx);
-  const size_t want = bytes <= kReadChunk ? bytes : kReadChunk * kReadBufs;
+  const size_t piece = std::min(kReadMax, std::max(kReadMin, (bytes / 8 + 0xffff) & ~size_t(0xffff)));
+  const size_t want = bytes <= kReadMin ? std::max(bytes, size_t(1) << 16) : piece * kReadBufs;
   if (ctx->read_cap < want) {
     if (ctx->read_h) GGEM_HIP(ctx, hipHostFree(ctx->read_h));
     ctx->read_h = nullptr;
     ctx->read_cap = 0;
-    const size_t cap = std::min(kReadChunk * kReadBufs, std::max(want, size_t(1) << 16));
-    GGEM_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->read_h), cap));
-    ctx->read_cap = cap;
+    GGEM_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->read_h), want));
+    ctx->read_cap = want;
   }
   char* const to = static_cast<char*>(host);
   const char* const from = static_cast<const char*>(dev);
-  if (bytes <= kReadChunk) {
+  if (bytes <= kReadMin) {
     GGEM_HIP(ctx, hipMemcpyAsync(ctx->read_h, from, bytes, hipMemcpyDeviceToHost, ctx->stream));
     const int rc = sync(ctx);
     if (!rc) std::memcpy(to, ctx->read_h, bytes);
@@ -490,10 +505,10 @@ int ggem::d2h(ggem_ctx* ctx, void* host, const void* dev, size_t bytes) {
   }
   for (hipEvent_t& ev : ctx->read_ev)
     if (!ev) GGEM_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-  const size_t n = (bytes + kReadChunk - 1) / kReadChunk;
-  auto part = [&](size_t i) { return std::min(kReadChunk, bytes - i * kReadChunk); };
+  const size_t n = (bytes + piece - 1) / piece;
+  auto part = [&](size_t i) { return std::min(piece, bytes - i * piece); };
   auto fetch = [&](size_t i) {
-    hipError_t e = hipMemcpyAsync(ctx->read_h + (i % kReadBufs) * kReadChunk, from + i * kReadChunk, part(i),
+    hipError_t e = hipMemcpyAsync(ctx->read_h + (i % kReadBufs) * piece, from + i * piece, part(i),
                                   hipMemcpyDeviceToHost, ctx->stream);
     return e != hipSuccess ? e : hipEventRecord(ctx->read_ev[i % kReadBufs], ctx->stream);
   };
@@ -501,7 +516,7 @@ int ggem::d2h(ggem_ctx* ctx, void* host, const void* dev, size_t bytes) {
   for (size_t i = 0; i < size_t(kReadBufs) && i < n && e == hipSuccess; ++i) e = fetch(i);
   for (size_t i = 0; i < n && e == hipSuccess; ++i) {
     if ((e = hipEventSynchronize(ctx->read_ev[i % kReadBufs])) != hipSuccess) break;
-    std::memcpy(to + i * kReadChunk, ctx->read_h + (i % kReadBufs) * kReadChunk, part(i));
+    std::memcpy(to + i * piece, ctx->read_h + (i % kReadBufs) * piece, part(i));
     if (i + kReadBufs < n) e = fetch(i + kReadBufs);
   }
   if (e == hipSuccess) return GGEM_OK;
@@ -1370,14 +1385,21 @@ int ggem_local_velocity_points(ggem_ctx* ctx, int64_t m, const double* pts, cons
   if (elem) {
     if ((rc = h2d(ctx, P.ids, elem, sizeof(int32_t) * m))) return rc;
   } else {
-    if ((e = launch_locate(ctx, m, P.io, P.ids)) != hipSuccess) return hip_fail(ctx, e, "locate");
-    std::vector<int32_t> el(m);
-    if ((rc = d2h(ctx, el.data(), P.ids, sizeof(int32_t) * m))) return rc;
-    for (int64_t q = 0; q < m; ++q)
-      if (el[q] < 0) return fail(ctx, GGEM_ERR_OUT_OF_DOMAIN, "a point lies outside the mesh");
+    // (the flag is the build's, zero while its counters are clear; the sums
+    // skip a point outside, so one synchronisation tells whether there was one)
+    if (!ctx->counters_clear) GGEM_HIP(ctx, hipMemsetAsync(ctx->flag, 0, sizeof(int32_t), ctx->stream));
+    if ((e = launch_locate(ctx, m, P.io, P.ids, ctx->flag)) != hipSuccess) return hip_fail(ctx, e, "locate");
   }
   if ((e = launch_pair_points(ctx, ctx->p.precision, m, P.io, P.ids, P.io2)) != hipSuccess)
     return hip_fail(ctx, e, "pair_points");
+  if (!elem) {
+    int64_t outside = 0;
+    if ((rc = peek(ctx, {{ctx->flag, 4}}, &outside))) return rc;
+    if (outside) {
+      ctx->counters_clear = false;
+      return fail(ctx, GGEM_ERR_OUT_OF_DOMAIN, "a point lies outside the mesh");
+    }
+  }
   return d2h(ctx, u, P.io2, sizeof(double) * 3 * m);
 }
 

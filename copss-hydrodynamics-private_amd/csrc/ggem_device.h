@@ -271,58 +271,23 @@ __device__ __forceinline__ bool brick_elem(const BoxGeom& B, int l, int& ci, int
   return ci < B.n[0] && cj < B.n[1] && ck < B.n[2];
 }
 
-// Stencil rows r0 .. r1 - 1 of the element in grid cell (ci, cj, ck) of the brick as runs
-// of box cells: calls run(q0, q1, code) for box cells q0..q1 of one row
-// with the periodic shift code of that run, in the order for_each_segment
-// visits the same cells (rows in stencil order; within a row the part past
-// the low face, then the part past the high face, then the rest, x
-// ascending), so the particles come out in the same order.
+// Stencil rows r0 .. r1 - 1 of the cell at box cell q as runs of box cells,
+// run(q0, q1) for box cells q0..q1, rows in stencil order.  Box cells outside
+// a non-periodic domain are empty and periodic images lie in the box
+// unwrapped, so no row is clamped, skipped or split; the particles come out
+// in record order.
 template <class Run>
 __device__ __forceinline__ void box_walk_rows(const BoxGeom& B, const StencilRow* __restrict__ rows, int r0, int r1,
-                                              int ci, int cj, int ck, Run&& run) {
+                                              int q, Run&& run) {
   for (int r = r0; r < r1; ++r) {
     const StencilRow R = rows[r];
-    const int jj = cj + R.dj, kk = ck + R.dk;
-    uint32_t cy = 0, cz = 0;
-    if (jj < 0 || jj >= B.n[1]) {
-      if (!B.per[1]) continue;
-      cy = jj < 0 ? 2u : 1u;
-    }
-    if (kk < 0 || kk >= B.n[2]) {
-      if (!B.per[2]) continue;
-      cz = kk < 0 ? 2u : 1u;
-    }
-    const uint32_t cyz = (cy << 2) | (cz << 4);
-    const int rowq = ((kk - B.oz) * B.ey + (jj - B.oy)) * B.ex - B.ox;  // box cell of unwrapped x = rowq + x
-    int lo = ci + R.di_lo, hi = ci + R.di_hi;
-    if (B.per[0]) {
-      if (lo < 0) {
-        run(rowq + lo, rowq - 1, cyz | 2u);
-        lo = 0;
-      }
-      if (hi >= B.n[0]) {
-        run(rowq + B.n[0], rowq + hi, cyz | 1u);
-        hi = B.n[0] - 1;
-      }
-    } else {
-      lo = lo < 0 ? 0 : lo;
-      hi = hi >= B.n[0] ? B.n[0] - 1 : hi;
-    }
-    if (lo <= hi) run(rowq + lo, rowq + hi, cyz);
+    const int qr = q + (R.dk * B.ey + R.dj) * B.ex;
+    run(qr + R.di_lo, qr + R.di_hi);
   }
 }
 
-// box_walk_rows over the whole stencil
-template <class Run>
-__device__ __forceinline__ void box_walk(const BoxGeom& B, const StencilRow* __restrict__ rows, int nrows,
-                                         int ci, int cj, int ck, Run&& run) {
-  box_walk_rows(B, rows, 0, nrows, ci, cj, ck, run);
-}
-
 // The stencil rows as offsets of box cells: row r of the cell at box cell
-// q covers box cells q + lo .. q + hi - 1 (hi one past the end).  Box cells
-// outside a non-periodic domain are empty and periodic images lie in the
-// box unwrapped, so no row is clamped or skipped.
+// q covers box cells q + lo .. q + hi - 1 (hi one past the end).
 struct BoxRow {
   int32_t lo, hi;
 };
@@ -360,11 +325,9 @@ __device__ __forceinline__ void box_walk_flat(const BoxRow* rt, const int32_t* c
 template <class Rec>
 __device__ __forceinline__ void box_walk_rec(const BoxGeom& B, const StencilRow* __restrict__ rows, int nrows,
                                              const int32_t* cst, int q, Rec&& rec) {
-  for (int r = 0; r < nrows; ++r) {
-    const StencilRow R = rows[r];
-    const int qr = q + (R.dk * B.ey + R.dj) * B.ex;
-    for (int i = cst[qr + R.di_lo], e = cst[qr + R.di_hi + 1]; i < e; ++i) rec(i);
-  }
+  box_walk_rows(B, rows, 0, nrows, q, [&](int q0, int q1) {
+    for (int i = cst[q0], e = cst[q1 + 1]; i < e; ++i) rec(i);
+  });
 }
 
 // Membership of the stencil by cell difference: per (dj, dk) the packed
@@ -389,11 +352,14 @@ struct BoxStencil {
       t[(R.dk + rz) * wy + R.dj + ry] = uint16_t((R.di_lo + 128) | ((R.di_hi + 128) << 8));
     }
   }
-  // d: cell difference + 128 per axis, one byte each (record - target)
-  __device__ __forceinline__ bool has(uint32_t d) const {
+  // d: cell difference + 128 per axis, one byte each (record - target);
+  // the row of its (dj, dk)
+  __device__ __forceinline__ uint32_t row(uint32_t d) const {
     const uint32_t j = ((d >> 8) & 0xffu) - uint32_t(128 - ry), k = ((d >> 16) & 0xffu) - uint32_t(128 - rz);
-    if (j >= uint32_t(wy) || k > uint32_t(2 * rz)) return false;
-    const uint32_t w = t[k * uint32_t(wy) + j], x = d & 0xffu;
+    return j >= uint32_t(wy) || k > uint32_t(2 * rz) ? 0x00FFu : t[k * uint32_t(wy) + j];
+  }
+  __device__ __forceinline__ bool has(uint32_t d) const {
+    const uint32_t w = row(d), x = d & 0xffu;
     return x >= (w & 0xffu) && x <= (w >> 8);
   }
 };
@@ -457,16 +423,24 @@ __device__ __forceinline__ int group_sum(int v, int g) {
   return v;
 }
 
+// LDS writes of a wave become visible to its other lanes
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 // Walk the particle slots of every element of the stencil of element
 // (ci, cj, ck): calls seg(a, b, code) for each contiguous slot range [a, b)
 // with the periodic shift code of that range (a row's x-run is one range
-// per brick it crosses), rows in stencil order, x ascending within a row.
+// per brick it crosses), rows in stencil order, x ascending within a row;
+// rows r0, r0 + step, ... where several lanes share a walk.
 template <class Seg>
 __device__ __forceinline__ void for_each_segment(const Grid& g, const StencilRow* __restrict__ rows,
                                                  int nrows, const int32_t* __restrict__ cell_start,
-                                                 int ci, int cj, int ck, Seg&& seg) {
+                                                 int ci, int cj, int ck, Seg&& seg, int r0 = 0, int step = 1) {
   const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
-  for (int r = 0; r < nrows; ++r) {
+  for (int r = r0; r < nrows; r += step) {
     const StencilRow R = rows[r];
     int jj = cj + R.dj, kk = ck + R.dk;
     uint32_t cy = 0, cz = 0;

@@ -100,8 +100,10 @@ inline int sync(ggem_ctx* ctx) {
 // of 26 MB into it took 1.5 to 1.9 ms, a copy into pinned memory 0.46 ms and
 // one thread's memcpy from there 0.35 to 0.49 ms.  So the bytes go through
 // kReadBufs pinned buffers of the context, the copy engine filling the next
-// ones while the host empties one.
-constexpr size_t kReadChunk = size_t(512) << 10;
+// ones while the host empties one.  A piece costs about 5 us beside its
+// bytes, and pinned memory about 0.1 ms a MB when it is first allocated: the
+// pieces are an eighth of the copy, between kReadMin and kReadMax.
+constexpr size_t kReadMin = size_t(512) << 10, kReadMax = size_t(2) << 20;
 constexpr int kReadBufs = 3;
 int d2h(ggem_ctx* ctx, void* host, const void* dev, size_t bytes);
 

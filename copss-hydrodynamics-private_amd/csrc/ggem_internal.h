@@ -443,7 +443,8 @@ hipError_t launch_count_pairs(ggem_ctx* ctx, int64_t* counts_d);
 hipError_t launch_fill_csr(ggem_ctx* ctx, const int64_t* offsets_d, int32_t* ids_d);
 hipError_t launch_elem_point_csr(ggem_ctx* ctx, int64_t e0, int64_t ne, int64_t* offsets_d,
                                  int32_t* ids_d, int pass);
-hipError_t launch_locate(ggem_ctx* ctx, int64_t m, const double* pts, int32_t* elem);
+// element of each point (-1 outside the mesh, which sets *outside)
+hipError_t launch_locate(ggem_ctx* ctx, int64_t m, const double* pts, int32_t* elem, int32_t* outside = nullptr);
 // slot positions and FP32C records from x_in, lists kept (PointMesh::reinit(false))
 hipError_t launch_update_slots(ggem_ctx* ctx);
 // GGEM_COMPAT_STALE_LISTS: slots with an empty new list take their kept
@@ -527,8 +528,9 @@ struct ChebEpi {
 };
 // pair tensors of every list entry for the given precision
 hipError_t launch_pair_tensors(ggem_ctx* ctx, int precision);
-// records and record numbers of every staged brick
-hipError_t launch_box_fill(ggem_ctx* ctx);
+// records and record numbers of every staged brick; FP64 with with_lists:
+// the sliced lists too (every brick with targets staged)
+hipError_t launch_box_fill(ggem_ctx* ctx, bool with_lists);
 // whether the context's FP32C lists can be staged per brick
 bool box_supported(const ggem_ctx* ctx);
 hipError_t launch_pair_beads(ggem_ctx* ctx, int precision, int epi, const double* u_glob,

@@ -705,6 +705,7 @@ struct BoxArgs {
   int32_t waves_cap;
   int32_t recs_cap;
   int32_t fp64;          // FP64: every pair stored, at its list position
+  uint32_t* ell;         // FP64: the lists themselves, written along (null: already filled)
   const StencilRow* rows;  // stencil rows (a batched context: all systems', SysGrid::row_off)
   int32_t nrows;
 };
@@ -753,6 +754,7 @@ __global__ void __launch_bounds__(kBoxThreads) k_box_fill(PairArgs a, BoxArgs b)
   int32_t* wpre = cst + b.cells_cap + 1;                               // [waves_cap + 1] entry rows before each wave
   __shared__ int32_t s_w[kBoxThreads / 64];
   __shared__ uint16_t s_st[kStencilTab];
+  uint32_t* rent = reinterpret_cast<uint32_t*>(wpre + b.waves_cap + 1);  // [recs_cap] list entry of each record (ell)
   const int64_t brick = blockIdx.x;
   const int64_t c0 = brick * kBrickCells;
   const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
@@ -818,6 +820,7 @@ __global__ void __launch_bounds__(kBoxThreads) k_box_fill(PairArgs a, BoxArgs b)
           b.pos[r0 + i] = rec;
         }
         rpos[i] = rec;
+        if (b.ell) rent[i] = uint32_t(t[u]) | (B.shift_code(x, y, z) << kSlotBits);
       }
     }
   }
@@ -882,13 +885,17 @@ __global__ void __launch_bounds__(kBoxThreads) k_box_fill(PairArgs a, BoxArgs b)
       const int64_t bb = b.eoff[brick] + 64 * int64_t(wpre[i >> 6]) + (i & 63);
       const Target T = target(s);
       uint16_t* __restrict__ out = entries(s, bb);
+      uint32_t* __restrict__ lst = b.ell ? b.ell + a.slice_off[s >> 6] + (s & 63) : nullptr;
       const int kept = wave_records(
           B, st, cst, T.z,
           [&](int r) {
             const float4 pt = rpos[r];
             return r != T.self && st.has(__float_as_uint(pt.w) + T.kb) && (all || keeps(T, pt));
           },
-          [&](int r, int k) { out[int64_t(k) * kSlice] = uint16_t(r); });
+          [&](int r, int k) {
+            out[int64_t(k) * kSlice] = uint16_t(r);
+            if (lst) lst[int64_t(k) * kSlice] = rent[r];
+          });
       if (lane == 0) b.base[sb + i] = packed(T, bb, kept);
     }
     return;
@@ -902,11 +909,16 @@ __global__ void __launch_bounds__(kBoxThreads) k_box_fill(PairArgs a, BoxArgs b)
     }
     const Target T = target(s);
     uint16_t* out = entries(s, bb);
+    uint32_t* lst = b.ell ? b.ell + a.slice_off[s >> 6] + (s & 63) : nullptr;
     int kept = 0;
     box_walk_rec(B, rows, nrows, cst, T.q, [&](int r) {
       if (r == T.self || !(all || keeps(T, rpos[r]))) return;
       *out = uint16_t(r);
       out += kSlice;
+      if (lst) {
+        *lst = rent[r];
+        lst += kSlice;
+      }
       ++kept;
     });
     b.base[sb + i] = packed(T, bb, kept);
@@ -1468,6 +1480,16 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box64(PairArgs a, BoxView
 
 // Field points: sum over the element's particle list, own element
 // included, no exclusion (ggem_stokes.C:396-420), full minimum image.
+// kPointLanes lanes share a point: lane l walks the stencil rows l, l +
+// kPointLanes, ... (a chain of dependent loads) and leaves their particles in
+// the point's list in LDS, then the lanes take the list's entries in turn, so
+// that the tensors, two erf and two exp each, are evaluated on full lanes; the
+// lanes' sums are added pairwise.  100,000 points of the 20,000-bead
+// suspension (29 rows, 9.5 particles a point), FP64: a lane per point 210 us,
+// sixteen that sum as they walk 125 us, with the lists 60 us.  A point with
+// more than kPointList particles is summed on the walk.  Points without an
+// element (elem < 0, the caller reports them) are skipped.
+constexpr int kPointLanes = 16, kPointList = 128;
 template <int P>
 __global__ void __launch_bounds__(kBlock) k_pair_points(PairArgs a, const StencilRow* __restrict__ rows,
                                                        int nrows, const int32_t* __restrict__ cell_start,
@@ -1476,40 +1498,67 @@ __global__ void __launch_bounds__(kBlock) k_pair_points(PairArgs a, const Stenci
                                                        const double* __restrict__ pts,
                                                        const int32_t* __restrict__ elem,
                                                        double* __restrict__ u) {
-  const int64_t q = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (q >= m) return;
+  __shared__ int32_t s_list[kBlock / kPointLanes][kPointList];
+  const int64_t q = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kPointLanes;
+  const int l = int(threadIdx.x) & (kPointLanes - 1);
+  if (q >= m || elem[q] < 0) return;  // (a point's lanes together)
+  int32_t* const list = s_list[threadIdx.x / kPointLanes];
   int ci, cj, ck;
   elem_ijk(a.g, elem[q], ci, cj, ck);
   const double4 xq = make_double4(pts[3 * q], pts[3 * q + 1], pts[3 * q + 2], 0.0);
-  double ux = 0, uy = 0, uz = 0;
+  double us[3] = {0.0, 0.0, 0.0};
   KahanF kx, ky, kz;
-  for_each_segment(a.g, rows, nrows, cell_start, ci, cj, ck, [&](int32_t lo, int32_t hi, uint32_t) {
-    for (int32_t t = lo; t < hi; ++t) {
-      double dx, dy, dz;
-      pair_disp<true>(a.g, xq, a.x4[t], 0u, dx, dy, dz);
-      if (P == GGEM_FP64) {
-        const double4 f = fg64[t];
-        green_acc_f64(a.k, dx, dy, dz, f.x, f.y, f.z, ux, uy, uz);
-      } else {
-        const float4 f = fg32[t];
-        const float fx = float(dx), fy = float(dy), fz = float(dz);
-        float A, Bx;
-        green_coef_f32(a.k32, fx * fx + fy * fy + fz * fz, A, Bx);
-        const float B = Bx * (fx * f.x + fy * f.y + fz * f.z);
-        kx.add(A * f.x + B * fx);
-        ky.add(A * f.y + B * fy);
-        kz.add(A * f.z + B * fz);
-      }
+  auto add = [&](int32_t t) {
+    double dx, dy, dz;
+    pair_disp<true>(a.g, xq, a.x4[t], 0u, dx, dy, dz);
+    if (P == GGEM_FP64) {
+      const double4 f = fg64[t];
+      green_acc_f64(a.k, dx, dy, dz, f.x, f.y, f.z, us[0], us[1], us[2]);
+    } else {
+      const float4 f = fg32[t];
+      const float fx = float(dx), fy = float(dy), fz = float(dz);
+      float A, Bx;
+      green_coef_f32(a.k32, fx * fx + fy * fy + fz * fz, A, Bx);
+      const float B = Bx * (fx * f.x + fy * f.y + fz * f.z);
+      kx.add(A * f.x + B * fx);
+      ky.add(A * f.y + B * fy);
+      kz.add(A * f.z + B * fz);
     }
-  });
-  if (P != GGEM_FP64) {
-    ux = kx.value();
-    uy = ky.value();
-    uz = kz.value();
+  };
+  auto walk = [&](auto&& seg) {
+    for_each_segment(a.g, rows, nrows, cell_start, ci, cj, ck, seg, l, kPointLanes);
+  };
+  int mine = 0;
+  walk([&](int32_t lo, int32_t hi, uint32_t) { mine += hi - lo; });
+  int incl = mine;
+#pragma unroll
+  for (int o = 1; o < kPointLanes; o <<= 1) {
+    const int y = __shfl_up(incl, o, kPointLanes);
+    if (l >= o) incl += y;
   }
-  u[3 * q] = ux;
-  u[3 * q + 1] = uy;
-  u[3 * q + 2] = uz;
+  const int total = __shfl(incl, kPointLanes - 1, kPointLanes);
+  if (total <= kPointList) {
+    int at = incl - mine;
+    walk([&](int32_t lo, int32_t hi, uint32_t) {
+      for (int32_t t = lo; t < hi; ++t) list[at++] = t;
+    });
+    wave_lds_sync();  // (a point's lanes are in one wave)
+    for (int j = l; j < total; j += kPointLanes) add(list[j]);
+  } else {
+    walk([&](int32_t lo, int32_t hi, uint32_t) {
+      for (int32_t t = lo; t < hi; ++t) add(t);
+    });
+  }
+  if (P != GGEM_FP64) {
+    us[0] = kx.value();
+    us[1] = ky.value();
+    us[2] = kz.value();
+  }
+#pragma unroll
+  for (int o = 1; o < kPointLanes; o <<= 1)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) us[d] += __shfl_xor(us[d], o, 64);
+  if (l < 3) u[3 * q + l] = l == 0 ? us[0] : (l == 1 ? us[1] : us[2]);
 }
 
 // erfcx fit (see erfcx_f32): coefficients of Q in x = 2t/t_max - 1,
@@ -1578,6 +1627,7 @@ BoxArgs box_args(const ggem_ctx* ctx) {
   b.pos = ctx->box_pos;
   b.idx = ctx->box_idx;
   b.fp64 = ctx->box_fp64 ? 1 : 0;
+  b.ell = nullptr;
   return b;
 }
 
@@ -1769,7 +1819,7 @@ hipError_t launch_pair_tensors(ggem_ctx* ctx, int precision) {
 
 bool box_supported(const ggem_ctx* ctx) { return ctx->n > 0 && !explicit_minimg(ctx); }
 
-hipError_t launch_box_fill(ggem_ctx* ctx) {
+hipError_t launch_box_fill(ggem_ctx* ctx, bool with_lists) {
   ProfScope ps(ctx, "box_fill");
   BoxArgs b = box_args(ctx);
   // LDS tables sized for the largest box and the most crowded brick
@@ -1783,7 +1833,9 @@ hipError_t launch_box_fill(ggem_ctx* ctx) {
   b.recs_cap = ctx->max_recs;
   if (b.waves_cap > kBoxMaxWaves || b.recs_cap > kBoxMaxRecs) return hipErrorInvalidValue;
   const unsigned split = brick_split(ctx);
-  const size_t lds = sizeof(float4) * size_t(b.recs_cap) + sizeof(int32_t) * (2 * size_t(b.cells_cap) + b.waves_cap + 2);
+  b.ell = with_lists ? ctx->ell : nullptr;
+  const size_t lds = sizeof(float4) * size_t(b.recs_cap) + sizeof(int32_t) * (2 * size_t(b.cells_cap) + b.waves_cap + 2) +
+                     (with_lists ? sizeof(uint32_t) * size_t(b.recs_cap) : 0);
   if (ctx->nsys > 1)
     hipLaunchKernelGGL(k_box_fill<true>, dim3(n_bricks(ctx), split), dim3(kBoxThreads), lds, ctx->stream, make_args(ctx),
                        b);
@@ -1822,10 +1874,10 @@ hipError_t launch_pair_points(ggem_ctx* ctx, int precision, int64_t m, const dou
   const PairArgs a = make_args(ctx);
   ProfScope ps(ctx, precision == GGEM_FP64 ? "pair_points_fp64" : "pair_points_fp32c");
   if (precision == GGEM_FP64)
-    hipLaunchKernelGGL(k_pair_points<GGEM_FP64>, dim3(blocks_for(m)), dim3(kBlock), 0, ctx->stream, a,
+    hipLaunchKernelGGL(k_pair_points<GGEM_FP64>, dim3(blocks_for(m * kPointLanes)), dim3(kBlock), 0, ctx->stream, a,
                        ctx->rows_d, ctx->n_rows, ctx->cell_start, ctx->fg32, ctx->fg64, m, pts, elem, u);
   else
-    hipLaunchKernelGGL(k_pair_points<GGEM_FP32C>, dim3(blocks_for(m)), dim3(kBlock), 0, ctx->stream, a,
+    hipLaunchKernelGGL(k_pair_points<GGEM_FP32C>, dim3(blocks_for(m * kPointLanes)), dim3(kBlock), 0, ctx->stream, a,
                        ctx->rows_d, ctx->n_rows, ctx->cell_start, ctx->fg32, ctx->fg64, m, pts, elem, u);
   return hipGetLastError();
 }

@@ -340,7 +340,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_spread(SpreadArgs<T> a, const do
 // the next group of 64 / NQ1 consecutive elements of the brick with
 // k_spread's lane layout (NQ1 lanes an element, one per Gauss x-index):
 // the element lists, the record numbers of each stencil in the element
-// list's order (box_walk), go to the wave's own LDS buffer, the lanes of
+// list's order (box_walk_rows), go to the wave's own LDS buffer, the lanes of
 // an element walking a third (half) of the stencil rows each; the lists
 // are summed with k_spread's operations (the cell difference from the
 // packed box cells equals the one k_spread forms from the list's shift
@@ -368,13 +368,6 @@ struct BrickSpreadArgs {
   int32_t list_cap;        // 16-bit entries of each wave's list buffer (at least recs_cap)
   uint8_t* unstaged;       // [bricks] 1: the box exceeds the record table (written by k_spread_brick)
 };
-
-// LDS writes of a wave visible to its other lanes
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
 
 __device__ __forceinline__ float pick3(float a0, float a1, float a2, int k) { return k == 0 ? a0 : (k == 1 ? a1 : a2); }
 
@@ -532,7 +525,7 @@ __device__ __forceinline__ void spread_brick(const BrickSpreadArgs& a, const dou
       int c = 0, ci, cj, ck;
       int64_t e;
       if (lw < EPW && l < kBrickCells && brick_elem(B, l, ci, cj, ck, e))
-        box_walk_rows(B, a.rows, rlo, rhi, ci, cj, ck, [&](int q0, int q1, uint32_t) { c += cst[q1 + 1] - cst[q0]; });
+        box_walk_rows(B, a.rows, rlo, rhi, B.box_cell(ci, cj, ck), [&](int q0, int q1) { c += cst[q1 + 1] - cst[q0]; });
       if (lw < EPW && l < kBrickCells) s_cnt[l * NQ1 + qa] = uint16_t(c);
     }
     for (int i = int(threadIdx.x); i < kSortBuckets; i += NT) s_hist[i] = 0;
@@ -606,7 +599,7 @@ __device__ __forceinline__ void spread_brick(const BrickSpreadArgs& a, const dou
         // (3) the lists
         if (elem && lw < take) {
           int k = off;
-          box_walk_rows(B, a.rows, rlo, rhi, ci, cj, ck, [&](int q0, int q1, uint32_t) {
+          box_walk_rows(B, a.rows, rlo, rhi, B.box_cell(ci, cj, ck), [&](int q0, int q1) {
             for (int r = cst[q0], re = cst[q1 + 1]; r < re; ++r) mine[k++] = uint16_t(r);
           });
         }
@@ -663,7 +656,7 @@ __device__ __forceinline__ void spread_brick(const BrickSpreadArgs& a, const dou
           }
         } else {
           int k = 0;
-          box_walk(B, a.rows, a.nrows, ci, cj, ck, [&](int q0, int q1, uint32_t) {
+          box_walk_rows(B, a.rows, 0, a.nrows, B.box_cell(ci, cj, ck), [&](int q0, int q1) {
             for (int q = q0; q <= q1; ++q) {
               int x, y, z;
               B.xyz(q, x, y, z);

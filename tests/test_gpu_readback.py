@@ -1,6 +1,6 @@
-"""Results copied to the host in pieces arrive whole: sizes around the pinned
-buffers' 512 KiB (21845.3 vectors of three doubles) and around the three of
-them, odd remainders, several copies in turn."""
+"""Results copied to the host in pieces arrive whole: sizes around the smallest
+piece's 512 KiB (21845.3 vectors of three doubles), around three of them and
+eight (longer pieces from there on), odd remainders, several copies in turn."""
 import numpy as np
 import pytest
 
@@ -10,7 +10,7 @@ import workloads as W
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 2730, 21845, 21846, 65535, 65536, 65537, 87382, 150001])
+@pytest.mark.parametrize("n", [1, 2730, 21845, 21846, 65535, 65536, 65537, 87382, 150001, 174762, 174763, 800001])
 def test_noise_round_trip(n):
     cfg = W._cfg([0, 0, 0], [400] * 3, [1, 1, 1], [100] * 3)
     with G.Context(cfg) as ctx:
