@@ -94,6 +94,8 @@ __device__ __forceinline__ int div_small(int q, float inv_d) { return int((float
 constexpr int kBrickCells = 1 << (3 * kBrickBits);
 // blocks that share a brick's targets in the quad pair sums
 constexpr int kQuadShare = 64, kQuadShares = 4;
+constexpr int kItemRecShift = 48;
+constexpr int64_t kItemRecMask = (int64_t(1) << kItemRecShift) - 1;
 __device__ __forceinline__ int quad_shares(int nt) { return min(kQuadShares, (nt + kQuadShare - 1) / kQuadShare); }
 constexpr int kBoxMaxCells = 8192;  // box cells whose tables a brick kernel keeps in LDS
 constexpr int kBoxBits = 6;         // box coordinates: below 2^6 per axis

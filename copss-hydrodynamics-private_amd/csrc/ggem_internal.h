@@ -63,6 +63,14 @@ struct SysGrid {
   int32_t reach[3];  // largest stencil offset per axis, in cells
 };
 
+// What one block of the quad pair sums takes: a share of a brick's targets
+// and the brick's records.  One 16-byte word, so that a block starts with one
+// load instead of a chain of three.
+struct alignas(16) QuadItem {
+  int32_t t0, nt;  // first target (slot order), targets
+  int64_t rec;     // first record (low kItemRecShift bits), records above
+};
+
 // Layout of the FP32C coefficient table (ggem_util_fp32c_table): n1
 // intervals of width d1 on [0, s1), then n2 of width d2, then one zero
 // interval; 16 floats per interval.
@@ -232,7 +240,7 @@ struct ggem_ctx {
   int32_t max_targets = 0;        // most targets of a brick
   int32_t unstaged = 0;           // bricks with targets that are not staged
   int32_t full_bricks = 0;        // bricks with targets
-  uint32_t* quad_work = nullptr;  // [quad_items] brick and share of every block of the quad pair sums
+  ggem::QuadItem* quad_work = nullptr;  // [quad_items] what every block of the quad pair sums takes
   size_t quad_work_cap = 0;
   int64_t quad_items = 0;
   uint8_t* spread_unstaged = nullptr;  // [bricks] the brick spreading's boxes over its record table

@@ -743,7 +743,7 @@ struct SizesArgs {
   int64_t nbricks;
   int32_t* flag;
   int64_t* pairs;
-  uint32_t* work;
+  QuadItem* work;
   int64_t* host;  // [10] flag, pairs, records, entries, list slots, the maxima (4), work items
 };
 __global__ void __launch_bounds__(kSizesThreads) k_build_sizes(SizesArgs a) {
@@ -753,22 +753,42 @@ __global__ void __launch_bounds__(kSizesThreads) k_build_sizes(SizesArgs a) {
   if (blockIdx.x == 4) {
     __shared__ int32_t s_n[NW];
     int carry = 0;
+    int64_t rcarry = 0;
     for (int64_t c0 = 0; c0 < a.nbricks; c0 += kSizesThreads) {
       const int64_t k = c0 + threadIdx.x;
-      const int m = k < a.nbricks ? quad_shares(a.cs[(k + 1) * kBrickCells] - a.cs[k * kBrickCells]) : 0;
+      const int sb = k < a.nbricks ? a.cs[k * kBrickCells] : 0;
+      const int nt = k < a.nbricks ? a.cs[(k + 1) * kBrickCells] - sb : 0;
+      const int64_t nrec = k < a.nbricks ? a.box_cnt[k] : 0;
+      const int m = quad_shares(nt);
       int incl = m;
+      int64_t rincl = nrec;
       for (int o = 1; o < 64; o <<= 1) {
         const int y = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += y;
+        const int64_t r = __shfl_up(rincl, o, 64);
+        if (lane >= o) {
+          incl += y;
+          rincl += r;
+        }
       }
-      if (lane == 63) s_n[wv] = incl;
+      if (lane == 63) {
+        s_n[wv] = incl;
+        sh[wv] = rincl;
+      }
       __syncthreads();
       int at = carry + incl - m;
+      int64_t r0 = rcarry + rincl - nrec;
       for (int w = 0; w < NW; ++w) {
-        if (w < wv) at += s_n[w];
+        if (w < wv) {
+          at += s_n[w];
+          r0 += sh[w];
+        }
         carry += s_n[w];
+        rcarry += sh[w];
       }
-      for (int y = 0; y < m; ++y) a.work[at + y] = uint32_t(k) * kQuadShares + uint32_t(y);
+      for (int y = 0; y < m; ++y) {
+        const int t0 = int(int64_t(nt) * y / m), t1 = int(int64_t(nt) * (y + 1) / m);
+        a.work[at + y] = QuadItem{sb + t0, t1 - t0, r0 | (nrec << kItemRecShift)};
+      }
       __syncthreads();
     }
     if (threadIdx.x == 0) a.host[9] = carry;

@@ -222,12 +222,10 @@ __global__ void __launch_bounds__(BLK) k_tensors(PairArgs a, double4* __restrict
 // What the epilogue of a target slot reads once for all its components.
 struct EpiTarget {
   double da, db, ck, cm1, c0;  // EPI_CHEB
-  int64_t p;                   // EPI_LOCAL, EPI_MOBILITY: particle of the slot
 };
 template <int EPI>
 __device__ __forceinline__ EpiTarget epi_target(const PairArgs& a, int64_t s, const ChebEpi& epi) {
-  EpiTarget T{epi.da, epi.db, epi.c, epi.cm1, epi.c0, 0};
-  if (EPI == EPI_LOCAL || EPI == EPI_MOBILITY) T.p = a.perm[s];
+  EpiTarget T{epi.da, epi.db, epi.c, epi.cm1, epi.c0};
   if (EPI == EPI_CHEB && epi.dpar) {
     const double* pp = epi.dpar + int64_t(epi.sys ? epi.sys[s] : 0) * epi.pstride;
     T.da = pp[0];
@@ -239,31 +237,63 @@ __device__ __forceinline__ EpiTarget epi_target(const PairArgs& a, int64_t s, co
   return T;
 }
 
-// Epilogue of component q of the pair sum of target slot s for operand r, m
-// the sum (see Epi); the value of the new vector (EPI_CHEB, EPI_REF), whose
-// gather record is left to epi_record.
+// What the epilogue of component q of target slot s and operand r reads
+// besides the pair sum: a kernel with a short pair loop loads it ahead.
+struct EpiIn {
+  double xv;  // own force, own component of the operand
+  double xm;  // u_glob; x_{k-1}
+  double y, my;
+  int64_t p;  // EPI_LOCAL, EPI_MOBILITY: particle of the slot
+};
 template <int EPI>
-__device__ __forceinline__ double epi_component(const PairArgs& a, const EpiTarget& T, int64_t s, int r, int q, double m,
-                                                const double* __restrict__ xsoa, const SlotVec& v, const ChebEpi& epi,
-                                                const double* __restrict__ u_glob, double* __restrict__ out,
-                                                double (&dots)[3]) {
+__device__ __forceinline__ EpiIn epi_in(const PairArgs& a, int64_t s, int r, int q,
+                                        const double* __restrict__ xsoa, const ChebEpi& epi,
+                                        const double* __restrict__ u_glob) {
+  EpiIn I{0.0, 0.0, 0.0, 0.0, 0};
+  if constexpr (EPI == EPI_LOCAL || EPI == EPI_MOBILITY) {
+    I.xv = a.fs[q * a.n + s];  // forces are the operand: own force from the FP64 store
+    I.p = a.perm[s];
+    if (EPI == EPI_MOBILITY && u_glob) I.xm = u_glob[3 * I.p + q];
+  } else {
+    const int64_t idx = int64_t(r) * 3 * a.n + int64_t(q) * a.n + s;
+    I.xv = xsoa[idx];
+    if constexpr (EPI == EPI_REF) {
+      if (epi.ref.term != 0) {
+        I.y = epi.y[idx];
+        I.my = epi.ref.my[idx];
+        I.xm = epi.xm1.soa[idx];
+      }
+    } else if (epi.kind > 1) {
+      I.xm = epi.xm1.soa[idx];
+      if (epi.ymask) I.y = epi.y[idx];
+    }
+  }
+  return I;
+}
+
+// Epilogue of component q of the pair sum of target slot s for operand r, m
+// the sum (see Epi) and I = epi_in(...); the value of the new vector
+// (EPI_CHEB, EPI_REF), whose gather record is left to epi_record.
+template <int EPI>
+__device__ __forceinline__ double epi_component(const PairArgs& a, const EpiTarget& T, const EpiIn& I, int64_t s,
+                                                int r, int q, double m, const SlotVec& v, const ChebEpi& epi,
+                                                double* __restrict__ out, double (&dots)[3]) {
   const int64_t n = a.n;
   if constexpr (EPI == EPI_LOCAL || EPI == EPI_MOBILITY) {
-    // forces are the operand: own force from the FP64 store
-    const double fo = a.fs[q * n + s];
+    const double fo = I.xv;
     double u = m;
     if (a.k.point_type == GGEM_LAGRANGIAN_POINT) u += a.k.coeff_2 * fo;  // self term
     if (EPI == EPI_MOBILITY) {
-      const double ug = u_glob ? u_glob[3 * T.p + q] : 0.0;
+      const double ug = I.xm;
       if (a.k.point_type == GGEM_POLYMER_BEAD) u = ug + u - a.k.coeff_1 * fo + fo;
       else if (a.k.point_type == GGEM_LAGRANGIAN_POINT) u = ug + u;
       else u = 0.0;
     }
-    out[3 * T.p + q] = u;
+    out[3 * I.p + q] = u;
     return u;
   } else {
     const int64_t idx = int64_t(r) * 3 * n + int64_t(q) * n + s;
-    const double xv = xsoa[idx];
+    const double xv = I.xv;
     if (a.k.point_type == GGEM_POLYMER_BEAD) m = m - a.k.coeff_1 * xv + xv;
     else if (a.k.point_type == GGEM_LAGRANGIAN_POINT) m = m + a.k.coeff_2 * xv;
     else m = 0.0;
@@ -275,9 +305,9 @@ __device__ __forceinline__ double epi_component(const PairArgs& a, const EpiTarg
         nv = T.db * xv + T.da * m;
         dots[0] += m * xv;
       } else {
-        y += epi.y[idx];
-        my += R.my[idx];
-        nv = 2. * T.db * xv + 2. * T.da * m - epi.xm1.soa[idx];
+        y += I.y;
+        my += I.my;
+        nv = 2. * T.db * xv + 2. * T.da * m - I.xm;
         dots[0] += my * my;
       }
       dots[1] += y * y;
@@ -289,17 +319,17 @@ __device__ __forceinline__ double epi_component(const PairArgs& a, const EpiTarg
     } else if (epi.kind == 1) {
       nv = T.db * xv + T.da * m;
     } else {
-      const double xm = epi.xm1.soa[idx];
+      const double xm = I.xm;
       nv = 2. * T.db * xv + 2. * T.da * m;
       nv += -1.0 * xm;
       if (epi.ymask == 4) {
-        epi.y[idx] += T.ck * nv;
+        epi.y[idx] = I.y + T.ck * nv;
       } else if (epi.ymask) {  // x_{k-1}, x_k and x_{k+1} terms in one update of y
         double add = 0.0;
         if (epi.ymask & 1) add += T.cm1 * xm;
         if (epi.ymask & 2) add += T.c0 * xv;
         if (epi.ymask & 4) add += T.ck * nv;
-        epi.y[idx] += add;
+        epi.y[idx] = I.y + add;
       }
     }
     v.soa[idx] = nv;
@@ -328,7 +358,8 @@ __device__ __forceinline__ void apply_epilogue(const PairArgs& a, int64_t s, con
     double nv[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q)
-      nv[q] = epi_component<EPI>(a, T, s, r, q, acc[r][q], xsoa, v, epi, u_glob, out, dots);
+      nv[q] = epi_component<EPI>(a, T, epi_in<EPI>(a, s, r, q, xsoa, epi, u_glob), s, r, q, acc[r][q], v, epi, out,
+                                 dots);
     epi_record<NR, EPI>(s, r, nv[0], nv[1], nv[2], v);
   }
 }
@@ -357,17 +388,13 @@ __device__ __forceinline__ T quad_add(T p, T v) {
 }
 
 // Epilogue of the pair sum of target slot s of a quad whose lanes all hold
-// it: lane c < 3 takes component c
+// it: lane c < 3 takes component c, with I = epi_in(..., c, ...)
 template <int EPI>
-__device__ __forceinline__ void quad_epilogue(const PairArgs& a, int64_t s, int c, double m0, double m1, double m2,
-                                              const double* __restrict__ xsoa, const SlotVec& v, const ChebEpi& epi,
-                                              const double* __restrict__ u_glob, double* __restrict__ out,
-                                              double (&dots)[3]) {
+__device__ __forceinline__ void quad_epilogue(const PairArgs& a, const EpiTarget& T, const EpiIn& I, int64_t s, int c,
+                                              double m0, double m1, double m2, const SlotVec& v, const ChebEpi& epi,
+                                              double* __restrict__ out, double (&dots)[3]) {
   double nv = 0.0;
-  if (c < 3) {
-    const EpiTarget T = epi_target<EPI>(a, s, epi);
-    nv = epi_component<EPI>(a, T, s, 0, c, c == 0 ? m0 : (c == 1 ? m1 : m2), xsoa, v, epi, u_glob, out, dots);
-  }
+  if (c < 3) nv = epi_component<EPI>(a, T, I, s, 0, c, c == 0 ? m0 : (c == 1 ? m1 : m2), v, epi, out, dots);
   const double x = quad_get<0>(nv), y = quad_get<1>(nv), z = quad_get<2>(nv);
   if (c == 0) epi_record<1, EPI>(s, 0, x, y, z, v);
 }
@@ -681,6 +708,13 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
 // A brick whose box holds more than kBoxMaxRecs records reads its list and
 // gathers the neighbours' records from global memory.
 constexpr int kBoxThreads = 256;
+// FP64 with a lane per target: threads for twice 256 targets.  A block of 256
+// goes round a second time in every brick with more (23 of 100 at 244 targets
+// a brick), with a few lanes and at the latency of a whole list; the further
+// threads cost nothing and help to stage.  125,000 beads: 41.6 -> 35.2 us per
+// application, and 34.2 us with the tensors loaded a group ahead (3.0 TB/s).
+// FP32C is not bound by that latency (1M beads: 82.7 us either way).
+constexpr int kDenseThreads = 512;
 // A target's packed entry base: the offset of its entry 0 (below 2^40), its
 // own record number (12 bits) and, in staged bricks, its count of stored
 // (kept) entries (12 bits; a staged box holds at most kBoxMaxRecs records).
@@ -721,7 +755,7 @@ struct BoxView {
   const uint32_t* slot;
   const float4* pos;
   const uint16_t* idx;
-  const uint32_t* work;  // k_apply_quad: brick * kQuadShares + share of every block
+  const QuadItem* work;  // k_apply_quad: what every block sums
 };
 
 // Entry layout of a brick: its targets in the order tgt, in waves of 64;
@@ -1137,42 +1171,43 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box(PairArgs a, BoxView b
 // (20,000 beads: 39 of 256 lanes) and walks each list alone: one operand 9.1
 // -> 6.6 us per application there, 30 -> 21 us for chains in a slit (25,600
 // beads).  Several operands used to gather from global memory, a lane per
-// target: eight of 20,000 beads 34.8 -> 12.9 us, four of 272,000 beads in 64
-// suspensions 176 -> 131 us (bound by staging 16 records per target).
+// target: eight of 20,000 beads 34.8 -> 12.8 us, four of 272,000 beads in 64
+// suspensions 176 -> 128 us (16 records staged per target, three blocks per
+// CU in LDS).
+// A block of 39 targets is a chain of dependent loads, not work: the item
+// word holds what took two more loads, and the first target's words, record
+// numbers and epilogue inputs are requested while the records are staged
+// (20,000 beads 6.6 -> 5.6 us, chains 21.9 -> 21.1 us).
 template <int EPI, bool ONE, int NR>
 __global__ void __launch_bounds__(kBoxThreads) k_apply_quad(PairArgs a, BoxView b, const float4* __restrict__ xg,
                                                            const double* __restrict__ xsoa, SlotVec v, ChebEpi epi,
                                                            const double* __restrict__ u_glob,
                                                            double* __restrict__ out) {
   extern __shared__ float4 lds[];
-  if (epi.skip && *epi.skip) return;  // uniform over the grid
-  const uint32_t item = b.work[block_index(a.xcd)];
-  const int64_t brick = item / kQuadShares;
-  const int64_t c0 = brick * kBrickCells;
-  const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
-  const int nt = se - sb, shares = quad_shares(nt), y = int(item % kQuadShares);
-  const int t0 = nt * y / shares, t1 = nt * (y + 1) / shares;
+  const QuadItem item = b.work[block_index(a.xcd)];
+  if ((epi.skip && *epi.skip) || item.nt <= 0) return;  // uniform over the grid (every item has targets)
+  const int nt = item.nt, nrec = int(item.rec >> kItemRecShift);
+  const int64_t r0 = item.rec & kItemRecMask;
   double dots[3] = {0.0, 0.0, 0.0};
-  const int64_t r0 = b.off[brick];
-  const int nrec = int(b.off[brick + 1] - r0);
   const int c = int(threadIdx.x) & 3;
-  int i = t0 + (int(threadIdx.x) >> 2);
-  // the first target's words are on their way while the records are staged
-  int32_t s = 0;
-  int64_t bpk = 0;
-  if (i < t1) {
-    s = b.tgt[sb + i];
-    bpk = b.base[sb + i];
-  }
+  constexpr int PER = NR <= 4 ? 1 : NR / 4;  // operands per lane
+  const int op = NR == 1 ? 0 : (NR == 2 ? (c & 1) : c);
   float4* s_tab = lds;                       // coefficient table
   float4* rpos = lds + kTabStride * a.ct.n;  // [nrec] offset xyz, packed box cell
   float4* rval = rpos + nrec;                // [nrec][NR] operands
-  load_tab(s_tab, a);
+  float hx = float(a.g.h[0]), hy = float(a.g.h[1]), hz = float(a.g.h[2]);
+  if (a.sys) {
+    const SysGrid* S = a.sys + a.sys_slot[item.t0];
+    hx = float(S->g.h[0]);
+    hy = float(S->g.h[1]);
+    hz = float(S->g.h[2]);
+  }
   if (nrec == 0) {  // not staged (one operand only)
+    load_tab(s_tab, a);
     __syncthreads();
     if constexpr (NR == 1)
-      for (int j = t0 + int(threadIdx.x); j < t1; j += kBoxThreads) {
-        const int64_t sj = b.tgt[sb + j];
+      for (int j = int(threadIdx.x); j < nt; j += kBoxThreads) {
+        const int64_t sj = b.tgt[item.t0 + j];
         double acc[1][3];
         fp32c_pairs_global(a, sj, s_tab, xg, acc);
         apply_epilogue<1, EPI>(a, sj, acc, xsoa, v, epi, u_glob, out, dots);
@@ -1180,23 +1215,76 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad(PairArgs a, BoxView 
     if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
     return;
   }
-  for (int j = int(threadIdx.x); j < nrec; j += kBoxThreads) {
-    const uint32_t t = b.slot[r0 + j];
-    rpos[j] = b.pos[r0 + j];
+  // A target's words, its first record numbers and what its epilogue reads;
+  // the first target's are on their way while the records are staged.
+  int i = int(threadIdx.x) >> 2;
+  int32_t s = 0;
+  int64_t bpk = 0;
+  const uint16_t* __restrict__ ci = b.idx;
+  int cnt = 0, last = 0;
+  uint32_t e0 = 0, e1 = 0;
+  const EpiTarget T = epi_target<EPI>(a, item.t0, epi);  // (a brick's targets are of one system)
+  constexpr int NC = NR == 1 ? 1 : 3;  // components per lane
+  EpiIn in[PER][NC];
+  auto words = [&]() {
+    if (i >= nt) return;
+    s = b.tgt[item.t0 + i];
+    bpk = b.base[item.t0 + i];
+  };
+  auto ahead = [&]() {
+    if (i >= nt) return;
+    ci = b.idx + (bpk & kBaseMask);
+    cnt = int((uint64_t(bpk) >> kKeptShift) & kField12);  // stored (kept) entries
+    last = cnt - 1;
+    if (cnt > 0) {
+      e0 = ci[int64_t(min(c, last)) * kSlice];
+      if (NR == 1) e1 = ci[int64_t(min(c + 4, last)) * kSlice];
+    }
 #pragma unroll
-    for (int r = 0; r < NR; ++r) rval[j * NR + r] = xg[int64_t(t) * NR + r];
+    for (int r = 0; r < PER; ++r)
+#pragma unroll
+      for (int q = 0; q < NC; ++q)
+        in[r][q] = epi_in<EPI>(a, s, op + 4 * r, NR == 1 ? min(c, 2) : q, xsoa, epi, u_glob);
+  };
+  words();
+  load_tab(s_tab, a);
+  {
+    // positions, then operands: U loads in flight per thread, neighbouring
+    // threads on neighbouring words of a record
+    constexpr int U = NR == 1 ? 2 : 8;  // (eight operand sets: 4 or 8 within 2 %)
+    const uint32_t* __restrict__ slot = b.slot + r0;
+    const float4* __restrict__ pos = b.pos + r0;
+    const int nv = nrec * NR;
+    uint32_t t[U];
+    int j0 = int(threadIdx.x);
+#pragma unroll
+    for (int u = 0; u < U; ++u) t[u] = slot[min(j0 + u * kBoxThreads, nv - 1) / NR];
+    ahead();
+    while (j0 < nv) {
+      float4 f[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) f[u] = xg[int64_t(t[u]) * NR + min(j0 + u * kBoxThreads, nv - 1) % NR];
+      if constexpr (NR == 1) {
+        static_assert(U == 2);
+        const int j1 = j0 + kBoxThreads;
+        const float4 p0 = pos[j0], p1 = pos[min(j1, nv - 1)];
+        rpos[j0] = p0;
+        if (j1 < nv) rpos[j1] = p1;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (j0 + u * kBoxThreads < nv) rval[j0 + u * kBoxThreads] = f[u];
+      j0 += U * kBoxThreads;
+#pragma unroll
+      for (int u = 0; u < U; ++u) t[u] = slot[min(j0 + u * kBoxThreads, nv - 1) / NR];
+    }
+    if constexpr (NR > 1)
+      for (int j = int(threadIdx.x); j < nrec; j += kBoxThreads) rpos[j] = pos[j];
   }
   __syncthreads();
-  BoxGeom B;
-  box_init(B, a, b.reach, brick, sb);
-  const float hx = B.h[0], hy = B.h[1], hz = B.h[2];
-  constexpr int PER = NR <= 4 ? 1 : NR / 4;  // operands per lane
-  const int op = NR == 1 ? 0 : (NR == 2 ? (c & 1) : c);
-  while (i < t1) {
-    const uint16_t* __restrict__ ci = b.idx + (bpk & kBaseMask);
+  while (i < nt) {
     const float4 po = rpos[int((uint64_t(bpk) >> kSelfShift) & kField12)];  // the target's own record
     const uint32_t kb = 0x808080u - __float_as_uint(po.w);
-    const int cnt = int((uint64_t(bpk) >> kKeptShift) & kField12), last = cnt - 1;  // stored (kept) entries
     float ps[PER][3];
     KahanF kh[PER][3];
 #pragma unroll
@@ -1233,11 +1321,6 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad(PairArgs a, BoxView 
         if (!in) x = y = z = 0.f;
       };
       // two steps (eight entries) at a time, their record numbers loaded one ahead
-      uint32_t e0 = 0, e1 = 0;
-      if (cnt > 0) {
-        e0 = ci[int64_t(min(c, last)) * kSlice];
-        e1 = ci[int64_t(min(c + 4, last)) * kSlice];
-      }
       int k = 0;
       auto steps = [&](bool in0, bool in1) {
         const float4 p0 = rpos[e0], p1 = rpos[e1], f0 = rval[e0], f1 = rval[e1];
@@ -1255,10 +1338,9 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad(PairArgs a, BoxView 
       for (; k + 8 <= cnt; k += 8) steps(true, true);
       if (k < cnt) steps(k + c < cnt, k + 4 + c < cnt);
     } else {
-      uint32_t en = cnt > 0 ? ci[int64_t(min(c, last)) * kSlice] : 0u;
       for (int k = 0; k < cnt; k += 4) {
-        const int e = int(en);
-        en = ci[int64_t(min(k + 4 + c, last)) * kSlice];
+        const int e = int(e0);
+        e0 = ci[int64_t(min(k + 4 + c, last)) * kSlice];
         const Geo g = geometry(rpos[e]);
         auto entry = [&](auto M) {
           constexpr int m = decltype(M)::value;
@@ -1289,23 +1371,20 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad(PairArgs a, BoxView 
         acc[r][q] = kh[r][q].value();
       }
     if constexpr (NR == 1) {
-      quad_epilogue<EPI>(a, s, c, acc[0][0], acc[0][1], acc[0][2], xsoa, v, epi, u_glob, out, dots);
+      quad_epilogue<EPI>(a, T, in[0][0], s, c, acc[0][0], acc[0][1], acc[0][2], v, epi, out, dots);
     } else if (c < NR) {
-      const EpiTarget T = epi_target<EPI>(a, s, epi);
 #pragma unroll
       for (int r = 0; r < PER; ++r) {
         double nv[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q)
-          nv[q] = epi_component<EPI>(a, T, s, op + 4 * r, q, acc[r][q], xsoa, v, epi, u_glob, out, dots);
+          nv[q] = epi_component<EPI>(a, T, in[r][q], s, op + 4 * r, q, acc[r][q], v, epi, out, dots);
         epi_record<NR, EPI>(s, op + 4 * r, nv[0], nv[1], nv[2], v);
       }
     }
     i += kBoxThreads / 4;
-    if (i < t1) {
-      s = b.tgt[sb + i];
-      bpk = b.base[sb + i];
-    }
+    words();
+    ahead();
   }
   if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
 }
@@ -1319,34 +1398,68 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad64(PairArgs a, BoxVie
                                                              const double* __restrict__ u_glob,
                                                              double* __restrict__ out) {
   extern __shared__ double4 lds64[];
-  if (epi.skip && *epi.skip) return;  // uniform over the grid
-  const uint32_t item = b.work[block_index(a.xcd)];
-  const int64_t brick = item / kQuadShares;
-  const int64_t c0 = brick * kBrickCells;
-  const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
-  const int nt = se - sb, shares = quad_shares(nt), y = int(item % kQuadShares);
-  const int t0 = nt * y / shares, t1 = nt * (y + 1) / shares;
+  const QuadItem item = b.work[block_index(a.xcd)];
+  if ((epi.skip && *epi.skip) || item.nt <= 0) return;  // uniform over the grid (every item has targets)
+  const int nt = item.nt, nrec = int(item.rec >> kItemRecShift);
+  const int64_t r0 = item.rec & kItemRecMask;
   double dots[3] = {0.0, 0.0, 0.0};
-  const int64_t r0 = b.off[brick];
-  const int nrec = int(b.off[brick + 1] - r0);
   double4* rval = lds64;  // [nrec] operand
   const double sg = a.bsign;
   const int c = int(threadIdx.x) & 3;
-  // the first target's words are on their way while the records are staged
-  int i = t0 + (int(threadIdx.x) >> 2);
+  constexpr int U = 2;  // steps per group, the next group's tensors and record numbers loaded one ahead
+  // A target's words, its first tensors and what its epilogue reads; the
+  // first target's are on their way while the operands are staged.
+  int i = int(threadIdx.x) >> 2;
   int cnt = 0;
   int64_t base = 0;
+  double4 tn[U];
+  uint32_t en[U];
+  const EpiTarget T = epi_target<EPI>(a, item.t0, epi);  // (a brick's targets are of one system)
+  EpiIn in{};
   auto words = [&]() {
-    const int64_t s = sb + i;
+    if (i >= nt) return;
+    const int64_t s = item.t0 + i;
     cnt = a.cnt[s];
     base = a.slice_off[s >> 6] + (s & 63);
   };
-  if (i < t1) words();
-  for (int j = int(threadIdx.x); j < nrec; j += kBoxThreads) rval[j] = xg[b.slot[r0 + j]];
+  auto ahead = [&]() {
+    if (i >= nt) return;
+    if (nrec > 0 && cnt > 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t e = base + int64_t(min(4 * u + c, cnt - 1)) * kSlice;
+        en[u] = b.idx[e];
+        tn[u] = c64[e];
+      }
+    }
+    const int64_t s = item.t0 + i;
+    in = epi_in<EPI>(a, s, 0, min(c, 2), xsoa, epi, u_glob);
+  };
+  words();
+  {
+    constexpr int G = 2;  // records in flight per thread
+    const uint32_t* __restrict__ slot = b.slot + r0;
+    uint32_t t[G];
+    int j0 = int(threadIdx.x);
+    if (nrec > 0)
+#pragma unroll
+      for (int u = 0; u < G; ++u) t[u] = slot[min(j0 + u * kBoxThreads, nrec - 1)];
+    ahead();
+    while (j0 < nrec) {
+      double4 f[G];
+#pragma unroll
+      for (int u = 0; u < G; ++u) f[u] = xg[t[u]];
+#pragma unroll
+      for (int u = 0; u < G; ++u)
+        if (j0 + u * kBoxThreads < nrec) rval[j0 + u * kBoxThreads] = f[u];
+      j0 += G * kBoxThreads;
+#pragma unroll
+      for (int u = 0; u < G; ++u) t[u] = slot[min(j0 + u * kBoxThreads, nrec - 1)];
+    }
+  }
   __syncthreads();
-  constexpr int U = 2;  // steps per group, the next group's tensors and record numbers loaded one ahead
-  while (i < t1) {
-    const int64_t s = sb + i;
+  while (i < nt) {
+    const int64_t s = item.t0 + i;
     const int last = cnt - 1;
     double ps[3] = {0.0, 0.0, 0.0};
     const double4* __restrict__ cf = c64 + base;
@@ -1360,14 +1473,6 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad64(PairArgs a, BoxVie
     };
     if (nrec > 0 && cnt > 0) {
       const uint16_t* __restrict__ ci = b.idx + base;
-      double4 tn[U];
-      uint32_t en[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t e = int64_t(min(4 * u + c, last)) * kSlice;
-        en[u] = ci[e];
-        tn[u] = cf[e];
-      }
       for (int k = 0; k < cnt; k += 4 * U) {
         double4 t[U], f[U];
 #pragma unroll
@@ -1387,9 +1492,10 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad64(PairArgs a, BoxVie
         sum(cf[e], xg[a.ell[base + e] & kSlotMask], k + c < cnt);
       }
     }
-    quad_epilogue<EPI>(a, s, c, ps[0], ps[1], ps[2], xsoa, v, epi, u_glob, out, dots);
+    quad_epilogue<EPI>(a, T, in, s, c, ps[0], ps[1], ps[2], v, epi, out, dots);
     i += kBoxThreads / 4;
-    if (i < t1) words();
+    words();
+    ahead();
   }
   if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
 }
@@ -1401,7 +1507,7 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad64(PairArgs a, BoxVie
 // k_apply, so the sums are bit-identical.  A brick that is not staged
 // gathers the operands from global memory.
 template <int EPI>
-__global__ void __launch_bounds__(kBoxThreads) k_apply_box64(PairArgs a, BoxView b, const double4* __restrict__ c64,
+__global__ void __launch_bounds__(kDenseThreads) k_apply_box64(PairArgs a, BoxView b, const double4* __restrict__ c64,
                                                             const double4* __restrict__ xg,
                                                             const double* __restrict__ xsoa, SlotVec v, ChebEpi epi,
                                                             const double* __restrict__ u_glob,
@@ -1423,21 +1529,21 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box64(PairArgs a, BoxView
   if (nrec > 0) {
     // four records in flight per thread, then the remainder one at a time
     int i = int(threadIdx.x);
-    for (; i + 3 * kBoxThreads < nrec; i += 4 * kBoxThreads) {
-      const uint32_t t0 = b.slot[r0 + i], t1 = b.slot[r0 + i + kBoxThreads];
-      const uint32_t t2 = b.slot[r0 + i + 2 * kBoxThreads], t3 = b.slot[r0 + i + 3 * kBoxThreads];
+    for (; i + 3 * kDenseThreads < nrec; i += 4 * kDenseThreads) {
+      const uint32_t t0 = b.slot[r0 + i], t1 = b.slot[r0 + i + kDenseThreads];
+      const uint32_t t2 = b.slot[r0 + i + 2 * kDenseThreads], t3 = b.slot[r0 + i + 3 * kDenseThreads];
       const double4 f0 = xg[t0], f1 = xg[t1], f2 = xg[t2], f3 = xg[t3];
       rval[i] = f0;
-      rval[i + kBoxThreads] = f1;
-      rval[i + 2 * kBoxThreads] = f2;
-      rval[i + 3 * kBoxThreads] = f3;
+      rval[i + kDenseThreads] = f1;
+      rval[i + 2 * kDenseThreads] = f2;
+      rval[i + 3 * kDenseThreads] = f3;
     }
-    for (; i < nrec; i += kBoxThreads) rval[i] = xg[b.slot[r0 + i]];
+    for (; i < nrec; i += kDenseThreads) rval[i] = xg[b.slot[r0 + i]];
     __syncthreads();
   }
   const double sg = a.bsign;
-  constexpr int U = 2;  // entries per group, the next group's record numbers loaded one ahead (2 measured best of 2, 4, 8)
-  for (int i = int(threadIdx.x); i < nt; i += kBoxThreads) {
+  constexpr int U = 2;  // entries per group, the next group's tensors and record numbers loaded one ahead (4: 34.0)
+  for (int i = int(threadIdx.x); i < nt; i += kDenseThreads) {
     const int64_t s = sb + i;
     const int cnt = a.cnt[s];
     const int64_t base = a.slice_off[s >> 6] + (s & 63);
@@ -1447,26 +1553,31 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box64(PairArgs a, BoxView
       const uint16_t* __restrict__ ci = b.idx + base;
       const int last = cnt - 1;
       uint32_t en[U];
+      double4 cn[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) en[u] = ci[int64_t(min(u, last)) * kSlice];
+      for (int u = 0; u < U; ++u) {
+        en[u] = ci[int64_t(min(u, last)) * kSlice];
+        cn[u] = cf[int64_t(min(u, last)) * kSlice];
+      }
       int k = 0;
       for (; k + U <= cnt; k += U) {
-        uint32_t e[U];
         double4 c[U], f[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          e[u] = en[u];
-          en[u] = ci[int64_t(min(k + U + u, last)) * kSlice];
-          c[u] = cf[int64_t(k + u) * kSlice];
+          c[u] = cn[u];
+          f[u] = rval[en[u]];
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) f[u] = rval[e[u]];
+        for (int u = 0; u < U; ++u) {
+          en[u] = ci[int64_t(min(k + U + u, last)) * kSlice];
+          cn[u] = cf[int64_t(min(k + U + u, last)) * kSlice];
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u) fp64_acc(c[u], sg, f[u], ps[0], ps[1], ps[2]);
       }
 #pragma unroll
       for (int u = 0; u < U - 1; ++u)
-        if (k + u < cnt) fp64_acc(cf[int64_t(k + u) * kSlice], sg, rval[en[u]], ps[0], ps[1], ps[2]);
+        if (k + u < cnt) fp64_acc(cn[u], sg, rval[en[u]], ps[0], ps[1], ps[2]);
     } else if (cnt > 0) {
       const uint32_t* __restrict__ lst = a.ell + base;
       for (int k = 0; k < cnt; ++k)
@@ -1722,7 +1833,7 @@ hipError_t launch_box64(ggem_ctx* ctx, PairArgs a, const double4* xg, const doub
     hipLaunchKernelGGL((k_apply_quad64<EPI>), dim3(unsigned(ctx->quad_items)), dim3(kBoxThreads), lds, ctx->stream, a,
                        box_view(ctx), ctx->coef64, xg, soa, v, epi, u_glob, out);
   else
-    hipLaunchKernelGGL((k_apply_box64<EPI>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream, a,
+    hipLaunchKernelGGL((k_apply_box64<EPI>), dim3(n_bricks(ctx)), dim3(kDenseThreads), lds, ctx->stream, a,
                        box_view(ctx), ctx->coef64, xg, soa, v, epi, u_glob, out);
   return hipGetLastError();
 }

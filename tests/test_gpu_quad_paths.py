@@ -41,7 +41,8 @@ def pin_lists(ctx, n, prec):
     (9000, 64.0, 32, (1, 1, 1), 0, 8, G.FP32C), (10200, 64.0, 32, (1, 0, 1), 0, 2, G.FP32C),
     (4100, 48.0, 24, (1, 1, 1), 0, 7, G.FP32C), (3000, 100.0, 25, (1, 1, 1), 700, 4, G.FP32C),
     (300, 40.0, 20, (1, 1, 0), 0, 1, G.FP64), (2000, 64.0, 32, (1, 1, 1), 330, 1, G.FP64),
-    (20000, 128.0, 64, (1, 1, 1), 0, 1, G.FP64), (21500, 128.0, 64, (1, 1, 1), 0, 1, G.FP64)])
+    (20000, 128.0, 64, (1, 1, 1), 0, 1, G.FP64), (21500, 128.0, 64, (1, 1, 1), 0, 1, G.FP64),
+    (30000, 156.25, 40, (1, 1, 1), 400, 1, G.FP64)])  # bricks of about 240 targets, one over 512
 def test_staged_sums_equal_the_list_order_kernel(n, box, ne, periodic, crowd, nrhs, prec):
     dw = G.normal(nrhs * 3 * n, 31).reshape(nrhs, n, 3)
     got = []
