@@ -1766,7 +1766,8 @@ unsigned n_bricks(const ggem_ctx* ctx) { return unsigned(ctx->grid.n_cells >> (3
 //   FP64                10.9->10.3  8.3->7.3   10.6->9.8   9.6->9.8    16.6->17.0  24.3->26.3  43.9->45.7
 // and 87 -> 122 us at 1M beads (244, FP32C): there the lanes are busy either
 // way and the sums on every lane of a quad only cost.  FP64 streams its
-// tensors and gains by the split only where the blocks leave CUs idle.
+// tensors and gains by the split only where the blocks leave CUs idle (the
+// lane kernel has since gone to 34.2 us at 244 targets, quads there 37.1).
 bool quad_lanes(const ggem_ctx* ctx, int precision) {
   if (precision == GGEM_FP32C) return ctx->n <= 150 * int64_t(ctx->full_bricks);
   return ctx->n <= 40 * int64_t(ctx->full_bricks) || ctx->quad_items <= 256;
