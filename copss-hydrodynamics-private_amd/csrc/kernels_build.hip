@@ -578,9 +578,10 @@ __global__ void __launch_bounds__(kBrickThreads) k_brick_elist_count(BrickArgs a
 // record's (dj, dk) row of the stencil and differ by one in x, and the
 // matching lanes write one run of an element's list.  (A lane per element
 // that walked its rows through the global cell starts: 83 us for 69,120
-// elements and 6,400 beads in a slit; now 36 us.)  Bricks over kBoxMaxRecs
-// records walk the rows with a lane per element, in the same order; boxes
-// over the packing walk the global cell starts.
+// elements and 6,400 beads in a slit; now 36 us.  At 1M beads in 2.1M elements,
+// 244 a brick, 425 us; a lane per element over the box cells in LDS 599 us.)
+// Bricks over kBoxMaxRecs records walk the rows with a lane per element, in
+// the same order; boxes over the packing walk the global cell starts.
 __global__ void __launch_bounds__(kBrickThreads) k_brick_elist_fill(BrickArgs a, const int64_t* __restrict__ off,
                                                                     uint32_t* __restrict__ elist) {
   extern __shared__ int32_t lds[];
