@@ -1,0 +1,53 @@
+"""Calls whose route depends on what the context went through before:
+captured graphs and tuned launch shapes met again after the positions moved
+on kept lists or after a fuller build.  Each result is compared with that of
+a context without the graph or the tuner, bit for bit (the routes sum the
+same terms in the same order)."""
+import numpy as np
+import pytest
+
+import copss_ggem as G
+import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def context(n, box, ne, prec, seed=3):
+    rng = np.random.default_rng([n, ne, seed])
+    x = rng.random((n, 3)) * box
+    f = rng.normal(size=(n, 3))
+    ctx = G.Context(W._cfg([0, 0, 0], [box] * 3, [1, 1, 1], [ne] * 3, precision=prec))
+    ctx.reinit(x, f)
+    return ctx, x, f
+
+
+def moved(x, box):
+    """Every bead a third of a unit along x, wrapped into the box."""
+    y = x + np.array([0.35, 0.0, 0.0])
+    y[:, 0] -= box * (y[:, 0] >= box)
+    return y
+
+
+@pytest.mark.parametrize("prec", [G.FP32C, G.FP64])
+@pytest.mark.parametrize("nrhs", [1, 2])
+def test_graph_after_update_positions(prec, nrhs):
+    """One-unit elements: no brick's box fits the staged kernels, before and
+    after the move.  Beads that crossed a face keep lists with the shifts of
+    the build, so the step after the move takes the explicit minimum image."""
+    n, box = 400, 24.0
+    dw = G.normal(nrhs * 3 * n, 5).reshape(nrhs, n, 3)
+    got = []
+    for graph in (False, True):
+        ctx, x, f = context(n, box, 24, prec)
+        with ctx:
+            ctx.set_graph(graph)
+            steps = []
+            for _ in range(2):
+                steps.append(ctx.cheb_brownian(8, 0.02, 3.0, dw, mode=G.CHEB_FIXED)[:2])
+            ctx.update_positions(moved(x, box), f)
+            for _ in range(2):
+                steps.append(ctx.cheb_brownian(8, 0.02, 3.0, dw, mode=G.CHEB_FIXED)[:2])
+            got.append(steps)
+    for (ya, da), (yb, db) in zip(*got):
+        assert np.array_equal(ya, yb) and np.array_equal(da, db)
+    assert not np.array_equal(got[0][0][1], got[0][2][1])  # the move shows
