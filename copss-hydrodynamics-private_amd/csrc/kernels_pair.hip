@@ -1854,6 +1854,12 @@ int apply_default(const ggem_ctx* ctx, int precision, int nr) {
 int apply_candidates(const ggem_ctx* ctx, int precision, int nr) {
   return box_ready(ctx, precision, nr) ? kNApply + 1 : kNApply;
 }
+// A pick is kept by operand count and size alone: the staged shape it names
+// may not apply to the present lists (positions moved on kept lists, fuller
+// boxes); the list-order kernel serves then.
+int apply_pick(const ggem_ctx* ctx, int precision, int nr, int c) {
+  return c == kBoxShape && !box_ready(ctx, precision, nr) ? 0 : c;
+}
 
 // one apply launch in candidate shape c
 template <int P, int NR, int EPI>
@@ -1974,8 +1980,9 @@ hipError_t launch_pair_beads(ggem_ctx* ctx, int precision, int epi, const double
                                                        out);
   };
   // both epilogues write out[] only: idempotent, so the shape can be tuned here
-  const int c = tune_pick(ctx, tune_key("pair_beads", precision, epi, ctx->n), apply_candidates(ctx, precision, 1),
-                          run, apply_default(ctx, precision, 1));
+  const int c = apply_pick(ctx, precision, 1,
+                           tune_pick(ctx, tune_key("pair_beads", precision, epi, ctx->n),
+                                     apply_candidates(ctx, precision, 1), run, apply_default(ctx, precision, 1)));
   ProfScope ps(ctx, precision == GGEM_FP64 ? "pair_beads_fp64" : "pair_beads_fp32c");
   return run(c);
 }
@@ -2021,7 +2028,8 @@ hipError_t launch_apply_ref(ggem_ctx* ctx, int precision, const SlotVec& x, cons
   if (ctx->n == 0) return hipSuccess;
   const PairArgs a = make_args(ctx);
   // (the term updates y in place: the pick of plain applications serves)
-  const int c = tune_lookup(ctx, tune_key("apply", precision, 1, ctx->n), apply_default(ctx, precision, 1));
+  const int c = apply_pick(ctx, precision, 1,
+                           tune_lookup(ctx, tune_key("apply", precision, 1, ctx->n), apply_default(ctx, precision, 1)));
   ProfScope ps(ctx, precision == GGEM_FP64 ? "apply_fp64" : "apply_fp32c");
   return precision == GGEM_FP64
              ? launch_k<GGEM_FP64, 1, EPI_REF>(ctx, a, c, x.g64, x.g32, x.soa, v, epi, nullptr, nullptr)
@@ -2068,6 +2076,7 @@ hipError_t launch_apply(ggem_ctx* ctx, int precision, int nrhs, const SlotVec& x
                           [&](int c) { return run(chunks[i], c); }, dflt);
     else
       pick[i] = tune_lookup(ctx, key, dflt);
+    pick[i] = apply_pick(ctx, precision, chunks[i].nr, pick[i]);
   }
   ProfScope ps(ctx, precision == GGEM_FP64 ? "apply_fp64" : "apply_fp32c");
   for (size_t i = 0; i < chunks.size(); ++i) {

@@ -51,3 +51,46 @@ def test_graph_after_update_positions(prec, nrhs):
     for (ya, da), (yb, db) in zip(*got):
         assert np.array_equal(ya, yb) and np.array_equal(da, db)
     assert not np.array_equal(got[0][0][1], got[0][2][1])  # the move shows
+
+
+def tuned_and_plain(n, box, ne, prec, then, nrhs=1, mode=None):
+    """Steps and velocities of a context whose tuner has recorded the staged
+    kernels, and of one without a tuner, after `then` changed both."""
+    dw = G.normal(nrhs * 3 * n, 7).reshape(nrhs, n, 3)
+    got = []
+    for tune in (True, False):
+        ctx, x, f = context(n, box, ne, prec)
+        with ctx:
+            if tune:
+                ctx.set_autotune(True)
+                lg = n.bit_length() - 1
+                p = "fp32c" if prec == G.FP32C else "fp64"
+                for key in ["apply/%s/%d/%d" % (p, nr, lg) for nr in ((1, 2, 4, 8) if prec == G.FP32C else (1,))] + \
+                        ["pair_beads/%s/%d/%d" % (p, epi, lg) for epi in (0, 1)]:
+                    ctx.tune_set(key, 5)  # what the tuner records where the staged kernels win
+            run = lambda: (ctx.local_velocity_beads(), ctx.combine_velocity(),
+                           *ctx.cheb_brownian(8, 0.02, 3.0, dw, mode=G.CHEB_FIXED)[:2],
+                           *ctx.cheb_brownian(8, 0.02, 3.0, dw, mode=G.CHEB_REFERENCE)[:2])
+            run()
+            then(ctx, x, f)
+            got.append(run())
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("prec", [G.FP32C, G.FP64])
+@pytest.mark.parametrize("nrhs", [1, 3, 8])
+def test_tuned_shape_after_update_positions(prec, nrhs):
+    """The explicit minimum image has no staged kernel."""
+    tuned_and_plain(1500, 40.0, 20, prec, lambda ctx, x, f: ctx.update_positions(moved(x, 40.0), f), nrhs)
+
+
+@pytest.mark.parametrize("prec", [G.FP32C, G.FP64])
+@pytest.mark.parametrize("nrhs", [1, 2, 8])
+def test_tuned_shape_after_a_fuller_build(prec, nrhs):
+    """Beads gather in one corner: brick boxes with more records than the
+    several operands' LDS holds, some with more than are staged at all."""
+    def crowd(ctx, x, f):
+        ctx.reinit(x * np.where(np.arange(len(x)) % 8 < 6, 0.3, 1.0)[:, None], f)
+
+    tuned_and_plain(3000, 64.0, 32, prec, crowd, nrhs)
