@@ -93,10 +93,13 @@ extern "C" int ggem_local_velocity_points_noalloc(ggem_ctx* ctx, int64_t m, cons
     hipLaunchKernelGGL(k_flag_outside, dim3(unsigned((m + 255) / 256)), dim3(256), 0, ctx->stream, m, d_el, d_flag);
     GGEM_HIP(ctx, hipGetLastError());
     int32_t outside = 0;
-    if ((rc = d2h(ctx, &outside, d_flag, sizeof(int32_t)))) return rc;
+    GGEM_HIP(ctx, hipMemcpyAsync(&outside, d_flag, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+    if ((rc = sync(ctx))) return rc;
     if (outside) return fail(ctx, GGEM_ERR_OUT_OF_DOMAIN, "a point lies outside the mesh");
   }
   const hipError_t e = launch_pair_points(ctx, ctx->p.precision, m, d_pts, d_el, d_u);
   if (e != hipSuccess) return hip_fail(ctx, e, "pair_points");
-  return d2h(ctx, u, d_u, sizeof(double) * 3 * m);
+  // (not through the context's pinned buffers, which grow with the copy)
+  GGEM_HIP(ctx, hipMemcpyAsync(u, d_u, sizeof(double) * 3 * m, hipMemcpyDeviceToHost, ctx->stream));
+  return sync(ctx);
 }
