@@ -486,6 +486,9 @@ int grow_scan64(ggem_ctx* ctx, int64_t len) {
 int ggem::d2h(ggem_ctx* ctx, void* host, const void* dev, size_t bytes) {
   static_assert(kReadBufs == sizeof(ctx->read_ev) / sizeof(ctx->read_ev[0]), "an event per buffer");
   if (bytes == 0) return sync(ctx);
+  // (an event serves the streams of the device it was created on; some entry
+  // points that only read back leave the caller's current device as it is)
+  GGEM_HIP(ctx, hipSetDevice(ctx->device));
   const size_t piece = std::min(kReadMax, std::max(kReadMin, (bytes / 8 + 0xffff) & ~size_t(0xffff)));
   const size_t want = bytes <= kReadMin ? std::max(bytes, size_t(1) << 16) : piece * kReadBufs;
   if (ctx->read_cap < want) {
