@@ -1005,14 +1005,16 @@ int ggem_build_neighbors(ggem_ctx* ctx) {
   ctx->unstaged = int32_t(v[7]);
   ctx->full_bricks = int32_t(v[8]);
   ctx->quad_items = v[9];
-  if (ctx->box_recs < 0 || ctx->box_entries < 0 || ctx->ell_len < 0) {  // arrays longer than one block scans
-    const int64_t nb = ctx->grid.n_cells >> (3 * kBrickBits), nsl = (ctx->n + kSlice - 1) / kSlice;
-    int64_t w[3];
-    if ((rc = peek(ctx, {{ctx->box_off + nb, 8}, {ctx->box_eoff + nb, 8}, {ctx->slice_off + nsl, 8}}, w))) return rc;
+  // arrays longer than one block scans: their totals, and only theirs (a store
+  // without particles has no slice offsets)
+  const int64_t nb = ctx->grid.n_cells >> (3 * kBrickBits), nsl = (ctx->n + kSlice - 1) / kSlice;
+  if (ctx->box_recs < 0) {  // (records and entries are per brick both)
+    int64_t w[2];
+    if ((rc = peek(ctx, {{ctx->box_off + nb, 8}, {ctx->box_eoff + nb, 8}}, w))) return rc;
     ctx->box_recs = w[0];
     ctx->box_entries = w[1];
-    ctx->ell_len = w[2];
   }
+  if (ctx->ell_len < 0 && (rc = peek(ctx, {{ctx->slice_off + nsl, 8}}, &ctx->ell_len))) return rc;
   ctx->pairs = pairs;
   ctx->ell_valid = false;
   ctx->elem_valid = true;
