@@ -388,7 +388,8 @@ class Context:
     """One GGEM context on one HIP device (PointMesh + GGEMStokes + BrownianSystem state).
 
     Output arrays are allocated unset: a call that returns has filled them
-    (zeroing 26 MB of fresh pages first cost 0.6 ms).
+    (zeroing 26 MB of fresh pages first cost 0.6 ms).  Rows of a nodal array
+    past the mesh's nodes are zero.
 
     cfg: one workload dict, or a list of them for a batch of independent
     suspensions in one context (see BatchContext)."""
@@ -517,6 +518,13 @@ class Context:
         """Velocity mesh: elem_nodes[n_elem, 20] node numbers in HEX20 order."""
         conn = np.ascontiguousarray(elem_nodes, dtype=np.int32)
         self._c(lib().ggem_set_fe_mesh(self._h, int(n_nodes), _p(conn)))
+        self._fe_nodes = int(n_nodes)
+
+    def _nodal(self, n_nodes):
+        """Output array of n_nodes rows, those past the velocity mesh's nodes zero."""
+        F = np.empty((int(n_nodes), 3))
+        F[getattr(self, "_fe_nodes", 0):] = 0.0
+        return F
 
     def global_velocity_beads(self, node_u):
         """U_glob of every bead from the nodal velocity node_u[n_nodes, 3]."""
@@ -566,7 +574,7 @@ class Context:
     def spread_nodes(self, nqp_1d, IF, n_nodes):
         """Spreading summed into one force per node of the velocity mesh: [n_nodes, 3]."""
         IF = _f64(IF).ravel()
-        F = np.empty((int(n_nodes), 3))
+        F = self._nodal(n_nodes)
         self._c(lib().ggem_spread_nodes(self._h, nqp_1d, _p(IF), _p(F)))
         return F
 
@@ -583,7 +591,7 @@ class Context:
         mesh, periodic images condensed onto the min faces when condense
         (out=False: kept on the device)."""
         IF = None if IF is None else _f64(IF).ravel()
-        F = np.empty((int(n_nodes), 3)) if out else None
+        F = self._nodal(n_nodes) if out else None
         self._c(lib().ggem_assemble_rhs(self._h, nqp_1d, _p(IF), C.byref(opts), int(bool(condense)), _p(F)))
         return F
 

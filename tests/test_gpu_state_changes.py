@@ -94,3 +94,23 @@ def test_tuned_shape_after_a_fuller_build(prec, nrhs):
         ctx.reinit(x * np.where(np.arange(len(x)) % 8 < 6, 0.3, 1.0)[:, None], f)
 
     tuned_and_plain(3000, 64.0, 32, prec, crowd, nrhs)
+
+
+def test_nodes_past_the_mesh_are_zero():
+    """Nodal results of a longer array than the mesh's nodes end in zeros."""
+    ctx, x, f = context(200, 40.0, 20, G.FP64)
+    with ctx:
+        xyz, conn = G.hex20_box_mesh(ctx.cfg)
+        n = len(xyz)
+        ctx.set_fe_mesh(n, conn)
+        IF = G.hex20_if_table(ctx.consts().h, 2)
+        junk = np.full((n + 500, 3), 7.0)  # the allocation that the results may reuse
+        want = ctx.spread_nodes(2, IF, n)
+        del junk
+        got = ctx.spread_nodes(2, IF, n + 500)
+        assert np.array_equal(got[:n], want) and not got[n:].any()
+        want = ctx.assemble_rhs(2, IF, G.rhs_opts(), n)
+        junk = np.full((n + 500, 3), 7.0)
+        del junk
+        got = ctx.assemble_rhs(2, IF, G.rhs_opts(), n + 500)
+        assert np.array_equal(got[:n], want) and not got[n:].any()
