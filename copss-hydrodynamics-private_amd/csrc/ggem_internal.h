@@ -477,9 +477,8 @@ hipError_t launch_fix_forces(ggem_ctx* ctx, int32_t chain, double k, double b, i
 
 // ---- launchers (kernels_pair.hip) ----
 // A vector operand of the pair sum: FP64 SoA by slot for the element-wise
-// algebra plus a one-record-per-slot copy for the neighbour gathers.  Of
-// several operands, each launch's (apply_chunk) lie together by slot, record
-// (s, r) of nr at s nr + r: a neighbour is one run of memory.
+// algebra plus a one-record-per-slot copy for the neighbour gathers, the
+// records of one launch's (apply_chunk) nr operands at gather_index.
 struct SlotVec {
   double* soa;    // [3][n]
   float4* g32;    // [n]
@@ -487,6 +486,19 @@ struct SlotVec {
 };
 
 // Epilogue of the pair sum, per target slot s with sum m_s = sum_t G f_t:
+// Record of slot s, operand r of nr: together by slot, a neighbour being one
+// run of memory; but FP64's four and more in a plane each.  Those are read by
+// the list-order kernel alone, whose neighbouring lanes read neighbouring
+// slots more often than not: a load of 64 records of 32 bytes then touches 21
+// to 24 lines of 128 bytes, and together by slot 30 to 35.  Eight vectors
+// FP64, together by slot -> in planes, us per application: 2,000 beads (200 a
+// brick) 85 -> 62, 10,000 beads 89 -> 67, 50,000 beads 95 -> 83; two vectors
+// are faster by slot, 10,000 beads 25 against 28.
+__host__ __device__ constexpr bool gather_planes(bool fp64, int nr) { return fp64 && nr >= 4; }
+__host__ __device__ constexpr int64_t gather_index(bool fp64, int nr, int64_t n, int64_t s, int r) {
+  return gather_planes(fp64, nr) ? r * n + s : s * nr + r;
+}
+
 enum Epi : int {
   EPI_LOCAL = 0,     // out[3p+c] = U_loc  (p = particle id, interleaved)
   EPI_MOBILITY = 1,  // out[3p+c] = U_glob + U_loc - coeff_1 f + f (type rules)

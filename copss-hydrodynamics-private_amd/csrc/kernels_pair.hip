@@ -338,11 +338,11 @@ __device__ __forceinline__ double epi_component(const PairArgs& a, const EpiTarg
 }
 // gather record of the new vector, operand r of NR
 template <int NR, int EPI>
-__device__ __forceinline__ void epi_record(int64_t s, int r, double x, double y, double z,
+__device__ __forceinline__ void epi_record(int64_t n, int64_t s, int r, double x, double y, double z,
                                            const SlotVec& v) {
   if constexpr (EPI == EPI_CHEB || EPI == EPI_REF) {
-    if (v.g32) v.g32[s * NR + r] = make_float4(float(x), float(y), float(z), 0.f);
-    if (v.g64) v.g64[s * NR + r] = make_double4(x, y, z, 0.0);
+    if (v.g32) v.g32[gather_index(false, NR, n, s, r)] = make_float4(float(x), float(y), float(z), 0.f);
+    if (v.g64) v.g64[gather_index(true, NR, n, s, r)] = make_double4(x, y, z, 0.0);
   }
 }
 
@@ -360,7 +360,7 @@ __device__ __forceinline__ void apply_epilogue(const PairArgs& a, int64_t s, con
     for (int q = 0; q < 3; ++q)
       nv[q] = epi_component<EPI>(a, T, epi_in<EPI>(a, s, r, q, xsoa, epi, u_glob), s, r, q, acc[r][q], v, epi, out,
                                  dots);
-    epi_record<NR, EPI>(s, r, nv[0], nv[1], nv[2], v);
+    epi_record<NR, EPI>(a.n, s, r, nv[0], nv[1], nv[2], v);
   }
 }
 
@@ -396,7 +396,7 @@ __device__ __forceinline__ void quad_epilogue(const PairArgs& a, const EpiTarget
   double nv = 0.0;
   if (c < 3) nv = epi_component<EPI>(a, T, I, s, 0, c, c == 0 ? m0 : (c == 1 ? m1 : m2), v, epi, out, dots);
   const double x = quad_get<0>(nv), y = quad_get<1>(nv), z = quad_get<2>(nv);
-  if (c == 0) epi_record<1, EPI>(s, 0, x, y, z, v);
+  if (c == 0) epi_record<1, EPI>(a.n, s, 0, x, y, z, v);
 }
 
 // the block's sums of three values, on every thread (one barrier pair)
@@ -550,7 +550,7 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
 #pragma unroll
       for (int i = 0; i < U; ++i)
 #pragma unroll
-        for (int r = 0; r < NR; ++r) f[i][r] = xg[int64_t(e[i] & kSlotMask) * NR + r];
+        for (int r = 0; r < NR; ++r) f[i][r] = xg[gather_index(true, NR, a.n, e[i] & kSlotMask, r)];
 #pragma unroll
       for (int i = 0; i < U; ++i) pair_acc(c[i], f[i]);
     }
@@ -559,7 +559,7 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
       if (k + i < cnt) {  // entries en[0 .. cnt - k)
         double4 f[NR];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) f[r] = xg[int64_t(en[i] & kSlotMask) * NR + r];
+        for (int r = 0; r < NR; ++r) f[r] = xg[gather_index(true, NR, a.n, en[i] & kSlotMask, r)];
         pair_acc(cf[int64_t(k + i) * kSlice], f);
       }
     }
@@ -656,7 +656,7 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
         const uint32_t t = c[i] & kSlotMask;
         pt[i] = pc[t];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) f[i][r] = xg[int64_t(t) * NR + r];
+        for (int r = 0; r < NR; ++r) f[i][r] = xg[gather_index(false, NR, a.n, t, r)];
       }
 #pragma unroll
       for (int i = 0; i < U; ++i) pair_acc(c[i], pt[i], f[i]);
@@ -667,7 +667,7 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
         const uint32_t t = en[i] & kSlotMask;
         float4 f[NR];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) f[r] = xg[int64_t(t) * NR + r];
+        for (int r = 0; r < NR; ++r) f[r] = xg[gather_index(false, NR, a.n, t, r)];
         pair_acc(en[i], pc[t], f);
       }
     }
@@ -1379,7 +1379,7 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad(PairArgs a, BoxView 
 #pragma unroll
         for (int q = 0; q < 3; ++q)
           nv[q] = epi_component<EPI>(a, T, in[r][q], s, op + 4 * r, q, acc[r][q], v, epi, out, dots);
-        epi_record<NR, EPI>(s, op + 4 * r, nv[0], nv[1], nv[2], v);
+        epi_record<NR, EPI>(a.n, s, op + 4 * r, nv[0], nv[1], nv[2], v);
       }
     }
     i += kBoxThreads / 4;

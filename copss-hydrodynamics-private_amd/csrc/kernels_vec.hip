@@ -44,8 +44,8 @@ __global__ void k_make_gather(int64_t n, int nrhs, const double* __restrict__ so
   if (s >= n) return;
   for (int r = 0; r < nrhs; ++r) {
     const double x = soa[r * 3 * n + s], y = soa[r * 3 * n + n + s], z = soa[r * 3 * n + 2 * n + s];
-    if (g32) g32[s * nrhs + r] = make_float4(float(x), float(y), float(z), 0.f);
-    if (g64) g64[s * nrhs + r] = make_double4(x, y, z, 0.0);
+    if (g32) g32[gather_index(false, nrhs, n, s, r)] = make_float4(float(x), float(y), float(z), 0.f);
+    if (g64) g64[gather_index(true, nrhs, n, s, r)] = make_double4(x, y, z, 0.0);
   }
 }
 

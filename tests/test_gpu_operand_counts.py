@@ -1,0 +1,57 @@
+"""Several noise vectors at once, in every launch size they split into (8, 4,
+2, 1) and both layouts of the gather records: each vector's step is what it
+is alone, bit for bit.  With the staged kernels, with bricks that are not
+staged, under the explicit minimum image, through graph replay, and with the
+kept vectors applied again after a rebuild."""
+import numpy as np
+import pytest
+
+import copss_ggem as G
+import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+N, BOX = 1100, 48.0
+
+
+def context(prec, state):
+    rng = np.random.default_rng(17)
+    x = rng.random((N, 3)) * BOX
+    if state == "crowded":
+        x[:500] = 4.0 + rng.random((500, 3)) * 6.0
+    if state == "unstaged":  # a box over the staged records, and lists of hundreds
+        x[:] = 20.0 + rng.random((N, 3)) * 8.0
+        x = np.concatenate([x, x[:, ::-1] + 0.125])
+    f = rng.normal(size=x.shape)
+    ctx = G.Context(W._cfg([0, 0, 0], [BOX] * 3, [1, 1, 0], [24, 24, 24], precision=prec))
+    ctx.reinit(x, f)
+    if state == "moved":
+        ctx.update_positions(np.where(np.arange(3) == 0, (x + 0.7) % BOX, x), f)
+    return ctx, x, f
+
+
+@pytest.mark.parametrize("prec", [G.FP64, G.FP32C])
+@pytest.mark.parametrize("state", ["plain", "crowded", "unstaged", "moved"])
+@pytest.mark.parametrize("nrhs", [2, 3, 4, 7, 8, 13, 16])
+def test_vectors_together_equal_vectors_alone(prec, state, nrhs):
+    ctx, x, f = context(prec, state)
+    with ctx:
+        dw = G.normal(nrhs * x.size, 23).reshape(nrhs, -1, 3)
+        step = lambda w: ctx.cheb_brownian(5, 0.02, 30.0, w, mode=G.CHEB_FIXED, keep=True)[:2]
+        alone = [step(w[None]) for w in dw]
+        y, d = step(dw)
+        for r in range(nrhs):
+            assert np.array_equal(y[r], alone[r][0][0]) and np.array_equal(d[r], alone[r][1][0]), r
+        assert np.array_equal(ctx.displacement_apply(), d)
+        ctx.set_graph(True)
+        for _ in range(3):
+            yg, dg = step(dw)
+            assert np.array_equal(yg, y) and np.array_equal(dg, d)
+        ctx.set_graph(False)
+        if state != "moved":  # the kept vectors at other positions, against each alone there
+            x2 = np.where(np.arange(3) == 1, (x + 0.9) % BOX, x)
+            ctx.reinit(x2, f)
+            d2 = ctx.displacement_apply()
+            for r in (0, nrhs - 1):
+                ctx.set_forces(y[r])
+                assert np.array_equal(d2[r], ctx.mobility_apply(None)), r
