@@ -1159,7 +1159,8 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_box(PairArgs a, BoxView b
 }
 
 
-// The staged pair sum with four lanes (a quad) per target, for NR operands.
+// The staged pair sum with four lanes (a quad) per target, for NR operands
+// (in which bricks: quad_lanes).
 // One operand: lane c takes entries c, c + 4, ...; the four terms of a step
 // are added in list order by every lane (quad_add).  Several operands: lane c
 // forms the displacement and the tensor of its entry, then the quad goes
@@ -1387,6 +1388,114 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad(PairArgs a, BoxView 
     ahead();
   }
   if constexpr (EPI == EPI_REF) ref_finish(epi, dots);
+}
+
+// k_apply_box for NR = 2 and 4 operands, for dense bricks (quad_lanes): a lane
+// per target, the box's positions and the operands' records in LDS, a plane
+// per operand ([NR][nrec]: the lanes of a wave read one operand of records at
+// random, which a plane spreads over all banks), each kept pair's tensor
+// formed once for all NR.  Sums, merge points and epilogue are k_apply's for
+// NR operands, bit for bit.  Every brick with targets is staged.
+template <int EPI, bool ONE, int NR>
+__global__ void __launch_bounds__(kBoxThreads) k_apply_box_nr(PairArgs a, BoxView b, const float4* __restrict__ xg,
+                                                             const double* __restrict__ xsoa, SlotVec v, ChebEpi epi,
+                                                             const double* __restrict__ u_glob,
+                                                             double* __restrict__ out) {
+  static_assert(NR > 1 && EPI != EPI_REF, "one operand: k_apply_box");
+  extern __shared__ float4 lds[];
+  if (epi.skip && *epi.skip) return;  // uniform over the grid
+  const int64_t brick = block_index(a.xcd);
+  const int64_t c0 = brick * kBrickCells;
+  const int32_t sb = b.cs[c0], se = b.cs[c0 + kBrickCells];
+  if (sb >= se) return;  // no targets (uniform over the block)
+  const int64_t r0 = b.off[brick];
+  const int nrec = int(b.off[brick + 1] - r0);
+  const int nt = se - sb;
+  if (nrec == 0) return;  // not staged: never launched so (uniform over the block)
+  float4* s_tab = lds;                       // coefficient table
+  float4* rpos = lds + kTabStride * a.ct.n;  // [nrec] offset xyz, packed box cell
+  float4* rval = rpos + nrec;                // [NR][nrec] operands
+  load_tab(s_tab, a);
+  for (int i = int(threadIdx.x); i < nrec; i += kBoxThreads) {
+    const uint32_t t = b.slot[r0 + i];
+    rpos[i] = b.pos[r0 + i];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) rval[r * nrec + i] = xg[gather_index(false, NR, a.n, t, r)];
+  }
+  __syncthreads();
+  BoxGeom B;
+  box_init(B, a, b.reach, brick, sb);
+  const float hx = B.h[0], hy = B.h[1], hz = B.h[2];
+  constexpr int U = 2;  // entries per group, the next group's record numbers loaded one ahead
+  for (int i = int(threadIdx.x); i < nt; i += kBoxThreads) {
+    const int64_t s = b.tgt[sb + i];
+    const int64_t bpk = b.base[sb + i];
+    const float4 po = rpos[int((uint64_t(bpk) >> kSelfShift) & kField12)];  // the target's own record
+    const uint32_t kb = 0x808080u - __float_as_uint(po.w);
+    const int cnt = int((uint64_t(bpk) >> kKeptShift) & kField12);  // stored (kept) entries
+    float ps[NR][3];
+    KahanF kh[NR][3];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) ps[r][0] = ps[r][1] = ps[r][2] = 0.f;
+    auto disp = [&](const float4& pt, float& dx, float& dy, float& dz, float& y) {
+      float di, dj, dk;
+      box_diff(__float_as_uint(pt.w), kb, di, dj, dk);
+      dx = __builtin_fmaf(di, hx, pt.x - po.x);
+      dy = __builtin_fmaf(dj, hy, pt.y - po.y);
+      dz = __builtin_fmaf(dk, hz, pt.z - po.z);
+      return ONE ? fp32c_interval1(a.ct, fp32c_r2(dx, dy, dz), y) : fp32c_interval(a.ct, fp32c_r2(dx, dy, dz), y);
+    };
+    auto add = [&](int it, float y, float dx, float dy, float dz, const float4* f, int k) {
+      float A, Bx;
+      fp32c_eval(s_tab, it, y, A, Bx);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) fp32c_acc(A, Bx, dx, dy, dz, f[r].x, f[r].y, f[r].z, ps[r][0], ps[r][1], ps[r][2]);
+      if ((k & (kMergeEvery - 1)) == kMergeEvery - 1) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            kh[r][q].add(ps[r][q]);
+            ps[r][q] = 0.f;
+          }
+      }
+    };
+    if (cnt > 0) {  // an empty list has no storage
+      const uint16_t* __restrict__ ci = b.idx + (bpk & kBaseMask);
+      const int last = cnt - 1;
+      uint32_t en[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) en[u] = ci[int64_t(min(u, last)) * kSlice];
+      for (int k = 0; k < cnt; k += U) {
+        float4 pt[U], f[U][NR];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const uint32_t c = en[u];
+          en[u] = ci[int64_t(min(k + U + u, last)) * kSlice];
+          pt[u] = rpos[c];
+#pragma unroll
+          for (int r = 0; r < NR; ++r) f[u][r] = rval[r * nrec + c];
+        }
+        float dx[U], dy[U], dz[U], y[U];
+        int it[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) it[u] = disp(pt[u], dx[u], dy[u], dz[u], y[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (u == 0 || k + u < cnt) add(it[u], y[u], dx[u], dy[u], dz[u], f[u], k + u);
+      }
+    }
+    double acc[NR][3];
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        kh[r][q].add(ps[r][q]);
+        acc[r][q] = kh[r][q].value();
+      }
+    double dots[3];  // (EPI_REF only)
+    apply_epilogue<NR, EPI>(a, s, acc, xsoa, v, epi, u_glob, out, dots);
+  }
 }
 
 // k_apply_box64 (below) with four lanes per target: lane c takes entries c,
@@ -1768,9 +1877,31 @@ unsigned n_bricks(const ggem_ctx* ctx) { return unsigned(ctx->grid.n_cells >> (3
 // way and the sums on every lane of a quad only cost.  FP64 streams its
 // tensors and gains by the split only where the blocks leave CUs idle (the
 // lane kernel has since gone to 34.2 us at 244 targets, quads there 37.1).
-bool quad_lanes(const ggem_ctx* ctx, int precision) {
-  if (precision == GGEM_FP32C) return ctx->n <= 150 * int64_t(ctx->full_bricks);
-  return ctx->n <= 40 * int64_t(ctx->full_bricks) || ctx->quad_items <= 256;
+// FP32C with several operands, quads -> one lane (k_apply_box_nr; 8 as 4 + 4;
+// * as 2 + 2, the records of 4 exceed the LDS), us per application:
+//   beads    targets   2 operands      4 operands      8 operands
+//   25,000     49      11.8 -> 14.6    13.3 -> 19.4    18.5 -> 36.9
+//             200      14.4 -> 17.4    17.3 -> 23.0    32.1 -> 43.7
+//   50,000     98      14.8 -> 15.8    17.7 -> 21.6    33.1 -> 41.9
+//             146      18.3 -> 19.5    29.6 -> 27.8    56.4 -> 53.5
+//             231      42.3 -> 34.8    82.5 -> 67.1*   161 -> 132*
+//   65,536     49      17.8 -> 16.6    21.9 -> 32.0    33.4 -> 61.3
+//              90      18.2 -> 16.2    23.2 -> 22.4    43.4 -> 42.0
+//             191      23.8 -> 20.1    39.1 -> 27.8    76.2 -> 53.1
+//   100,000    58      22.9 -> 21.2    27.8 -> 39.6    64.3 -> 76.2
+//             100      22.5 -> 18.2    28.4 -> 26.4    58.9 -> 49.9
+//             195      28.7 -> 21.6    52.2 -> 30.4    102 -> 57.1
+//             292      64.9 -> 42.2    127 -> 80.8*    252 -> 160*
+// A quad block stages its brick's records for about 64 targets, a lane block
+// for all of them: quads lose where bricks use the threads of a lane block (45
+// targets at two operands, 95 at four) and the lanes fill the chip (beads, or
+// beads times targets a brick where the staging decides).
+bool quad_lanes(const ggem_ctx* ctx, int precision, int nr) {
+  const int64_t n = ctx->n, b = ctx->full_bricks;
+  if (nr == 2) return n < 45 * b || (n < 65536 && n * n < 10000000 * b);
+  if (nr > 2) return n < 95 * b || n * n < 6200000 * b;
+  if (precision == GGEM_FP32C) return n <= 150 * b;
+  return n <= 40 * b || ctx->quad_items <= 256;
 }
 
 size_t box_lds(const ggem_ctx* ctx, int nr) {
@@ -1796,7 +1927,7 @@ hipError_t launch_box(ggem_ctx* ctx, PairArgs a, const float4* xg, const double*
   if (!ctx->box_valid || ctx->box_fp64 || ctx->box_max <= 0 || ctx->box_max > kBoxMaxRecs)
     return hipErrorInvalidConfiguration;
   a.xcd = 1;
-  if (quad_lanes(ctx, GGEM_FP32C)) return launch_quad<EPI, 1>(ctx, a, xg, soa, v, epi, u_glob, out);
+  if (quad_lanes(ctx, GGEM_FP32C, 1)) return launch_quad<EPI, 1>(ctx, a, xg, soa, v, epi, u_glob, out);
   const size_t lds = box_lds(ctx, 1);
   if (ctx->tab.n2 == 0)
     hipLaunchKernelGGL((k_apply_box<EPI, true>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream, a,
@@ -1820,6 +1951,17 @@ hipError_t launch_box_nr(ggem_ctx* ctx, PairArgs a, const float4* xg, const doub
                          const ChebEpi& epi, const double* u_glob, double* out) {
   if (!box_nr_ready(ctx, NR)) return hipErrorInvalidConfiguration;
   a.xcd = 1;
+  if constexpr (NR <= 4)
+    if (!quad_lanes(ctx, GGEM_FP32C, NR)) {
+      const size_t lds = box_lds(ctx, NR);
+      if (ctx->tab.n2 == 0)
+        hipLaunchKernelGGL((k_apply_box_nr<EPI, true, NR>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream,
+                           a, box_view(ctx), xg, soa, v, epi, u_glob, out);
+      else
+        hipLaunchKernelGGL((k_apply_box_nr<EPI, false, NR>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds,
+                           ctx->stream, a, box_view(ctx), xg, soa, v, epi, u_glob, out);
+      return hipGetLastError();
+    }
   return launch_quad<EPI, NR>(ctx, a, xg, soa, v, epi, u_glob, out);
 }
 
@@ -1830,7 +1972,7 @@ hipError_t launch_box64(ggem_ctx* ctx, PairArgs a, const double4* xg, const doub
     return hipErrorInvalidConfiguration;
   a.xcd = 1;
   const size_t lds = size_t(ctx->box_max) * sizeof(double4);
-  if (quad_lanes(ctx, GGEM_FP64))
+  if (quad_lanes(ctx, GGEM_FP64, 1))
     hipLaunchKernelGGL((k_apply_quad64<EPI>), dim3(unsigned(ctx->quad_items)), dim3(kBoxThreads), lds, ctx->stream, a,
                        box_view(ctx), ctx->coef64, xg, soa, v, epi, u_glob, out);
   else
@@ -2006,11 +2148,12 @@ int64_t apply_ref_blocks(const ggem_ctx* ctx) {
 }
 
 // operands of the next launch of `left`: the largest power of two up to 8,
-// halved while only a smaller one fits the staged kernel's LDS
+// halved while only a smaller one fits the staged kernel's LDS, and 4 at once
+// where a lane per target sums them (quad_lanes)
 int apply_chunk(const ggem_ctx* ctx, int precision, int left) {
   int nr = left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1;
   if (precision == GGEM_FP32C)
-    for (int m = nr; m > 1; m /= 2)
+    for (int m = nr == 8 && !quad_lanes(ctx, precision, nr) ? 4 : nr; m > 1; m /= 2)
       if (box_nr_ready(ctx, m)) return m;
   return nr;
 }

@@ -55,3 +55,27 @@ def test_vectors_together_equal_vectors_alone(prec, state, nrhs):
             for r in (0, nrhs - 1):
                 ctx.set_forces(y[r])
                 assert np.array_equal(d2[r], ctx.mobility_apply(None)), r
+
+
+# 70,000 beads: 70, 137 and 137 beads a brick, the last with remainders of the
+# 8-cell bricks and walls; two, four and eight vectors a lane per target
+@pytest.mark.parametrize("box,ne,periodic,nrhs", [
+    (240.0, 80, (1, 1, 1), 3), (249.6, 64, (1, 1, 1), 4), (249.6, 64, (1, 1, 1), 16), (241.8, 62, (1, 0, 1), 11)])
+def test_dense_bricks_equal_the_list_order_kernel(box, ne, periodic, nrhs):
+    n = 70000
+    rng = np.random.default_rng(ne)
+    x, f = rng.random((n, 3)) * box, rng.normal(size=(n, 3))
+    dw = G.normal(nrhs * 3 * n, 29).reshape(nrhs, n, 3)
+    got = []
+    for lists in (False, True):
+        with G.Context(W._cfg([0, 0, 0], [box] * 3, periodic, [ne] * 3, precision=G.FP32C)) as ctx:
+            ctx.reinit(x, f)
+            if lists:
+                for nr in (1, 2, 4, 8):
+                    ctx.tune_set("apply/fp32c/%d/16" % nr, 0)
+                ctx.set_autotune(True)
+            got.append(ctx.cheb_brownian(3, 0.02, 3.0, dw, mode=G.CHEB_FIXED)[:2])
+            ctx.set_graph(True)
+            got.append(ctx.cheb_brownian(3, 0.02, 3.0, dw, mode=G.CHEB_FIXED)[:2])
+    for y, d in got[1:]:
+        assert np.array_equal(y, got[0][0]) and np.array_equal(d, got[0][1])
