@@ -435,8 +435,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 // Walk the particle slots of every element of the stencil of element
 // (ci, cj, ck): calls seg(a, b, code) for each contiguous slot range [a, b)
 // with the periodic shift code of that range (a row's x-run is one range
-// per brick it crosses), rows in stencil order, x ascending within a row;
-// rows r0, r0 + step, ... where several lanes share a walk.
+// per brick it crosses), in the records' order of a staged box: rows in
+// stencil order, x ascending within a row through both faces; rows r0, r0 +
+// step, ... where several lanes share a walk.
 template <class Seg>
 __device__ __forceinline__ void for_each_segment(const Grid& g, const StencilRow* __restrict__ rows,
                                                  int nrows, const int32_t* __restrict__ cell_start,
@@ -479,21 +480,10 @@ __device__ __forceinline__ void for_each_segment(const Grid& g, const StencilRow
         p = q + 1;
       }
     };
-    int lo = ci + R.di_lo, hi = ci + R.di_hi;
-    if (g.periodic[0]) {
-      if (lo < 0) {
-        run(lo + nx, nx - 1, cyz | 2u);
-        lo = 0;
-      }
-      if (hi >= nx) {
-        run(0, hi - nx, cyz | 1u);
-        hi = nx - 1;
-      }
-    } else {
-      lo = lo < 0 ? 0 : lo;
-      hi = hi >= nx ? nx - 1 : hi;
-    }
-    if (lo <= hi) run(lo, hi, cyz);
+    const int lo = ci + R.di_lo, hi = ci + R.di_hi;
+    if (g.periodic[0] && lo < 0) run(lo + nx, nx - 1, cyz | 2u);
+    if (max(lo, 0) <= min(hi, nx - 1)) run(max(lo, 0), min(hi, nx - 1), cyz);
+    if (g.periodic[0] && hi >= nx) run(0, hi - nx, cyz | 1u);
   }
 }
 

@@ -576,10 +576,9 @@ __global__ void __launch_bounds__(kBrickThreads) k_brick_elist_count(BrickArgs a
 // The element lists, a wave per x-row of eight elements of a brick over the
 // records of the z layers in reach, 64 at a time: the eight elements share a
 // record's (dj, dk) row of the stencil and differ by one in x, and the
-// matching lanes write one run of an element's list.  (A lane per element
-// that walked its rows through the global cell starts: 83 us for 69,120
-// elements and 6,400 beads in a slit; now 36 us.  At 1M beads in 2.1M elements,
-// 244 a brick, 425 us; a lane per element over the box cells in LDS 599 us.)
+// matching lanes write one run of an element's list.  (69,120 elements and
+// 6,400 beads in a slit: 36 us, with k_elist_fill's lane per element 83 us;
+// launch_elist_fill says which where.)
 // Bricks over kBoxMaxRecs records walk the rows with a lane per element, in
 // the same order; boxes over the packing walk the global cell starts.
 __global__ void __launch_bounds__(kBrickThreads) k_brick_elist_fill(BrickArgs a, const int64_t* __restrict__ off,
@@ -659,6 +658,37 @@ __global__ void __launch_bounds__(kBrickThreads) k_brick_elist_fill(BrickArgs a,
       }
     }
   }
+}
+
+// The element lists, a lane per element walking its stencil rows through the
+// global cell starts: the lists of a block's consecutive elements form one
+// output range, which is assembled in LDS and written with whole lines (direct
+// stores when it exceeds the buffer).
+constexpr int kElistLds = 10240;
+__global__ void __launch_bounds__(kBlock) k_elist_fill(Grid g, const StencilRow* __restrict__ rows, int nrows,
+                                                      const int32_t* __restrict__ cell_start,
+                                                      const int64_t* __restrict__ off,
+                                                      uint32_t* __restrict__ elist) {
+  __shared__ uint32_t buf[kElistLds];
+  const int64_t e0 = int64_t(blockIdx.x) * kBlock, e_end = min(e0 + int64_t(kBlock), g.n_elem);
+  const int64_t base = off[e0], total = off[e_end] - base;
+  const bool fits = total <= kElistLds;  // uniform over the block
+  const int64_t e = e0 + threadIdx.x;
+  if (e < g.n_elem) {
+    int ci, cj, ck;
+    elem_ijk(g, e, ci, cj, ck);
+    int64_t k = off[e] - base;
+    for_each_segment(g, rows, nrows, cell_start, ci, cj, ck, [&](int32_t a, int32_t b, uint32_t code) {
+      const uint32_t hi = code << kSlotBits;
+      for (int32_t t = a; t < b; ++t, ++k) {
+        if (fits) buf[k] = uint32_t(t) | hi;
+        else elist[base + k] = uint32_t(t) | hi;
+      }
+    });
+  }
+  if (!fits) return;
+  __syncthreads();
+  for (int64_t i = threadIdx.x; i < total; i += kBlock) elist[base + i] = buf[i];
 }
 
 // Exclusive scan of int64 values (three phases, as the int32 scan).
@@ -1236,11 +1266,32 @@ hipError_t launch_elist_count(ggem_ctx* ctx) {
 
 hipError_t launch_elist_fill(ggem_ctx* ctx) {
   ProfScope ps(ctx, "elist_fill");
+  // A lane per element or a wave per eight (k_brick_elist_fill), by the beads
+  // of a brick for each stencil row: a wave reads its z layers' records for
+  // eight elements' rows, a lane its rows alone, and lanes win where rows are
+  // few or hold many beads, if there are elements enough.  Wave -> lane, us:
+  //   rows (element)  beads a brick    700 bricks and more  340 to 512  125 and fewer
+  //   69 (2.0)            45           89 -> 189            -           36 -> 92
+  //   29 (3.1)            39           65 -> 86             56 -> 50    27 -> 39
+  //   21 (3.9)            80           102 -> 125           43 -> 44    23 -> 34
+  //   21 (3.9)           175 to 200    93 -> 86             56 -> 47    28 -> 43
+  //   21 (3.9)           244           499 -> 371 (4,096)   97 -> 57    37 -> 45
+  //   13 (5.0)           200           93 -> 46             -           29 -> 23
+  //    9 (6.0)           500           -                    51 -> 29    27 -> 25
+  const unsigned nb = brick_count(ctx);
+  if (ctx->n_rows <= 16 || (nb >= 256 && ctx->n > 8 * int64_t(ctx->n_rows) * nb)) {
+    hipLaunchKernelGGL(k_elist_fill, dim3(blocks_for(ctx->grid.n_elem)), dim3(kBlock), 0, ctx->stream, ctx->grid,
+                       ctx->rows_d, ctx->n_rows, ctx->cell_start, ctx->elist_off, ctx->elist);
+    return hipGetLastError();
+  }
   const BrickArgs a = brick_args(ctx);
   const size_t lds =
       sizeof(int32_t) * (2 * size_t(a.cells_cap) + 1 + 2 * size_t(kBoxMaxRecs)) + sizeof(uint16_t) * kStencilTab;
-  // few bricks: several blocks each, to reach every CU
-  const unsigned nb = brick_count(ctx), split = nb >= 512 ? 1u : nb >= 256 ? 2u : 4u;
+  // few bricks: several blocks each, to reach every CU (of 512 to 1,023
+  // bricks two where the walk outweighs a second staging: 80 beads a brick
+  // and 29 rows 70 -> 58 us, 10 beads and 69 rows 44 -> 59)
+  const bool one = nb >= 1024 || (nb >= 512 && 2 * ctx->n < 3 * int64_t(ctx->n_rows) * nb);
+  const unsigned split = one ? 1u : nb >= 256 ? 2u : 4u;
   hipLaunchKernelGGL(k_brick_elist_fill, dim3(nb, split), dim3(kBrickThreads), lds, ctx->stream, a, ctx->elist_off,
                      ctx->elist);
   return hipGetLastError();
