@@ -387,6 +387,7 @@ void free_all(ggem_ctx* ctx) {
   f(ctx->box_cnt);
   f(ctx->box_tgt);
   f(ctx->quad_work);
+  f(ctx->size_tiles);
   f(ctx->box_base);
   f(ctx->box_slot);
   f(ctx->box_pos);
@@ -915,6 +916,7 @@ int ensure_build(ggem_ctx* ctx) {
   if (!rc) rc = ensure(ctx, &ctx->box_tgt, &ctx->box_tgt_cap, size_t(std::max<int64_t>(ctx->n, 1)));
   // (a brick's shares are at most one more than its 64ths of the targets)
   if (!rc) rc = ensure(ctx, &ctx->quad_work, &ctx->quad_work_cap, size_t(ctx->n / 64) + nb + 1);
+  if (!rc && size_tile_bytes(ctx) > 0) rc = ensure(ctx, &ctx->size_tiles, &ctx->size_tiles_cap, size_tile_bytes(ctx));
   return rc;
 }
 
@@ -1005,16 +1007,9 @@ int ggem_build_neighbors(ggem_ctx* ctx) {
   ctx->unstaged = int32_t(v[7]);
   ctx->full_bricks = int32_t(v[8]);
   ctx->quad_items = v[9];
-  // arrays longer than one block scans: their totals, and only theirs (a store
-  // without particles has no slice offsets)
-  const int64_t nb = ctx->grid.n_cells >> (3 * kBrickBits), nsl = (ctx->n + kSlice - 1) / kSlice;
-  if (ctx->box_recs < 0) {  // (records and entries are per brick both)
-    int64_t w[2];
-    if ((rc = peek(ctx, {{ctx->box_off + nb, 8}, {ctx->box_eoff + nb, 8}}, w))) return rc;
-    ctx->box_recs = w[0];
-    ctx->box_entries = w[1];
-  }
-  if (ctx->ell_len < 0 && (rc = peek(ctx, {{ctx->slice_off + nsl, 8}}, &ctx->ell_len))) return rc;
+  // (more slices than one block scans)
+  if (ctx->ell_len < 0 && (rc = peek(ctx, {{ctx->slice_off + (ctx->n + kSlice - 1) / kSlice, 8}}, &ctx->ell_len)))
+    return rc;
   ctx->pairs = pairs;
   ctx->ell_valid = false;
   ctx->elem_valid = true;

@@ -243,6 +243,8 @@ struct ggem_ctx {
   ggem::QuadItem* quad_work = nullptr;  // [quad_items] what every block of the quad pair sums takes
   size_t quad_work_cap = 0;
   int64_t quad_items = 0;
+  unsigned char* size_tiles = nullptr;  // the sizes' tile totals (meshes of many bricks)
+  size_t size_tiles_cap = 0;
   uint8_t* spread_unstaged = nullptr;  // [bricks] the brick spreading's boxes over its record table
   size_t spread_unstaged_cap = 0;
   int32_t box_max = 0;            // same on the host; 0 when no brick is staged
@@ -436,10 +438,11 @@ hipError_t launch_clear_counters(ggem_ctx* ctx);
 hipError_t launch_count_lists(ggem_ctx* ctx);
 // record, entry and slice offsets, the work list of the quad pair sums and
 // the sizes a build reads back: host[10] (pinned) = flag, pairs, records,
-// entries, list slots (-1: the total at the end of the scanned array),
-// largest record count, most targets of a brick, unstaged bricks, bricks
-// with targets, work items
+// entries, list slots (-1: the total at the end of slice_off), largest record
+// count, most targets of a brick, unstaged bricks, bricks with targets, work
+// items
 hipError_t launch_build_sizes(ggem_ctx* ctx, int64_t* host);
+size_t size_tile_bytes(const ggem_ctx* ctx);  // what size_tiles holds for it
 // exclusive scan of int64 values; out[len] receives the total
 hipError_t launch_scan64(ggem_ctx* ctx, const int64_t* in, int64_t len, int64_t* out);
 hipError_t launch_fill_ell(ggem_ctx* ctx);
