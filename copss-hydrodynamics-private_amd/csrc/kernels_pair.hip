@@ -2131,16 +2131,23 @@ hipError_t launch_pair_beads(ggem_ctx* ctx, int precision, int epi, const double
 
 hipError_t launch_pair_points(ggem_ctx* ctx, int precision, int64_t m, const double* pts,
                               const int32_t* elem, double* u) {
-  if (m == 0) return hipSuccess;
   const PairArgs a = make_args(ctx);
   ProfScope ps(ctx, precision == GGEM_FP64 ? "pair_points_fp64" : "pair_points_fp32c");
-  if (precision == GGEM_FP64)
-    hipLaunchKernelGGL(k_pair_points<GGEM_FP64>, dim3(blocks_for(m * kPointLanes)), dim3(kBlock), 0, ctx->stream, a,
-                       ctx->rows_d, ctx->n_rows, ctx->cell_start, ctx->fg32, ctx->fg64, m, pts, elem, u);
-  else
-    hipLaunchKernelGGL(k_pair_points<GGEM_FP32C>, dim3(blocks_for(m * kPointLanes)), dim3(kBlock), 0, ctx->stream, a,
-                       ctx->rows_d, ctx->n_rows, ctx->cell_start, ctx->fg32, ctx->fg64, m, pts, elem, u);
-  return hipGetLastError();
+  // a launch of 2^32 threads or more comes out short: up to 2^27 points each
+  constexpr int64_t kMost = (int64_t(1) << 31) / kPointLanes;
+  for (int64_t q = 0; q < m; q += kMost) {
+    const int64_t k = std::min(kMost, m - q);
+    const dim3 grid(blocks_for(k * kPointLanes));
+    if (precision == GGEM_FP64)
+      hipLaunchKernelGGL(k_pair_points<GGEM_FP64>, grid, dim3(kBlock), 0, ctx->stream, a, ctx->rows_d, ctx->n_rows,
+                         ctx->cell_start, ctx->fg32, ctx->fg64, k, pts + 3 * q, elem + q, u + 3 * q);
+    else
+      hipLaunchKernelGGL(k_pair_points<GGEM_FP32C>, grid, dim3(kBlock), 0, ctx->stream, a, ctx->rows_d, ctx->n_rows,
+                         ctx->cell_start, ctx->fg32, ctx->fg64, k, pts + 3 * q, elem + q, u + 3 * q);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 int64_t apply_ref_blocks(const ggem_ctx* ctx) {
