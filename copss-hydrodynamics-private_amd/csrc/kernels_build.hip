@@ -281,9 +281,11 @@ __global__ void k_gather_forces(int64_t n, const int32_t* __restrict__ perm, con
 // brick's box (the brick widened by the stencil reach) go to LDS once:
 // per box cell the first slot of its grid cell and the particles of the
 // box cells before it.  Each target (slot or element) of the brick then
-// walks its stencil rows through LDS (box_walk), in for_each_segment's
-// order, so the lists and counts equal the per-slot walks over the global
-// cell starts, which serve bricks whose box does not fit the LDS tables.
+// walks its stencil rows through LDS (box_walk_flat, box_walk_rec) or has a
+// wave test the records against the stencil (wave_records), all in
+// for_each_segment's order, so the lists and counts equal those of the walks
+// over the global cell starts, which serve bricks whose box does not fit the
+// LDS tables.
 constexpr int kBrickThreads = 256;
 
 struct BrickArgs {

@@ -18,9 +18,10 @@
 // record per neighbour.  FP32C, one operand: per brick of cells the
 // neighbours' records are staged in LDS and the entries stream a 2-byte
 // record number (k_box_fill, k_apply_box, k_apply_quad, below).  FP32C,
-// several operands: k_apply_quad, four lanes per target.  The explicit
-// minimum image, bricks that are not staged: k_apply evaluates (A, Bx) per
-// pair from the coefficient table in LDS.  Blocks are
+// several operands: k_apply_quad, four lanes per target, and in dense bricks
+// k_apply_box_nr, one.  The explicit minimum image, bricks that are not
+// staged: k_apply evaluates (A, Bx) per pair from the coefficient table in
+// LDS.  Blocks are
 // renumbered per XCD so a chip partition keeps a contiguous stretch of
 // cells and their neighbours in its L2.
 //
@@ -695,8 +696,8 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
 // particles of a cell in slot order, so a stencil run of box cells is one
 // range of records.  Once per list build k_box_fill writes every staged
 // brick's records (slot, cell-relative FP32 position with the packed box
-// cell) and walks each target's stencil through them in list order
-// (box_walk): per kept entry the neighbour's record number (16 bits).
+// cell) and finds each target's among them in list order (wave_records,
+// box_walk_rec): per kept entry the neighbour's record number (16 bits).
 // k_apply_box copies the records, their operands and the coefficient table
 // to LDS and streams the record numbers (2 bytes per pair): per pair the
 // neighbour from LDS and (A, Bx) from the table at the displacement, a
@@ -712,7 +713,8 @@ constexpr int kBoxThreads = 256;
 // goes round a second time in every brick with more (23 of 100 at 244 targets
 // a brick), with a few lanes and at the latency of a whole list; the further
 // threads cost nothing and help to stage.  125,000 beads: 41.6 -> 35.2 us per
-// application, and 34.2 us with the tensors loaded a group ahead (3.0 TB/s).
+// application, and 34.2 us with the tensors loaded a group ahead (211 MB at
+// 6.1 TB/s).
 // FP32C is not bound by that latency (1M beads: 82.7 us either way).
 constexpr int kDenseThreads = 512;
 // A target's packed entry base: the offset of its entry 0 (below 2^40), its

@@ -336,7 +336,9 @@ typedef struct ggem_op {
 typedef struct ggem_cheb_info {
   int32_t converged;  /* reference-compat mode: the stopping rule fired on err1 */
   int32_t terms;      /* highest Chebyshev index used                          */
-  int32_t applies;    /* operator applications                                 */
+  int32_t applies;    /* operator applications of the reference's algorithm
+                         (two a term, and M y where asked for; the device
+                         operator takes one a term in reference mode)         */
   int32_t pad;
   double err1, err2;  /* estimators of brownian_system.C:1076-1131             */
 } ggem_cheb_info;
