@@ -1898,11 +1898,21 @@ unsigned n_bricks(const ggem_ctx* ctx) { return unsigned(ctx->grid.n_cells >> (3
 // for all of them: quads lose where bricks use the threads of a lane block (45
 // targets at two operands, 95 at four) and the lanes fill the chip (beads, or
 // beads times targets a brick where the staging decides).
+// FP32C with one operand, quads -> one lane over many beads:
+//   beads    element (records a target)  targets: us per application
+//   100,000  3.1 (5.4)  58: 15.0 -> 15.9;  3.9 (3.4)  46: 13.3 -> 13.0  100: 15.0 -> 13.9
+//   200,000  2.0 (11)   41: 32 -> 42;      3.9        49: 19.7 -> 18.5   91: 22.4 -> 20.1
+//   400,000  3.1        38: 37 -> 35;      3.9        50: 31.4 -> 27.9   98: 37.3 -> 29.2
+//   800,000  2.0        41: 119 -> 140;    3.1  36: 67 -> 62  3.9  46: 57 -> 50  137: 69 -> 50
+// The chip is full either way there, and what counts is how many of a lane
+// block's threads the staging of a target's records keeps busy: targets a
+// brick over records a target.
 bool quad_lanes(const ggem_ctx* ctx, int precision, int nr) {
-  const int64_t n = ctx->n, b = ctx->full_bricks;
+  const int64_t n = ctx->n, b = ctx->full_bricks, recs = ctx->box_recs;
   if (nr == 2) return n < 45 * b || (n < 65536 && n * n < 10000000 * b);
   if (nr > 2) return n < 95 * b || n * n < 6200000 * b;
-  if (precision == GGEM_FP32C) return n <= 150 * b;
+  if (precision == GGEM_FP32C)
+    return n <= 150 * b && (n < 100000 || n * n <= (n < 262144 ? 13 : 6) * b * recs);
   return n <= 40 * b || ctx->quad_items <= 256;
 }
 

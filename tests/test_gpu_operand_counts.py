@@ -79,3 +79,23 @@ def test_dense_bricks_equal_the_list_order_kernel(box, ne, periodic, nrhs):
             got.append(ctx.cheb_brownian(3, 0.02, 3.0, dw, mode=G.CHEB_FIXED)[:2])
     for y, d in got[1:]:
         assert np.array_equal(y, got[0][0]) and np.array_equal(d, got[0][1])
+
+
+@pytest.mark.parametrize("n,ne,h", [(101000, 80, 3.9), (101000, 96, 3.1)])
+def test_one_vector_many_beads(n, ne, h):
+    """One FP32C vector on either side of the rule at 100,000 beads (101 and 59
+    a brick) against the list-order kernel."""
+    rng = np.random.default_rng(ne)
+    x, f = rng.random((n, 3)) * ne * h, rng.normal(size=(n, 3))
+    dw = G.normal(3 * n, 41).reshape(1, n, 3)
+    got = []
+    for lists in (False, True):
+        with G.Context(W._cfg([0, 0, 0], [ne * h] * 3, [1, 1, 0], [ne] * 3, precision=G.FP32C)) as ctx:
+            ctx.reinit(x, f)
+            if lists:
+                for key in ("apply/fp32c/1/16", "pair_beads/fp32c/0/16"):
+                    ctx.tune_set(key, 0)
+                ctx.set_autotune(True)
+            got.append((ctx.local_velocity_beads(), *ctx.cheb_brownian(3, 0.02, 3.0, dw, mode=G.CHEB_FIXED)[:2]))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
