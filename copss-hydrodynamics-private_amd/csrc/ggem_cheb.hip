@@ -230,6 +230,7 @@ int run_fixed_graph(ggem_ctx* ctx, Applier& apply, FixedStep s) {
   const std::vector<uintptr_t> key = {
       uintptr_t(s.N), uintptr_t(s.nrhs), uintptr_t(ctx->p.precision), uintptr_t(s.disp), uintptr_t(ctx->n),
       uintptr_t(explicit_minimg(ctx)),  // (a kernel argument of the list-order sums)
+      uintptr_t(apply_plan(ctx, ctx->p.precision)),
       uintptr_t(s.dw_dev), uintptr_t(s.dpar), uintptr_t(P.vec), uintptr_t(P.g32), uintptr_t(P.g64),
       uintptr_t(ctx->x4), uintptr_t(ctx->nbr_cnt), uintptr_t(ctx->slice_off), uintptr_t(ctx->ell),
       uintptr_t(ctx->perm), uintptr_t(ctx->fs), uintptr_t(ctx->tab32), uintptr_t(ctx->coef64),

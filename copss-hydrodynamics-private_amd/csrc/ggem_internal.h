@@ -566,6 +566,9 @@ hipError_t launch_apply_ref(ggem_ctx* ctx, int precision, const SlotVec& x, cons
 int64_t apply_ref_blocks(const ggem_ctx* ctx);
 // operands of the next launch of `left`
 int apply_chunk(const ggem_ctx* ctx, int precision, int left);
+// what the present lists make of every operand count: launch size, staged or
+// list order, lanes per target (for the key of a captured step)
+uint64_t apply_plan(const ggem_ctx* ctx, int precision);
 // whether some pair sum of nrhs operands reads the sliced lists (after prepare_box)
 bool apply_reads_lists(const ggem_ctx* ctx, int precision, int nrhs);
 // v = M x (+ epilogue) for nrhs slot vectors (x, v: nrhs consecutive SlotVecs

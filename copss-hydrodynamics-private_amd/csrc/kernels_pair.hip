@@ -2001,9 +2001,29 @@ bool box_ready(const ggem_ctx* ctx, int precision, int nr) {
   if (!ctx->box_valid || ctx->box_max <= 0) return false;
   return precision == GGEM_FP32C ? !ctx->box_fp64 : (ctx->box_fp64 && ctx->coef64_valid);
 }
-// the staged kernel by default wherever it applies
+// The staged kernel by default wherever it applies, except for several
+// operands in many sparse bricks: a quad block's cost is then the block, not
+// its few targets, while the list-order kernel fills its waves.  By bricks
+// with targets over the records of each, and bricks enough for the blocks to
+// outweigh a wave that walks its lists alone; quads -> list order, us:
+//   beads (bricks)    element  2 operands      4               8
+//   5,000 (3,500)     2.0      12.3 -> 10.2    12.6 -> 13.0    15.8 -> 18.9
+//   10,000 (7,000)    2.0      17.9 -> 10.3    19.0 -> 12.9    25.1 -> 18.8
+//   14,000 (1,750)    3.1      10.4 -> 12.0    -               -
+//   30,000 (1,728)    2.0      15.6 -> 22.4    17.0 -> 33.0    26.9 -> 53.0
+//   65,000 (9,261)    2.0      30.4 -> 17.5    33.6 -> 25.6    46.3 -> 38.7
+//   100,000 (5,832)   2.0      32.4 -> 30.2    36.4 -> 48.2    63.4 -> 73.9
+//   100,000 (5,832)   3.1      25.1 -> 18.6    29.0 -> 29.4    43.5 -> 44.1
+//   140,000 (8,000)   3.9      30.2 -> 18.4    34.5 -> 26.6    52.4 -> 45.3
+//   300,000 (10,648)  2.0      68.1 -> 69.6    90.4 -> 115     -
+//   300,000 (39,304)  2.0      109 -> 37.4     123 -> 60.8     -
+bool sparse_bricks(const ggem_ctx* ctx, int nr) {
+  const int64_t b = ctx->full_bricks;
+  return b >= (nr == 2 ? 3000 : nr == 4 ? 4500 : 6000) && b * b > (nr == 2 ? 33 : nr == 4 ? 65 : 100) * ctx->box_recs;
+}
 int apply_default(const ggem_ctx* ctx, int precision, int nr) {
-  return box_ready(ctx, precision, nr) ? kBoxShape : 0;
+  if (!box_ready(ctx, precision, nr)) return 0;
+  return nr > 1 && quad_lanes(ctx, precision, nr) && sparse_bricks(ctx, nr) ? 0 : kBoxShape;
 }
 int apply_candidates(const ggem_ctx* ctx, int precision, int nr) {
   return box_ready(ctx, precision, nr) ? kNApply + 1 : kNApply;
@@ -2176,11 +2196,18 @@ int apply_chunk(const ggem_ctx* ctx, int precision, int left) {
       if (box_nr_ready(ctx, m)) return m;
   return nr;
 }
+uint64_t apply_plan(const ggem_ctx* ctx, int precision) {
+  uint64_t plan = 0;
+  for (int nr = 1; nr <= 8; nr *= 2)
+    plan = (plan << 6) | (uint64_t(apply_chunk(ctx, precision, nr)) << 2) |
+           (apply_default(ctx, precision, nr) == kBoxShape ? 2u : 0u) | (quad_lanes(ctx, precision, nr) ? 1u : 0u);
+  return plan;
+}
 bool apply_reads_lists(const ggem_ctx* ctx, int precision, int nrhs) {
   if (ctx->tune.on) return true;
   for (int left = nrhs; left > 0;) {
     const int nr = apply_chunk(ctx, precision, left);
-    if (!box_ready(ctx, precision, nr) || ctx->box_unstaged) return true;
+    if (apply_default(ctx, precision, nr) != kBoxShape || ctx->box_unstaged) return true;
     left -= nr;
   }
   return false;

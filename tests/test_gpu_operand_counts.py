@@ -81,6 +81,37 @@ def test_dense_bricks_equal_the_list_order_kernel(box, ne, periodic, nrhs):
         assert np.array_equal(y, got[0][0]) and np.array_equal(d, got[0][1])
 
 
+@pytest.mark.parametrize("nrhs", [2, 4, 8, 13])
+def test_sparse_and_dense_builds_in_turn(nrhs):
+    """Several FP32C vectors on one context through builds that change their
+    route: 8,000 beads over 6,200 bricks (list order), the same beads in a
+    corner (staged), over the bricks again; the captured step follows.  Each
+    step against the staged kernels pinned, and against one vector alone."""
+    n, ne, h = 8000, 200, 2.0
+    rng = np.random.default_rng(nrhs)
+    wide = rng.random((n, 3)) * ne * h
+    sets = [wide, wide * 0.2, wide]
+    f = rng.normal(size=(n, 3))
+    dw = G.normal(nrhs * 3 * n, 37).reshape(nrhs, n, 3)
+    step = lambda c, w: c.cheb_brownian(4, 0.02, 3.0, w, mode=G.CHEB_FIXED)[:2]
+    cfg = W._cfg([0, 0, 0], [ne * h] * 3, [1, 1, 1], [ne] * 3, precision=G.FP32C)
+    with G.Context(cfg) as ctx, G.Context(cfg) as staged:
+        for nr in (1, 2, 4, 8):
+            staged.tune_set("apply/fp32c/%d/12" % nr, 5)
+        staged.set_autotune(True)
+        for x in sets:
+            ctx.reinit(x, f)
+            staged.reinit(x, f)
+            want = step(staged, dw)
+            ctx.set_graph(False)
+            got = step(ctx, dw)
+            ctx.set_graph(True)
+            for y, d in (got, step(ctx, dw), step(ctx, dw)):
+                assert np.array_equal(y, want[0]) and np.array_equal(d, want[1])
+            one = step(ctx, dw[:1])
+            assert np.array_equal(one[0][0], want[0][0]) and np.array_equal(one[1][0], want[1][0])
+
+
 @pytest.mark.parametrize("n,ne,h", [(101000, 80, 3.9), (101000, 96, 3.1)])
 def test_one_vector_many_beads(n, ne, h):
     """One FP32C vector on either side of the rule at 100,000 beads (101 and 59
