@@ -384,9 +384,8 @@ extern "C" int ggem_cheb_brownian(ggem_ctx* ctx, const ggem_op* op, int32_t N, d
     // at a time; the device's own operator decides where to stop on the
     // device, a host operator on the host
     if (!op) {
-      const int64_t nb = apply_ref_blocks(ctx);
       if ((rc = ensure(ctx, &P.cref, &P.cref_cap, size_t(8 * nrhs)))) return rc;
-      if ((rc = ensure(ctx, &P.red, &P.red_cap, size_t(3 * nb)))) return rc;
+      if ((rc = ensure(ctx, &P.red, &P.red_cap, size_t(apply_ref_parts(ctx))))) return rc;
       if ((rc = ensure(ctx, &P.cstop, &P.cstop_cap, size_t(nrhs + 1 + kRefGroups)))) return rc;
     }
     for (int r = 0; r < nrhs && !op; ++r) {

@@ -511,15 +511,16 @@ enum Epi : int {
 // The reference mode's term k (one operand): m = M x_k gives y += c_k x_k,
 // M y += c_k m and x_{k+1}, so the estimators of term k need no application
 // of their own (M y is the same combination of the M x_j as y is of the
-// x_j).  Every block of the pair sum leaves its part of three dot products
-// and the last block to finish adds them in block order, forms the
-// estimators and decides (brownian_system.C:1030-1155).
+// x_j).  Every block of the pair sum leaves its part of three dot products;
+// the last block to finish, or for many blocks a launch after it, adds them
+// in block order, forms the estimators and decides
+// (brownian_system.C:1030-1155).
 constexpr int kRefGroups = 32;
 struct RefEpi {
   double c;         // c_k
   double* my;       // [3][n] M y so far
   double* part;     // [3][blocks] each block's part of (M y).(M y) (term 0: (M x0).x0), y.y and x_k.x_k
-  int32_t* ticket;  // [1 + kRefGroups] blocks done (zero between launches)
+  int32_t* ticket;  // [1 + kRefGroups] blocks done (zero between launches); null: the parts are all
   double* st;       // [8] (M x0).x0, y.y of the last term, -, -, err1, err2, terms, converged
   int32_t* stop;
   double tol;
@@ -561,9 +562,9 @@ hipError_t launch_pair_beads(ggem_ctx* ctx, int precision, int epi, const double
 hipError_t launch_pair_points(ggem_ctx* ctx, int precision, int64_t m, const double* pts,
                               const int32_t* elem, double* u);
 // one term of the reference mode (EPI_REF) for one slot vector, and the
-// most blocks any launch shape of it has (the length of RefEpi::part / 3)
+// length of RefEpi::part for any launch shape of it
 hipError_t launch_apply_ref(ggem_ctx* ctx, int precision, const SlotVec& x, const SlotVec& v, const ChebEpi& epi);
-int64_t apply_ref_blocks(const ggem_ctx* ctx);
+int64_t apply_ref_parts(const ggem_ctx* ctx);
 // operands of the next launch of `left`
 int apply_chunk(const ggem_ctx* ctx, int precision, int left);
 // what the present lists make of every operand count: launch size, staged or

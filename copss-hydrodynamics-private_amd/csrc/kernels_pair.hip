@@ -419,53 +419,9 @@ __device__ __forceinline__ void block_add3(double (&t)[3]) {
   __syncthreads();
 }
 
-// End of a reference-mode launch, the whole block with its parts of the
-// three dot products: they go to memory past the XCD's L2 (agent scope), and
-// the last block to finish adds all blocks' parts (in block order, whichever
-// block that is) and applies the stopping rule.  Tickets are drawn in
-// kRefGroups groups, a group's last block drawing one of the top: a single
-// ticket's atomics follow one another at 11 ns each (700 blocks: 8 us).
-// One launch per term instead of six: per-term dot products, gather records
-// and the deciding kernel were 16 us of the 66 us a term took for 25,600
-// chain beads.
-__device__ __forceinline__ void ref_finish(const ChebEpi& epi, const double (&dots)[3]) {
-  __shared__ int s_last;
-  const RefEpi& R = epi.ref;
-  const int nb = int(gridDim.x), id = int(blockIdx.x);
-  double t[3] = {dots[0], dots[1], dots[2]};
-  block_add3(t);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q)
-      __hip_atomic_store(R.part + int64_t(q) * nb + id, t[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int g = id % kRefGroups, groups = min(nb, kRefGroups), in_group = (nb - g + kRefGroups - 1) / kRefGroups;
-    bool last = __hip_atomic_fetch_add(R.ticket + 1 + g, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == in_group - 1;
-    if (last) last = __hip_atomic_fetch_add(R.ticket, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
-    s_last = last;
-  }
-  __syncthreads();
-  if (!s_last) return;  // uniform over the block
-#pragma unroll
-  for (int q = 0; q < 3; ++q) t[q] = 0.0;
-  constexpr int U = 4;  // parts in flight per thread and product
-  for (int b = int(threadIdx.x); b < nb; b += U * int(blockDim.x)) {
-    double w[U][3];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int bu = min(b + u * int(blockDim.x), nb - 1);
-#pragma unroll
-      for (int q = 0; q < 3; ++q)
-        w[u][q] = __hip_atomic_load(R.part + int64_t(q) * nb + bu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (b + u * int(blockDim.x) < nb)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) t[q] += w[u][q];
-  }
-  block_add3(t);
-  if (threadIdx.x <= kRefGroups) R.ticket[threadIdx.x] = 0;  // (blocks have 64 threads or more)
-  if (threadIdx.x != 0) return;
+// The estimators and the stopping rule of a reference-mode term from its three
+// dot products t (one thread)
+__device__ __forceinline__ void ref_rule(const RefEpi& R, const double (&t)[3]) {
   if (R.term == 0) {
     R.st[0] = t[0];
   } else {
@@ -486,6 +442,90 @@ __device__ __forceinline__ void ref_finish(const ChebEpi& epi, const double (&do
     }
   }
   R.st[1] = t[1];
+}
+
+// The whole block's sums of the three dot products over parts b0 .. b1 - 1 of
+// nb, as load(q nb + b) reads them
+template <class Load>
+__device__ __forceinline__ void ref_sum(int b0, int b1, int nb, double (&t)[3], Load&& load) {
+#pragma unroll
+  for (int q = 0; q < 3; ++q) t[q] = 0.0;
+  constexpr int U = 4;  // parts in flight per thread and product
+  for (int b = b0 + int(threadIdx.x); b < b1; b += U * int(blockDim.x)) {
+    double w[U][3];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int bu = min(b + u * int(blockDim.x), b1 - 1);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) w[u][q] = load(int64_t(q) * nb + bu);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (b + u * int(blockDim.x) < b1)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) t[q] += w[u][q];
+  }
+  block_add3(t);
+}
+
+// The decision by the launch's last block to finish: every block's parts t go
+// to memory past the XCD's L2 (agent scope), and the last block adds all of
+// them (in block order, whichever block that is) and applies the stopping
+// rule.  Tickets are drawn in kRefGroups groups, a group's last block drawing
+// one of the top: a single ticket's atomics follow one another at 11 ns each
+// (700 blocks: 8 us).
+__device__ __forceinline__ void ref_tickets(const RefEpi& R, double (&t)[3]) {
+  __shared__ int s_last;
+  const int nb = int(gridDim.x), id = int(blockIdx.x);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      __hip_atomic_store(R.part + int64_t(q) * nb + id, t[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int g = id % kRefGroups, groups = min(nb, kRefGroups), in_group = (nb - g + kRefGroups - 1) / kRefGroups;
+    bool last = __hip_atomic_fetch_add(R.ticket + 1 + g, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == in_group - 1;
+    if (last) last = __hip_atomic_fetch_add(R.ticket, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
+    s_last = last;
+  }
+  __syncthreads();
+  if (!s_last) return;  // uniform over the block
+  ref_sum(0, nb, nb, t, [&](int64_t i) {
+    return __hip_atomic_load(R.part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  });
+  if (threadIdx.x <= kRefGroups) R.ticket[threadIdx.x] = 0;  // (blocks have 64 threads or more)
+  if (threadIdx.x == 0) ref_rule(R, t);
+}
+
+// End of a reference-mode launch, the whole block with its parts of the
+// three dot products: the decision in the launch itself where it has few
+// blocks (one launch per term instead of six: per-term dot products, gather
+// records and the deciding kernel were 16 us of the 66 us a term took for
+// 25,600 chain beads), else the parts left to k_ref_decide (null ticket).
+__device__ __forceinline__ void ref_finish(const ChebEpi& epi, const double (&dots)[3]) {
+  const RefEpi& R = epi.ref;
+  double t[3] = {dots[0], dots[1], dots[2]};
+  block_add3(t);
+  if (R.ticket) {
+    ref_tickets(R, t);
+  } else if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) R.part[int64_t(q) * gridDim.x + blockIdx.x] = t[q];
+  }
+}
+
+// The decision of a launch of many blocks, over the nb parts it left (nothing
+// after the stop): a ticket's release writes the XCD's L2 back, 20 to 40 ns a
+// block while the pair sums' results are in it.  Per term, one more launch
+// against tickets, us: 3,000 beads (125 blocks) 13.4 and 12.8; 8,000 (343)
+// 14.5 and 17.6; 26,000 (1,000) 16.8 and 34.5; 120,000 (4,096) 37 and 131;
+// 400,000 (50,653) 227 and 1,267.  One block for every kRefDecideParts parts.
+constexpr int kRefDecideThreads = 1024, kRefDecideParts = 8192;
+__global__ void __launch_bounds__(kRefDecideThreads) k_ref_decide(RefEpi R, const double* __restrict__ parts, int nb) {
+  if (*R.stop) return;  // uniform over the grid: set by the block that finishes last
+  const int b0 = int(int64_t(nb) * blockIdx.x / gridDim.x), b1 = int(int64_t(nb) * (blockIdx.x + 1) / gridDim.x);
+  double t[3];
+  ref_sum(b0, b1, nb, t, [&](int64_t i) { return parts[i]; });
+  if (gridDim.x > 1) ref_tickets(R, t);
+  else if (threadIdx.x == 0) ref_rule(R, t);
 }
 
 // Output of one target: m = sum over its list of G_ij x_j for NR operand
@@ -2182,8 +2222,10 @@ hipError_t launch_pair_points(ggem_ctx* ctx, int precision, int64_t m, const dou
   return hipSuccess;
 }
 
-int64_t apply_ref_blocks(const ggem_ctx* ctx) {
-  return std::max<int64_t>(blocks_for(ctx->n, 64), std::max<int64_t>(n_bricks(ctx), ctx->quad_items));
+int64_t apply_ref_parts(const ggem_ctx* ctx) {
+  const int64_t nb =
+      std::max<int64_t>(blocks_for(ctx->n, 64), std::max<int64_t>(n_bricks(ctx), ctx->quad_items));
+  return 3 * (nb + (nb + kRefDecideParts - 1) / kRefDecideParts);
 }
 
 // operands of the next launch of `left`: the largest power of two up to 8,
@@ -2213,16 +2255,32 @@ bool apply_reads_lists(const ggem_ctx* ctx, int precision, int nrhs) {
   return false;
 }
 
+// Most blocks of a reference-mode launch that decide by tickets (k_ref_decide:
+// both sides)
+constexpr int64_t kRefTicketBlocks = 128;
+
 hipError_t launch_apply_ref(ggem_ctx* ctx, int precision, const SlotVec& x, const SlotVec& v, const ChebEpi& epi) {
   if (ctx->n == 0) return hipSuccess;
   const PairArgs a = make_args(ctx);
   // (the term updates y in place: the pick of plain applications serves)
   const int c = apply_pick(ctx, precision, 1,
                            tune_lookup(ctx, tune_key("apply", precision, 1, ctx->n), apply_default(ctx, precision, 1)));
+  ChebEpi e = epi;
+  int64_t nb = 0;
+  if (c == kBoxShape) nb = quad_lanes(ctx, precision, 1) ? ctx->quad_items : int64_t(n_bricks(ctx));
+  else if (c >= 0 && c < kNApply) nb = blocks_for(ctx->n, kApplyShapes[c].block);
+  if (nb > kRefTicketBlocks) e.ref.ticket = nullptr;
   ProfScope ps(ctx, precision == GGEM_FP64 ? "apply_fp64" : "apply_fp32c");
-  return precision == GGEM_FP64
-             ? launch_k<GGEM_FP64, 1, EPI_REF>(ctx, a, c, x.g64, x.g32, x.soa, v, epi, nullptr, nullptr)
-             : launch_k<GGEM_FP32C, 1, EPI_REF>(ctx, a, c, x.g64, x.g32, x.soa, v, epi, nullptr, nullptr);
+  const hipError_t err =
+      precision == GGEM_FP64
+          ? launch_k<GGEM_FP64, 1, EPI_REF>(ctx, a, c, x.g64, x.g32, x.soa, v, e, nullptr, nullptr)
+          : launch_k<GGEM_FP32C, 1, EPI_REF>(ctx, a, c, x.g64, x.g32, x.soa, v, e, nullptr, nullptr);
+  if (err != hipSuccess || e.ref.ticket) return err;
+  RefEpi r = epi.ref;  // (the deciding blocks' own parts after the launch's)
+  r.part += 3 * nb;
+  hipLaunchKernelGGL(k_ref_decide, dim3(unsigned((nb + kRefDecideParts - 1) / kRefDecideParts)),
+                     dim3(kRefDecideThreads), 0, ctx->stream, r, epi.ref.part, int(nb));
+  return hipGetLastError();
 }
 
 hipError_t launch_apply(ggem_ctx* ctx, int precision, int nrhs, const SlotVec& x, const SlotVec& v,
