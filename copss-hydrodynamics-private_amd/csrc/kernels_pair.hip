@@ -749,12 +749,12 @@ __global__ void __launch_bounds__(BLK) k_apply(PairArgs a, const void* __restric
 // A brick whose box holds more than kBoxMaxRecs records reads its list and
 // gathers the neighbours' records from global memory.
 constexpr int kBoxThreads = 256;
-// FP64 with a lane per target: threads for twice 256 targets.  A block of 256
-// goes round a second time in every brick with more (23 of 100 at 244 targets
-// a brick), with a few lanes and at the latency of a whole list; the further
-// threads cost nothing and help to stage.  125,000 beads: 41.6 -> 35.2 us per
-// application, and 34.2 us with the tensors loaded a group ahead (211 MB at
-// 6.1 TB/s).
+// FP64 with a lane per target in dense bricks or few (dense64): threads for
+// twice 256 targets.  A block of 256 goes round a second time in every brick
+// with more (23 of 100 at 244 targets a brick), with a few lanes and at the
+// latency of a whole list; the further threads cost nothing there and help to
+// stage.  125,000 beads: 41.6 -> 35.2 us per application, and 34.2 us with the
+// tensors loaded a group ahead (211 MB at 6.1 TB/s).
 // FP32C is not bound by that latency (1M beads: 82.7 us either way).
 constexpr int kDenseThreads = 512;
 // A target's packed entry base: the offset of its entry 0 (below 2^40), its
@@ -1657,8 +1657,8 @@ __global__ void __launch_bounds__(kBoxThreads) k_apply_quad64(PairArgs a, BoxVie
 // layout), the operand read from LDS.  List order and fp64_acc as in
 // k_apply, so the sums are bit-identical.  A brick that is not staged
 // gathers the operands from global memory.
-template <int EPI>
-__global__ void __launch_bounds__(kDenseThreads) k_apply_box64(PairArgs a, BoxView b, const double4* __restrict__ c64,
+template <int EPI, int NT>
+__global__ void __launch_bounds__(NT) k_apply_box64(PairArgs a, BoxView b, const double4* __restrict__ c64,
                                                             const double4* __restrict__ xg,
                                                             const double* __restrict__ xsoa, SlotVec v, ChebEpi epi,
                                                             const double* __restrict__ u_glob,
@@ -1680,21 +1680,21 @@ __global__ void __launch_bounds__(kDenseThreads) k_apply_box64(PairArgs a, BoxVi
   if (nrec > 0) {
     // four records in flight per thread, then the remainder one at a time
     int i = int(threadIdx.x);
-    for (; i + 3 * kDenseThreads < nrec; i += 4 * kDenseThreads) {
-      const uint32_t t0 = b.slot[r0 + i], t1 = b.slot[r0 + i + kDenseThreads];
-      const uint32_t t2 = b.slot[r0 + i + 2 * kDenseThreads], t3 = b.slot[r0 + i + 3 * kDenseThreads];
+    for (; i + 3 * NT < nrec; i += 4 * NT) {
+      const uint32_t t0 = b.slot[r0 + i], t1 = b.slot[r0 + i + NT];
+      const uint32_t t2 = b.slot[r0 + i + 2 * NT], t3 = b.slot[r0 + i + 3 * NT];
       const double4 f0 = xg[t0], f1 = xg[t1], f2 = xg[t2], f3 = xg[t3];
       rval[i] = f0;
-      rval[i + kDenseThreads] = f1;
-      rval[i + 2 * kDenseThreads] = f2;
-      rval[i + 3 * kDenseThreads] = f3;
+      rval[i + NT] = f1;
+      rval[i + 2 * NT] = f2;
+      rval[i + 3 * NT] = f3;
     }
-    for (; i < nrec; i += kDenseThreads) rval[i] = xg[b.slot[r0 + i]];
+    for (; i < nrec; i += NT) rval[i] = xg[b.slot[r0 + i]];
     __syncthreads();
   }
   const double sg = a.bsign;
   constexpr int U = 2;  // entries per group, the next group's tensors and record numbers loaded one ahead (4: 34.0)
-  for (int i = int(threadIdx.x); i < nt; i += kDenseThreads) {
+  for (int i = int(threadIdx.x); i < nt; i += NT) {
     const int64_t s = sb + i;
     const int cnt = a.cnt[s];
     const int64_t base = a.slice_off[s >> 6] + (s & 63);
@@ -1917,8 +1917,18 @@ unsigned n_bricks(const ggem_ctx* ctx) { return unsigned(ctx->grid.n_cells >> (3
 //   FP64                10.9->10.3  8.3->7.3   10.6->9.8   9.6->9.8    16.6->17.0  24.3->26.3  43.9->45.7
 // and 87 -> 122 us at 1M beads (244, FP32C): there the lanes are busy either
 // way and the sums on every lane of a quad only cost.  FP64 streams its
-// tensors and gains by the split only where the blocks leave CUs idle (the
-// lane kernel has since gone to 34.2 us at 244 targets, quads there 37.1).
+// tensors and gains by the split only where few beads leave CUs idle.  Quads,
+// a lane per target in blocks of 256 and of 512, us per application:
+//   beads      targets:  quads 256  512    targets:  quads 256  512
+//   12,000     23 (3.9)   7.7  8.1  8.3     96        8.8 10.4 10.2
+//              188       14.1 18.6 13.9
+//   30,000     17 (2.5)  11.2 10.4 11.5     59       11.9 11.2 10.5
+//              240       18.7 23.7 16.6
+//   120,000    29 (3.9)  19.3 16.2 21.7     55 (3.1) 24.8 21.8 22.5
+//              120       26.0 23.1 23.9     234      41.1 41.6 37.0
+//   400,000    18 (2.5)  70.0 55.8 90.2     50 (3.9) 46.1 35.6 42.6
+//              182        132  119  120     231       158  150  137
+//   1,000,000  20 (3.1)   183  152  254     46 (3.9)  142  114  147
 // FP32C with several operands, quads -> one lane (k_apply_box_nr; 8 as 4 + 4;
 // * as 2 + 2, the records of 4 exceed the LDS), us per application:
 //   beads    targets   2 operands      4 operands      8 operands
@@ -1953,7 +1963,14 @@ bool quad_lanes(const ggem_ctx* ctx, int precision, int nr) {
   if (nr > 2) return n < 95 * b || n * n < 6200000 * b;
   if (precision == GGEM_FP32C)
     return n <= 150 * b && (n < 100000 || n * n <= (n < 262144 ? 13 : 6) * b * recs);
-  return n <= 40 * b || ctx->quad_items <= 256;
+  return n < 20000;
+}
+
+// FP64 with a lane per target: blocks of 512 threads, where bricks often hold
+// more than 256 targets or fewer blocks than two per CU leave wave slots free;
+// elsewhere most of their threads would have no target (the table above)
+bool dense64(const ggem_ctx* ctx) {
+  return ctx->n > 200 * int64_t(ctx->full_bricks) || n_bricks(ctx) <= 512;
 }
 
 size_t box_lds(const ggem_ctx* ctx, int nr) {
@@ -2027,8 +2044,11 @@ hipError_t launch_box64(ggem_ctx* ctx, PairArgs a, const double4* xg, const doub
   if (quad_lanes(ctx, GGEM_FP64, 1))
     hipLaunchKernelGGL((k_apply_quad64<EPI>), dim3(unsigned(ctx->quad_items)), dim3(kBoxThreads), lds, ctx->stream, a,
                        box_view(ctx), ctx->coef64, xg, soa, v, epi, u_glob, out);
+  else if (dense64(ctx))
+    hipLaunchKernelGGL((k_apply_box64<EPI, kDenseThreads>), dim3(n_bricks(ctx)), dim3(kDenseThreads), lds, ctx->stream,
+                       a, box_view(ctx), ctx->coef64, xg, soa, v, epi, u_glob, out);
   else
-    hipLaunchKernelGGL((k_apply_box64<EPI>), dim3(n_bricks(ctx)), dim3(kDenseThreads), lds, ctx->stream, a,
+    hipLaunchKernelGGL((k_apply_box64<EPI, kBoxThreads>), dim3(n_bricks(ctx)), dim3(kBoxThreads), lds, ctx->stream, a,
                        box_view(ctx), ctx->coef64, xg, soa, v, epi, u_glob, out);
   return hipGetLastError();
 }
@@ -2243,7 +2263,7 @@ uint64_t apply_plan(const ggem_ctx* ctx, int precision) {
   for (int nr = 1; nr <= 8; nr *= 2)
     plan = (plan << 6) | (uint64_t(apply_chunk(ctx, precision, nr)) << 2) |
            (apply_default(ctx, precision, nr) == kBoxShape ? 2u : 0u) | (quad_lanes(ctx, precision, nr) ? 1u : 0u);
-  return plan;
+  return plan << 1 | (dense64(ctx) ? 1u : 0u);
 }
 bool apply_reads_lists(const ggem_ctx* ctx, int precision, int nrhs) {
   if (ctx->tune.on) return true;
