@@ -2061,9 +2061,10 @@ bool box_ready(const ggem_ctx* ctx, int precision, int nr) {
   if (!ctx->box_valid || ctx->box_max <= 0) return false;
   return precision == GGEM_FP32C ? !ctx->box_fp64 : (ctx->box_fp64 && ctx->coef64_valid);
 }
-// The staged kernel by default wherever it applies, except for several
-// operands in many sparse bricks: a quad block's cost is then the block, not
-// its few targets, while the list-order kernel fills its waves.  By bricks
+// The staged kernel by default wherever it applies, except in many sparse
+// bricks for several operands and for FP64 (whose lists are there): a block's
+// cost is then the block, not its few targets, while the list-order kernel
+// fills its waves.  Several operands by bricks
 // with targets over the records of each, and bricks enough for the blocks to
 // outweigh a wave that walks its lists alone; quads -> list order, us:
 //   beads (bricks)    element  2 operands      4               8
@@ -2077,13 +2078,24 @@ bool box_ready(const ggem_ctx* ctx, int precision, int nr) {
 //   140,000 (8,000)   3.9      30.2 -> 18.4    34.5 -> 26.6    52.4 -> 45.3
 //   300,000 (10,648)  2.0      68.1 -> 69.6    90.4 -> 115     -
 //   300,000 (39,304)  2.0      109 -> 37.4     123 -> 60.8     -
+// FP64 by targets a brick; lanes -> list order, us per application (in a
+// convergence-checked term, whose every block also leaves its dot products):
+//   beads      element  targets
+//   60,000     2.0        9: 20.5 -> 13.5            18: 17.2 -> 18.9
+//              3.1       18: 12.9 -> 11.9 (27 -> 17) 27: 12.5 -> 13.6
+//   400,000    2.0        9: 95.5 -> 43.7 (250 -> 54 at 8)  18: 89.6 -> 87.6
+//              3.1       18: 49.8 -> 35.7 (122 -> 50)       29: 41.5 -> 42.8
+//   1,000,000  3.1       20:  152 -> 97  (355 -> 129)       28:  134 -> 127
 bool sparse_bricks(const ggem_ctx* ctx, int nr) {
   const int64_t b = ctx->full_bricks;
+  if (nr == 1) return b >= 2500 && ctx->n < 20 * b;
   return b >= (nr == 2 ? 3000 : nr == 4 ? 4500 : 6000) && b * b > (nr == 2 ? 33 : nr == 4 ? 65 : 100) * ctx->box_recs;
 }
 int apply_default(const ggem_ctx* ctx, int precision, int nr) {
   if (!box_ready(ctx, precision, nr)) return 0;
-  return nr > 1 && quad_lanes(ctx, precision, nr) && sparse_bricks(ctx, nr) ? 0 : kBoxShape;
+  const bool sparse = nr > 1 ? quad_lanes(ctx, precision, nr) && sparse_bricks(ctx, nr)
+                             : precision == GGEM_FP64 && sparse_bricks(ctx, nr);
+  return sparse ? 0 : kBoxShape;
 }
 int apply_candidates(const ggem_ctx* ctx, int precision, int nr) {
   return box_ready(ctx, precision, nr) ? kNApply + 1 : kNApply;

@@ -1,7 +1,10 @@
 """The staged FP64 pair sums of one operand against the list-order kernel
 pinned through the autotuner, bit for bit, where the split changes: quads below
 20,000 beads, blocks of 256 lanes above, of 512 in dense bricks or few.  Some
-bricks hold more targets than a block has threads, or more records than the LDS."""
+bricks hold more targets than a block has threads, or more records than the LDS.
+And the list-order kernel, the default in sparse bricks, against the staged one."""
+import math
+
 import numpy as np
 import pytest
 
@@ -30,3 +33,23 @@ def test_fp64_blocks_equal_the_list_order_kernel(n, box, ne, periodic, crowd):
     for a, b in zip(*got):
         assert np.array_equal(a, b)
     assert np.array_equal(got[0][1], got[0][3]) and np.array_equal(got[0][2], got[0][4])
+
+
+@pytest.mark.parametrize("n,box,ne,periodic", [(20000, 256.0, 128, (1, 1, 1)), (60000, 310.0, 100, (0, 1, 0))])
+def test_fp64_sparse_bricks_default_equals_the_staged_kernel(n, box, ne, periodic):
+    dw = G.normal(3 * n, 41).reshape(1, n, 3)
+    lg = int(math.floor(math.log2(n)))
+    got = []
+    for staged in (False, True):
+        with context(n, box, ne, periodic, G.FP64) as ctx:
+            if staged:
+                ctx.tune_set("apply/fp64/1/%d" % lg, 5)
+                for epi in (0, 1):
+                    ctx.tune_set("pair_beads/fp64/%d/%d" % (epi, lg), 5)
+                ctx.set_autotune(True)
+            u = ctx.combine_velocity()
+            y, d, _ = ctx.cheb_brownian(5, 0.02, 3.0, dw, mode=G.CHEB_FIXED)
+            yr, dr, info = ctx.cheb_brownian(12, 0.02, 3.0, dw, tol=1e-30, mode=G.CHEB_REFERENCE)
+            got.append((u, y, d, yr, dr))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
