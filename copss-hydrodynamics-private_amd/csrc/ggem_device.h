@@ -389,12 +389,20 @@ __device__ __forceinline__ int wave_records(const BoxGeom& B, const BoxStencil& 
 // wave_records: a lane per target costs the wave every row and, row by row,
 // its longest run (and leaves lanes idle below 64 targets); a wave per target
 // costs the records of the z layers in reach, of which a wide stencil keeps
-// more.  Record fill with a lane per target and with a wave per target: 44 ->
-// 16 us at 100 beads, 156 -> 80 us for chains in a slit (25,600 beads, 69
-// rows, 31 targets in the median brick and 167 in the largest), 821 -> 413 us
-// for 64 suspensions (272,000 beads, 69 rows, 34 targets); at 125,000 beads
-// (21 rows, 244 targets) 49 -> 110 us, so that stays with a lane per target.
-__device__ __forceinline__ bool wave_walk(int nt, int nrows) { return nt <= kWaveWalkPerRow * nrows; }
+// more.  Record fill with a lane per target and with a wave per target, us:
+// where the waves are few (list_walk), 44 -> 16 at 100 beads, 156 -> 80 for chains in a
+// slit (25,600 beads, 69 rows, 31 targets in the median brick and 167 in the
+// largest).  Where they fill the chip:
+//   beads      rows  targets a brick
+//   12,000      69    56: 73 -> 42      96: 84 -> 54      (few)
+//               29    56: 37 -> 28      96: 44 -> 45
+//   60,000      69    60: 152 -> 127    82: 102 -> 155   117: 109 -> 284
+//               29    18: 79 -> 59      35: 65 -> 67      82: 59 -> 82
+//               21     9: 89 -> 86      27: 46 -> 52      60: 37 -> 54
+//   1,000,000   69    57: 1626 -> 1151  94: 1198 -> 1347 146: 1322 -> 2343
+//               29    20: 909 -> 681    37: 564 -> 599    72: 431 -> 718
+//               21    20: 601 -> 656    37: 360 -> 456    72: 250 -> 371
+__device__ __forceinline__ bool wave_walk(int nt, int nrows, int walk) { return nt <= wave_targets(walk, nrows); }
 
 // Share [i0, i1) of a brick's nt targets for this block: with wave_walk, one
 // of up to gridDim.y blocks for every kShareTargets targets.

@@ -386,10 +386,25 @@ inline int32_t box_rows_cap(const ggem_ctx* c) {
 // otherwise; 4096 bricks fill the chip by themselves and staging a brick
 // twice only costs.
 constexpr int kShareTargets = 32;
-constexpr int kWaveWalkPerRow = 4;  // wave_walk: targets per stencil row
+// How a launch walks the lists: a lane per target throughout, or a wave where
+// a brick's targets allow it (both sides at wave_walk).  kWalkFew: latency
+// decides and not the chip's issue rate (a wave per target reads its brick's
+// records, work that goes as beads times targets a brick).  kWalkWaves: the
+// chip is full, and with the mean brick's targets a wave each is less work
+// than a lane; by the mean, since a launch of both is slower than either.
+enum : int { kWalkLanes, kWalkWaves, kWalkFew };
+inline int list_walk(const ggem_ctx* c) {
+  const int64_t n = c->n, b = c->full_bricks, rows = box_rows_cap(c);
+  if (n * n <= 42000 * std::max<int64_t>(rows - 10, 2) * b) return kWalkFew;
+  return rows > 24 && n <= rows * 7 / 6 * b ? kWalkWaves : kWalkLanes;
+}
+// most targets of a brick that take a wave each
+__host__ __device__ constexpr int wave_targets(int walk, int nrows) {
+  return walk == kWalkFew ? 4 * nrows : walk == kWalkWaves ? 2 * nrows : 0;
+}
 inline unsigned brick_split(const ggem_ctx* c) {
   const int64_t nb = c->grid.n_cells >> (3 * kBrickBits);
-  const int64_t most = std::min<int64_t>(c->max_targets, int64_t(kWaveWalkPerRow) * box_rows_cap(c));
+  const int64_t most = std::min<int64_t>(c->max_targets, wave_targets(list_walk(c), box_rows_cap(c)));
   const int64_t s = (most + kShareTargets - 1) / kShareTargets;
   return nb > 2048 || s < 1 ? 1u : unsigned(std::min<int64_t>(s, 8));
 }

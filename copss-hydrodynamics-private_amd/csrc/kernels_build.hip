@@ -297,8 +297,10 @@ struct BrickArgs {
   const int32_t* slot_cell;  // brick-order cell of each slot
   const SysGrid* sys;        // batched contexts (null: one system)
   const int32_t* sys_slot;
+  int walk;                  // list_walk (list fill)
   int32_t cells_cap;         // box cells and stencil rows the LDS tables hold
   int32_t rows_cap;
+  int32_t recs_cap;          // records of a brick the list fill's tables hold
   int32_t* cnt;              // [n] list lengths by slot
   int64_t* box_cnt;          // census of the staged records (k_brick_count)
   int64_t* box_ecnt;
@@ -471,7 +473,9 @@ __global__ void __launch_bounds__(kSliceBlock) k_slice_len(const int32_t* __rest
 
 // The lists of the brick's slots in the sliced layout.  In a staged brick a
 // list is its records in record order (rows in stencil order, x ascending
-// through the box, slots ascending within a cell).
+// through the box, slots ascending within a cell).  The record tables hold what
+// the build's fullest staged brick has: sized for kBoxMaxRecs they leave six
+// blocks to a CU (400,000 beads, 18 a brick, 21 rows: 301 us, now 218).
 template <bool BATCH>
 __global__ void __launch_bounds__(kBrickThreads) k_brick_fill_ell(BrickArgs a, const int64_t* __restrict__ slice_off,
                                                                   uint32_t* __restrict__ ell) {
@@ -479,25 +483,26 @@ __global__ void __launch_bounds__(kBrickThreads) k_brick_fill_ell(BrickArgs a, c
   __shared__ int32_t s_w[kBrickThreads / 64];
   int32_t* first = lds;                                                 // [cells_cap]
   int32_t* cst = lds + a.cells_cap;                                     // [cells_cap + 1]
-  uint32_t* rent = reinterpret_cast<uint32_t*>(cst + a.cells_cap + 1);  // [kBoxMaxRecs]
-  uint32_t* rcell = rent + kBoxMaxRecs;                                 // [kBoxMaxRecs]
+  uint32_t* rent = reinterpret_cast<uint32_t*>(cst + a.cells_cap + 1);  // [recs_cap]
+  uint32_t* rcell = rent + a.recs_cap;                                  // [recs_cap]
   BoxStencil st;
-  st.t = reinterpret_cast<uint16_t*>(rcell + kBoxMaxRecs);              // [kStencilTab]
+  st.ok = false;
+  st.t = reinterpret_cast<uint16_t*>(rcell + a.recs_cap);               // [kStencilTab]
   const int64_t brick = blockIdx.x;
   const int64_t c0 = brick * kBrickCells;
   const int32_t sb = a.cs[c0], se = a.cs[c0 + kBrickCells];
   if (sb >= se) return;
   BoxGeom B;
   const SysView v = brick_view<BATCH>(a, brick, sb, B);
-  const bool waves = wave_walk(se - sb, v.nrows);
+  const bool waves = wave_walk(se - sb, v.nrows, a.walk);
   int i0, i1;
   brick_share(se - sb, waves, i0, i1);
   if (i0 >= i1) return;  // uniform over the block
   bool recs = false;
   if (brick_staged(a, B)) {
-    st.init(B, v.rows, v.nrows);
+    if (waves) st.init(B, v.rows, v.nrows);
     stage_box_cells<kBrickThreads>(B, a.cs, first, cst, s_w);
-    recs = cst[B.nbc] <= kBoxMaxRecs;
+    recs = cst[B.nbc] <= a.recs_cap;
     if (recs) {
       stage_box_entries(B, first, cst, rent, rcell);
     }
@@ -1301,6 +1306,7 @@ BrickArgs brick_args(const ggem_ctx* ctx) {
   a.g = ctx->grid;
   a.rows = ctx->rows_d;
   a.nrows = ctx->n_rows;
+  a.walk = list_walk(ctx);
   for (int d = 0; d < 3; ++d) a.reach[d] = ctx->reach[d];
   a.cs = ctx->cell_start;
   a.slot_cell = ctx->slot_cell;
@@ -1314,6 +1320,7 @@ BrickArgs brick_args(const ggem_ctx* ctx) {
   for (int k = 0; k < ctx->nsys && ctx->nsys > 1; ++k) cap = std::max(cap, cells(ctx->sys_h[k].reach));
   a.cells_cap = std::min(cap, kBoxMaxCells);
   a.rows_cap = box_rows_cap(ctx);
+  a.recs_cap = ctx->max_recs;
   a.cnt = ctx->nbr_cnt;
   a.box_cnt = ctx->box_cnt;
   a.box_ecnt = ctx->box_ecnt;
@@ -1407,7 +1414,7 @@ hipError_t launch_fill_ell(ggem_ctx* ctx) {
   ProfScope ps(ctx, "fill_ell");
   const BrickArgs a = brick_args(ctx);
   const size_t lds =
-      sizeof(int32_t) * (2 * size_t(a.cells_cap) + 1 + 2 * size_t(kBoxMaxRecs)) + sizeof(uint16_t) * kStencilTab;
+      sizeof(int32_t) * (2 * size_t(a.cells_cap) + 1 + 2 * size_t(a.recs_cap)) + sizeof(uint16_t) * kStencilTab;
   const unsigned split = brick_split(ctx);
   if (a.sys)
     hipLaunchKernelGGL(k_brick_fill_ell<true>, dim3(brick_count(ctx), split), dim3(kBrickThreads), lds, ctx->stream, a,
