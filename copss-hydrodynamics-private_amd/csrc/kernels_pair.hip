@@ -1926,6 +1926,7 @@ unsigned n_bricks(const ggem_ctx* ctx) { return unsigned(ctx->grid.n_cells >> (3
 //   beads      targets:  quads 256  512    targets:  quads 256  512
 //   12,000     23 (3.9)   7.7  8.1  8.3     96        8.8 10.4 10.2
 //              188       14.1 18.6 13.9
+//   22,000     17 (2.5)   9.4  9.1   -      43 (2.0) 12.8   -  14.1
 //   30,000     17 (2.5)  11.2 10.4 11.5     59       11.9 11.2 10.5
 //              240       18.7 23.7 16.6
 //   120,000    29 (3.9)  19.3 16.2 21.7     55 (3.1) 24.8 21.8 22.5
@@ -1967,7 +1968,7 @@ bool quad_lanes(const ggem_ctx* ctx, int precision, int nr) {
   if (nr > 2) return n < 95 * b || n * n < 6200000 * b;
   if (precision == GGEM_FP32C)
     return n <= 150 * b && (n < 100000 || n * n <= (n < 262144 ? 13 : 6) * b * recs);
-  return n < 20000;
+  return n < 22000;
 }
 
 // FP64 with a lane per target: blocks of 512 threads, where bricks often hold
